@@ -28,8 +28,10 @@
 namespace nq {
 namespace {
 
-constexpr int kSampThreads = 256;
+constexpr int kSampThreads = 512;
 constexpr int kMaxVocab = 4096;
+constexpr int kFastTopK = kWave;            // top-k widths whose ranks fit the lanes of one wave
+constexpr int kFastCand = kSampThreads / 2; // candidates that the rank sort takes
 constexpr uint32_t kLog2eBits = 0x3fb8aa3bu;   // 1.44269504f
 constexpr uint32_t kLn2HiBits = 0x3f318000u;   // 0.693359375f
 constexpr uint32_t kLn2LoBits = 0xb95e8083u;   // -2.12194440e-4f
@@ -94,6 +96,11 @@ __device__ __forceinline__ void load_logits8<uint16_t>(const uint16_t *p, float 
     for (int e = 0; e < 8; ++e) x[e] = t[e];
 }
 
+// The value whose sort_key is k.
+__device__ __forceinline__ float key_value(uint32_t k) {
+    return __uint_as_float((k & 0x80000000u) ? k ^ 0x80000000u : ~k);
+}
+
 // Lanes of this wave below the calling lane among those whose bit is set.
 __device__ __forceinline__ int lanes_below(uint64_t mask) {
     return static_cast<int>(__builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(mask >> 32),
@@ -102,7 +109,8 @@ __device__ __forceinline__ int lanes_below(uint64_t mask) {
 
 
 
-constexpr int kSampPer = kMaxVocab / kSampThreads;  // elements per thread (8 consecutive, twice)
+constexpr int kSampPer = kMaxVocab / kSampThreads;  // elements per thread (8 consecutive)
+static_assert(kSampPer == 8, "a thread's ids are one vector load");
 
 // Philox-4x32-10 (Salmon, Moraes, Dror, Shaw, SC'11): 10 rounds, key bumped by
 // the Weyl constants.  Returns the first output word.
@@ -150,10 +158,13 @@ sample_kernel(const InT *__restrict__ logits, int64_t logits_s0, int vocab,
               int update_seen, int64_t *__restrict__ tokens, int splits, int64_t plane,
               uint16_t *__restrict__ logits_out, int64_t out_s0) {
     __shared__ float s_val[kMaxVocab];
-    __shared__ uint64_t s_sort[kMaxVocab];
+    __shared__ __attribute__((aligned(16))) uint64_t s_sort[kMaxVocab];
     __shared__ uint32_t s_hist[2][256];
     __shared__ int s_bin, s_above, s_count, s_whole;
     __shared__ uint64_t s_red[kSampThreads / kWave];
+    __shared__ uint32_t s_top[kSampThreads];
+    __shared__ uint64_t s_ranked[kFastTopK];
+    __shared__ uint32_t s_rank[kFastCand];
 
     const int row = blockIdx.x;
     const int tid = threadIdx.x;
@@ -166,10 +177,9 @@ sample_kernel(const InT *__restrict__ logits, int64_t logits_s0, int vocab,
     const bool sup_eos = suppress_eos && suppress_eos[row];
     uint8_t *srow = seen ? seen + row * seen_s0 : nullptr;
 
-    // 1. masks, penalty, temperature: thread t owns ids 8t .. 8t + 7 and
-    // 8 (t + 256) .. + 7, loaded in one round trip; values go to LDS and stay in
-    // registers with their sortable keys (ids past the vocabulary get key 0,
-    // below every value)
+    // 1. masks, penalty, temperature: thread t owns ids 8t .. 8t + 7, loaded in one
+    // round trip; values go to LDS and stay in registers with their sortable keys
+    // (ids past the vocabulary get key 0, below every value)
     float val[kSampPer];
     uint32_t key[kSampPer];
     {
@@ -244,6 +254,16 @@ sample_kernel(const InT *__restrict__ logits, int64_t logits_s0, int vocab,
     }
     for (int i = tid; i < 2 * 256; i += kSampThreads) (&s_hist[0][0])[i] = 0u;
     if (tid == 0) s_count = 0;
+    {   // each thread's largest key, for the narrow top-k below
+        uint32_t top = key[0];
+#pragma unroll
+        for (int i = 1; i < kSampPer; ++i) top = key[i] > top ? key[i] : top;
+        s_top[tid] = top;
+        if (tid < kFastCand) {
+            s_rank[tid] = 0u;
+            s_sort[tid] = 0ull;
+        }
+    }
     __syncthreads();
 
     int token;
@@ -272,6 +292,115 @@ sample_kernel(const InT *__restrict__ logits, int64_t logits_s0, int vocab,
         const int k_eff = (kq > 0 && kq < vocab) ? kq : vocab;
         float p = top_p[row];
         p = p < 1.0f ? p : 1.0f;
+
+        // Narrow top-k (up to 64, the serving default 50): no histogram and no sorting
+        // network.  k group maxima reach the threshold below, so at least k keys do: every key
+        // at or above it is a candidate (about 100 of 2048 normal logits for k = 50).  The
+        // candidates are ranked by counting, and one wave, rank r on lane r, does the weights,
+        // the scan, the nucleus and the draw in registers, with the same sums in the same order
+        // as the general path.  Both are chains of latencies: the radix select's passes of LDS
+        // atomics on a few hot bins, the 21-step network and the barriers between them took
+        // 11.4 us for one row of 2048 logits in four planes and 15.3 us for 64 rows of 3072;
+        // this takes 6.2 and 7.3 us (2.3 us of it the loads, 0.7 the threshold, 0.6 the
+        // collection, 0.9 the ranks, 0.8 the draw).  More candidates than ranks are kept for
+        // (many equal keys) take the general path, as a wider top-k does: its ranks need
+        // more than a lane each.
+        bool drawn = false;
+        if (k_eff <= kFastTopK) {
+            // group L: the threads of lane L (32 of 2048 ids), also where the ids past some point are masked
+            uint32_t top = 0;
+#pragma unroll
+            for (int w = 0; w < kSampThreads / kWave; ++w) top = s_top[w * kWave + lane] > top ? s_top[w * kWave + lane] : top;
+            // a threshold that k_eff .. k_eff + 2 group maxima reach, from the top bits down (at the last
+            // ones: the k_eff-th largest itself);
+            // two bits a step: three ballots in flight instead of a chain of two
+            uint32_t thr = 0;
+            for (int bit = 30; bit >= 0; bit -= 2) {
+                const uint32_t t1 = thr | (1u << bit), t2 = thr | (2u << bit), t3 = thr | (3u << bit);
+                const int n1 = __popcll(__ballot(top >= t1));
+                const int n2 = __popcll(__ballot(top >= t2));
+                const int n3 = __popcll(__ballot(top >= t3));
+                if (n1 < k_eff) continue;
+                thr = n3 >= k_eff ? t3 : n2 >= k_eff ? t2 : t1;
+                if ((n3 >= k_eff ? n3 : n2 >= k_eff ? n2 : n1) <= k_eff + 2) break;
+            }
+            int c = 0;
+#pragma unroll
+            for (int i = 0; i < kSampPer; ++i) c += key[i] != 0u && key[i] >= thr ? 1 : 0;
+            const int incl = wave_incl_scan(c);
+            int base = 0;
+            if (lane == kWave - 1) base = atomicAdd(&s_count, incl);
+            base = __builtin_amdgcn_readlane(base, kWave - 1) + incl - c;
+#pragma unroll
+            for (int i = 0; i < kSampPer; ++i) {
+                if (key[i] != 0u && key[i] >= thr) {
+                    const int id = (tid + (i / 8) * kSampThreads) * 8 + i % 8;
+                    if (base < kFastCand) s_sort[base] = composite(val[i], id);
+                    ++base;
+                }
+            }
+            __syncthreads();
+            const int n_c = s_count;
+            if (n_c <= kFastCand) {
+                // rank = candidates above; up to 64, 128, 256 candidates are shared by eight, four, two threads each
+                const int span = n_c <= kWave ? kWave : n_c <= 2 * kWave ? 2 * kWave : kFastCand;
+                const int parts = kSampThreads / span;
+                const int i = tid & (span - 1);
+                const int each = ((n_c + parts - 1) / parts + 7) & ~7;  // parts * each <= span
+                const int j0 = (tid / span) * each;
+                const uint64_t mine = s_sort[i];
+                uint32_t above = 0;
+                for (int j = j0; j < j0 + each; j += 8) {  // entries past n_c are 0, below every candidate
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) above += s_sort[j + e] > mine ? 1u : 0u;
+                }
+                if (i < n_c) atomicAdd(&s_rank[i], above);
+                __syncthreads();
+                if (tid < n_c && s_rank[tid] < static_cast<uint32_t>(kFastTopK)) s_ranked[s_rank[tid]] = s_sort[tid];
+                __syncthreads();
+                if (wave == 0) {
+                    const bool on = lane < k_eff;
+                    const uint64_t e = on ? s_ranked[lane] : 0ull;
+                    const uint32_t kv = static_cast<uint32_t>(e >> 32);
+                    const float v0 = key_value(static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(kv), 0)));
+                    const float w = on ? nq_exp(key_value(kv) - v0) : 0.0f;
+                    float S = 0.0f + w;
+                    const float loc = S;
+#pragma unroll
+                    for (int d = 1; d < kWave; d <<= 1) {
+                        const float o = __shfl_up(S, d, kWave);
+                        if (lane >= d) S = S + o;
+                    }
+                    float excl = __shfl_up(S, 1, kWave);
+                    if (lane == 0) excl = 0.0f;
+                    const float cum = excl + loc;
+                    const float total = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(cum), k_eff - 1));
+                    const float pt = p * total;
+                    const uint64_t drop = __ballot(on && !((cum - w) < pt));
+                    const int first_drop = drop ? __ffsll(static_cast<long long>(drop)) - 1 : k_eff;
+                    const int kept = first_drop > 0 ? first_drop : 1;
+                    const float mass = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(cum), kept - 1));
+                    const float u = uniforms ? uniforms[row]
+                                             : counter_uniform(seed[row * seed_stride], offset[row * offset_stride]);
+                    const float um = u * mass;
+                    const uint64_t hit = __ballot(lane < kept && cum >= um);
+                    int pick = hit ? __ffsll(static_cast<long long>(hit)) - 1 : kept - 1;
+                    if (v0 == -INFINITY) pick = 0;
+                    const uint32_t id = 0xffffffffu - static_cast<uint32_t>(__builtin_amdgcn_readlane(
+                                                          static_cast<int>(static_cast<uint32_t>(e)), pick));
+                    if (lane == 0) {
+                        tokens[row] = static_cast<int64_t>(id);
+                        if (update_seen && srow) srow[id] = 1;
+                    }
+                }
+                drawn = true;
+            } else {
+                __syncthreads();  // every thread has read the count
+                if (tid == 0) s_count = 0;
+                __syncthreads();
+            }
+        }
+        if (drawn) return;  // uniform: every thread of the row took the same path
 
         // 2. radix select of the k_eff-th largest sortable key, 8 bits a pass from
         // the top; wave 0 locates each pass's digit (lane L scans bins

@@ -87,6 +87,26 @@ def test_ties_resolve_to_lowest_id(nq, device):
     assert np.all(to_np(_check(logits, t, k, p, u, r, seen)) == 100)
 
 
+@pytest.mark.parametrize("vocab", [8, 60, 64, 257, 2048, 3072, 4096])
+@pytest.mark.parametrize("top_k", [1, 50, 57, 64, 65])
+@pytest.mark.parametrize("values", ["normal", "peaked", "steps", "masked"])
+def test_narrow_top_k_bit_exact(nq, device, vocab, top_k, values):
+    """Both sides of the 64-rank limit of the one-wave draw, with distributions that leave few, many and
+    more candidates than it takes (steps: seven distinct values), and rows of which most ids are masked."""
+
+    logits, t, k, p, u, r, seen = _inputs(device, 11 * vocab + top_k, 12, vocab, dtype=torch.bfloat16, top_k=top_k)
+    if values == "peaked":
+        logits[:, vocab // 3] += 20.0
+    elif values == "steps":
+        logits = logits.round()
+    elif values == "masked":
+        logits[:, : vocab - vocab // 16] = -float("inf")
+    u[0], u[1] = 0.0, 1.0 - 2.0 ** -24
+    p[2:4] = torch.tensor([1.0, 1e-3], device=device)
+    t[4] = 0.0
+    _check(logits, t, k, p, u, r, seen)
+
+
 def test_update_seen_marks_sampled_token(nq, device):
     from nari_qwen3_tts_amd.sampling import sample_with_uniforms
 
