@@ -263,17 +263,24 @@ constexpr int kSwK = 2048;
 constexpr int kSwRows = 64;
 static_assert(kSwRows / 16 == kSwQuarters, "the wave of quarter q finishes 16-row tile q");
 
-template <int K>
+// MT 16-row tiles (1, 2 or 4: the fewest that hold M).  The staging and the operand
+// reads of the activation block grow with its rows, zero rows included: back to back in a
+// graph over 100 MB of weights 8 rows take 7.0 us in one tile, 32 rows 7.9 in two, and any
+// count 9.5 in four.  At 8 rows the 25.2 MB of weights are 3.6 us of it at 7 TB/s of cache.
+// One or two column tiles a workgroup instead of three: 7.1 and 7.4 us at 8 rows, 10.2 and
+// 8.8 at 32.  The sums and bits of a row do not depend on MT.
+template <int K, int MT>
 __global__ void __launch_bounds__(kSwThreads)
 fp8_swiglu_kernel(const uint8_t *__restrict__ x, int64_t x_s0, const float *__restrict__ sx, int64_t sx_s0, int M,
                   const uint8_t *__restrict__ w, int64_t w_s0, const float *__restrict__ sw, int64_t sw_s0, int I,
                   uint16_t *__restrict__ out, int64_t o_s0) {
     constexpr int KB = K / 128;                    // K blocks
+    constexpr int kRows = 16 * MT;
     constexpr int QS = K / kSwQuarters / 128;      // K blocks per quarter
-    using Lds = Fp8Lds<kSwRows, K>;
+    using Lds = Fp8Lds<kRows, K>;
     __shared__ __attribute__((aligned(16))) uint8_t xs[Lds::kBytes];
-    __shared__ float sxs[KB * kSwRows];  // [K block][row]: a wave's 16 rows hit 16 banks
-    static_assert(kSwQuarters * kSwTiles * kWave * 16 * 4 <= Lds::kBytes, "reduction fits the X area");
+    __shared__ float sxs[KB * kRows];  // [K block][row]: a wave's 16 rows hit 16 banks
+    static_assert(kSwQuarters * kSwTiles * kWave * 16 * MT <= Lds::kBytes, "reduction fits the X area");
 
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = threadIdx.x / kWave;
@@ -287,9 +294,9 @@ fp8_swiglu_kernel(const uint8_t *__restrict__ x, int64_t x_s0, const float *__re
     // 1. the activation block and its scales (rows >= M zero), issued first:
     // loads complete in issue order, so the wait for them below leaves the
     // weights in flight and the X block reaches LDS long before the weights
-    constexpr int kVec = kSwRows * (K / 16);
+    constexpr int kVec = kRows * (K / 16);
     constexpr int kPer = (kVec + kSwThreads - 1) / kSwThreads;
-    constexpr int kSx = kSwRows * KB;
+    constexpr int kSx = kRows * KB;
     constexpr int kSxPer = (kSx + kSwThreads - 1) / kSwThreads;
     // Every workgroup reads the same block: each starts at its own (even)
     // rotation of it, so the CUs of an XCD do not all ask the same L2 lines
@@ -310,7 +317,7 @@ fp8_swiglu_kernel(const uint8_t *__restrict__ x, int64_t x_s0, const float *__re
     for (int u = 0; u < kSxPer; ++u) {
         const int i = threadIdx.x + u * kSwThreads;
         // element i of the [K block][row] table
-        sr[u] = (i < kSx && i % kSwRows < M) ? sx[(i % kSwRows) * sx_s0 + i / kSwRows] : 0.f;
+        sr[u] = (i < kSx && i % kRows < M) ? sx[(i % kRows) * sx_s0 + i / kRows] : 0.f;
     }
     // 2. the wave's weights (16 packed rows over its K quarter) and scales:
     // gate rows 8t.. lie in 128-row block t / 16, up rows in (I + 8t) / 128
@@ -354,18 +361,18 @@ fp8_swiglu_kernel(const uint8_t *__restrict__ x, int64_t x_s0, const float *__re
     __syncthreads();
 
     // 3. the quarter's MFMAs, scaled per K block: lane columns 0, 1 are gate, 2, 3 up
-    floatx4_t acc[4];
+    floatx4_t acc[MT];
 #pragma unroll
-    for (int m = 0; m < 4; ++m) acc[m] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+    for (int m = 0; m < MT; ++m) acc[m] = floatx4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int j = 0; j < QS; ++j) {
 #pragma unroll
-        for (int m = 0; m < 4; ++m) {
+        for (int m = 0; m < MT; ++m) {
             const int row = m * 16 + r16;
             const int8v_t b = Lds::read(xs, row, kb0 + j, kq);
             const floatx4_t t = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
                 wr[j], b, floatx4_t{0.f, 0.f, 0.f, 0.f}, 0, 0, 0, 127, 0, 127);
-            const float sxv = sxs[(kb0 + j) * kSwRows + row];
+            const float sxv = sxs[(kb0 + j) * kRows + row];
             const float sg = sxv * swg[j], su = sxv * swu[j];
             acc[m][0] = fmaf(t[0], sg, acc[m][0]);
             acc[m][1] = fmaf(t[1], sg, acc[m][1]);
@@ -375,7 +382,7 @@ fp8_swiglu_kernel(const uint8_t *__restrict__ x, int64_t x_s0, const float *__re
         // pin the block's sums here: the MFMAs (which start from zero and touch no
         // memory) may otherwise sink below every later LDS read
 #pragma unroll
-        for (int m = 0; m < 4; ++m) asm volatile("" : "+v"(acc[m]));
+        for (int m = 0; m < MT; ++m) asm volatile("" : "+v"(acc[m]));
         __builtin_amdgcn_sched_barrier(0);
     }
 
@@ -386,16 +393,17 @@ fp8_swiglu_kernel(const uint8_t *__restrict__ x, int64_t x_s0, const float *__re
     float *red = reinterpret_cast<float *>(xs);
     // layout [quarter][tile][m][lane][4]: a float4 access touches 64 consecutive float4s
     {
-        float *dst = red + ((quarter * kSwTiles + tl) * 4 * kWave + lane) * 4;
+        float *dst = red + ((quarter * kSwTiles + tl) * MT * kWave + lane) * 4;
 #pragma unroll
-        for (int m = 0; m < 4; ++m)
+        for (int m = 0; m < MT; ++m)
             *reinterpret_cast<float4 *>(dst + m * kWave * 4) = make_float4(acc[m][0], acc[m][1], acc[m][2], acc[m][3]);
     }
     __syncthreads();
     const int m = quarter;
+    if (m >= MT) return;
     float sum[4];
     {
-        const float4 v0 = *reinterpret_cast<const float4 *>(red + ((tl * 4 + m) * kWave + lane) * 4);
+        const float4 v0 = *reinterpret_cast<const float4 *>(red + ((tl * MT + m) * kWave + lane) * 4);
         sum[0] = v0.x;
         sum[1] = v0.y;
         sum[2] = v0.z;
@@ -403,7 +411,7 @@ fp8_swiglu_kernel(const uint8_t *__restrict__ x, int64_t x_s0, const float *__re
     }
 #pragma unroll
     for (int q = 1; q < kSwQuarters; ++q) {
-        const float4 v = *reinterpret_cast<const float4 *>(red + (((q * kSwTiles + tl) * 4 + m) * kWave + lane) * 4);
+        const float4 v = *reinterpret_cast<const float4 *>(red + (((q * kSwTiles + tl) * MT + m) * kWave + lane) * 4);
         sum[0] += v.x;
         sum[1] += v.y;
         sum[2] += v.z;
@@ -772,8 +780,11 @@ extern "C" int nq_linear_fp8_swiglu(const uint8_t *xq, int64_t x_s0, const float
     NQ_CHECK_ARG(x_s0 >= K && w_s0 >= K && x_s0 % 16 == 0 && w_s0 % 16 == 0 && al16(xq) && al16(packed));
     NQ_CHECK_ARG(sx_s0 >= K / 128 && sw_s0 >= K / 128 && o_s0 >= I && o_s0 % 2 == 0);
     NQ_CHECK_ARG(reinterpret_cast<uintptr_t>(out) % 4 == 0);
-    hipLaunchKernelGGL((fp8_swiglu_kernel<kSwK>), dim3(I / (8 * kSwTiles)), dim3(kSwThreads), 0,
-                       static_cast<hipStream_t>(stream), xq, x_s0, sx, sx_s0, M, packed, w_s0, sw, sw_s0, I, out, o_s0);
+    const auto kernel = M <= 16   ? fp8_swiglu_kernel<kSwK, 1>
+                        : M <= 32 ? fp8_swiglu_kernel<kSwK, 2>
+                                  : fp8_swiglu_kernel<kSwK, 4>;
+    hipLaunchKernelGGL(kernel, dim3(I / (8 * kSwTiles)), dim3(kSwThreads), 0, static_cast<hipStream_t>(stream), xq,
+                       x_s0, sx, sx_s0, M, packed, w_s0, sw, sw_s0, I, out, o_s0);
     return NQ_LAUNCH_STATUS();
 }
 

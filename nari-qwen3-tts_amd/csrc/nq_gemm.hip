@@ -277,53 +277,60 @@ void dispatch_gemm(const uint16_t *x, int64_t x_s0, int M, const uint16_t *w, in
 // (nq_fp8_pack_swiglu on the bf16 rows): 16-row tile t holds, for q = 0..3,
 // gate rows 8t + 2q, 8t + 2q + 1 then up rows 8t + 2q, 8t + 2q + 1, so MFMA
 // lane group q ends with two gate/up pairs of the same act columns
-// 8t + 2q + {0, 1}.  A workgroup owns kBsTiles tiles of one 64-row block; its
-// kBsTiles * kBsQuarters waves each take one tile over one quarter of K, the
+// 8t + 2q + {0, 1}.  A workgroup owns kTiles tiles of one row block; its
+// kTiles * kBsQuarters waves each take one tile over one quarter of K, the
 // chain of each quarter runs in k order from zero (the MFMA operands and
 // order of a K slice of the split-K kernel), the quarters are summed in
 // order through LDS, and the epilogue rounds gate and up to bf16 and stores
 // bf16(silu(g) * u) -- the bits of the split-K projection with four 256-wide
 // slices (its choice at 128 rows) followed by the SiLU-mul kernel.
 
-constexpr int kBsTiles = 3;
-constexpr int kBsQuarters = 4;
-constexpr int kBsThreads = kBsTiles * kBsQuarters * kWave;
-constexpr int kBsRows = 64;
-constexpr int kBsK = 1024;
-static_assert(kBsRows / 16 == kBsQuarters, "the wave of quarter q finishes 16-row block q");
+//
+// MT 16-row tiles (1, 2 or 4) of rows and kTiles column tiles (2 or 3) a
+// workgroup.  The kernel is a chain of latencies and LDS passes: the staging and
+// the operand reads grow with the block's rows, zero rows included, and with
+// three column tiles only 128 of the CUs stream the 12.6 MB of weights.  Cached
+// weights, I = 3072, back to back in a graph: 8 rows 6.3 us as one 64-row block of
+// three tiles, 5.2 with 16 rows, 4.3 with 16 rows and two tiles (5.1 with one);
+// 32 rows 6.9, 6.0, 5.1; 64 rows 7.4 and 6.4.
 
-template <int K>
-__global__ void __launch_bounds__(kBsThreads)
+constexpr int kBsQuarters = 4;
+constexpr int kBsK = 1024;
+
+template <int K, int MT, int kTiles>
+__global__ void __launch_bounds__(kTiles * kBsQuarters * kWave)
 bf16_swiglu_kernel(const uint16_t *__restrict__ x, int64_t x_s0, int M, const uint16_t *__restrict__ w,
                    int64_t w_s0, uint16_t *__restrict__ out, int64_t o_s0) {
+    constexpr int kRows = 16 * MT;
+    constexpr int kThreads = kTiles * kBsQuarters * kWave;
     constexpr int XP = x_pitch<K>();   // LDS row pitch (bf16)
     constexpr int QK = K / kBsQuarters;
     constexpr int QS = QK / 32;         // MFMA steps per quarter
-    __shared__ __attribute__((aligned(16))) uint16_t xs[kBsRows * XP];
-    static_assert(kBsQuarters * kBsTiles * 4 * kWave * 4 * 4 <= kBsRows * XP * 2, "reduction fits the X area");
+    __shared__ __attribute__((aligned(16))) uint16_t xs[kRows * XP];
+    static_assert(kBsQuarters * kTiles * MT * kWave * 4 * 4 <= kRows * XP * 2, "reduction fits the X area");
 
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = threadIdx.x / kWave;
     const int r16 = lane & 15;
     const int kq = lane >> 4;
-    const int tl = wave % kBsTiles;
-    const int quarter = wave / kBsTiles;
-    const int tile = blockIdx.x * kBsTiles + tl;
-    const int row0 = blockIdx.y * kBsRows;
-    const int rows = M - row0 < kBsRows ? M - row0 : kBsRows;
+    const int tl = wave % kTiles;
+    const int quarter = wave / kTiles;
+    const int tile = blockIdx.x * kTiles + tl;
+    const int row0 = blockIdx.y * kRows;
+    const int rows = M - row0 < kRows ? M - row0 : kRows;
 
     // 1. the activation block (rows past M zero), issued first: loads complete in
     // issue order, so the wait for them below leaves the weights in flight.  Each
     // workgroup starts at its own rotation of the block, so the CUs of an XCD do
     // not all ask the same L2 lines at the same moment.
-    constexpr int kVec = kBsRows * (K / 8);
-    constexpr int kPer = (kVec + kBsThreads - 1) / kBsThreads;
+    constexpr int kVec = kRows * (K / 8);
+    constexpr int kPer = (kVec + kThreads - 1) / kThreads;
     const int rot = (blockIdx.x * 258) % kVec;
     auto rot_of = [&](int i) { return i + rot < kVec ? i + rot : i + rot - kVec; };
     uint4 xr[kPer];
 #pragma unroll
     for (int u = 0; u < kPer; ++u) {
-        const int i = threadIdx.x + u * kBsThreads;
+        const int i = threadIdx.x + u * kThreads;
         const int v = rot_of(i);
         const int row = v / (K / 8), c = v % (K / 8);
         xr[u] = (i < kVec && row < rows) ? *reinterpret_cast<const uint4 *>(x + (row0 + row) * x_s0 + c * 8)
@@ -339,20 +346,20 @@ bf16_swiglu_kernel(const uint16_t *__restrict__ x, int64_t x_s0, int M, const ui
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int u = 0; u < kPer; ++u) {
-        const int i = threadIdx.x + u * kBsThreads;
+        const int i = threadIdx.x + u * kThreads;
         const int v = rot_of(i);
         if (i < kVec) *reinterpret_cast<uint4 *>(xs + (v / (K / 8)) * XP + (v % (K / 8)) * 8) = xr[u];
     }
     __syncthreads();
 
     // 3. the quarter's MFMA chains (W as the A operand, X^T from LDS as the B operand)
-    floatx4_t acc[4];
+    floatx4_t acc[MT];
 #pragma unroll
-    for (int m = 0; m < 4; ++m) acc[m] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+    for (int m = 0; m < MT; ++m) acc[m] = floatx4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int j = 0; j < QS; ++j) {
 #pragma unroll
-        for (int m = 0; m < 4; ++m) {
+        for (int m = 0; m < MT; ++m) {
             const uint4 b = *reinterpret_cast<const uint4 *>(xs + (m * 16 + r16) * XP + quarter * QK + j * 32 + kq * 8);
             acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(wr[j]), as_bf16x8(b), acc[m], 0, 0, 0);
         }
@@ -364,16 +371,17 @@ bf16_swiglu_kernel(const uint16_t *__restrict__ x, int64_t x_s0, int M, const ui
     __syncthreads();
     float *red = reinterpret_cast<float *>(xs);
     {
-        float *dst = red + ((quarter * kBsTiles + tl) * 4 * kWave + lane) * 4;
+        float *dst = red + ((quarter * kTiles + tl) * MT * kWave + lane) * 4;
 #pragma unroll
-        for (int m = 0; m < 4; ++m)
+        for (int m = 0; m < MT; ++m)
             *reinterpret_cast<float4 *>(dst + m * kWave * 4) = make_float4(acc[m][0], acc[m][1], acc[m][2], acc[m][3]);
     }
     __syncthreads();
     const int m = quarter;
+    if (m >= MT) return;
     float sum[4];
     {
-        const float4 v0 = *reinterpret_cast<const float4 *>(red + ((tl * 4 + m) * kWave + lane) * 4);
+        const float4 v0 = *reinterpret_cast<const float4 *>(red + ((tl * MT + m) * kWave + lane) * 4);
         sum[0] = v0.x;
         sum[1] = v0.y;
         sum[2] = v0.z;
@@ -381,7 +389,7 @@ bf16_swiglu_kernel(const uint16_t *__restrict__ x, int64_t x_s0, int M, const ui
     }
 #pragma unroll
     for (int q = 1; q < kBsQuarters; ++q) {
-        const float4 v = *reinterpret_cast<const float4 *>(red + (((q * kBsTiles + tl) * 4 + m) * kWave + lane) * 4);
+        const float4 v = *reinterpret_cast<const float4 *>(red + (((q * kTiles + tl) * MT + m) * kWave + lane) * 4);
         sum[0] += v.x;
         sum[1] += v.y;
         sum[2] += v.z;
@@ -501,13 +509,28 @@ extern "C" int nq_linear_add_rmsnorm_fp8(const uint16_t *x, int64_t x_s0, const 
 extern "C" int nq_linear_swiglu(const uint16_t *x, int64_t x_s0, int M, const uint16_t *packed, int64_t w_s0, int I,
                                 int K, uint16_t *out, int64_t o_s0, void *stream) {
     NQ_CHECK_ARG(x && packed && out && M > 0 && I > 0 && K > 0);
-    if (K != nq::kBsK || I % (8 * nq::kBsTiles) != 0) return NQ_ERR_UNSUPPORTED;
+    if (K != nq::kBsK || I % 24 != 0) return NQ_ERR_UNSUPPORTED;
     NQ_CHECK_ARG(x_s0 >= K && w_s0 >= K && x_s0 % 8 == 0 && w_s0 % 8 == 0);
     NQ_CHECK_ARG((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(packed)) % 16 == 0);
     NQ_CHECK_ARG(o_s0 >= I && o_s0 % 2 == 0 && reinterpret_cast<uintptr_t>(out) % 4 == 0);
-    const dim3 grid(static_cast<unsigned>(2 * I / (16 * nq::kBsTiles)),
-                    static_cast<unsigned>((M + nq::kBsRows - 1) / nq::kBsRows));
-    hipLaunchKernelGGL((nq::bf16_swiglu_kernel<nq::kBsK>), grid, dim3(nq::kBsThreads), 0,
-                       static_cast<hipStream_t>(stream), x, x_s0, M, packed, w_s0, out, o_s0);
+    // the fewest 16-row tiles that hold the rows (past 64 rows: blocks of four), and two column tiles a
+    // workgroup rather than three unless its 128 KB activation blocks then need a second round of the CUs
+    const int mt = M <= 16 ? 1 : M <= 32 ? 2 : 4;
+    const int blocks = (M + 16 * mt - 1) / (16 * mt);
+    const int pairs = I / 16 * blocks;
+#define NQ_BF16_SWIGLU(MT, TL)                                                                          \
+    hipLaunchKernelGGL((nq::bf16_swiglu_kernel<nq::kBsK, MT, TL>),                                       \
+                       dim3(static_cast<unsigned>(I / (8 * TL)), static_cast<unsigned>(blocks)),          \
+                       dim3(TL * nq::kBsQuarters * nq::kWave), 0, static_cast<hipStream_t>(stream), x, x_s0, \
+                       M, packed, w_s0, out, o_s0)
+    if (mt == 1 && I % 16 == 0)
+        NQ_BF16_SWIGLU(1, 2);
+    else if (mt == 2 && I % 16 == 0)
+        NQ_BF16_SWIGLU(2, 2);
+    else if (I % 16 == 0 && pairs <= 256)
+        NQ_BF16_SWIGLU(4, 2);
+    else
+        NQ_BF16_SWIGLU(4, 3);
+#undef NQ_BF16_SWIGLU
     return NQ_LAUNCH_STATUS();
 }

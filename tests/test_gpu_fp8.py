@@ -213,3 +213,23 @@ def test_fused_swiglu_integer_codes_exact(nq, device):
     got = fused.float().cpu().numpy()
     # gate and up are exact, so only silu's exp rounding separates the two (<= 1 bf16 ulp)
     assert np.all(np.abs(got - want) <= 2.0 ** -8 * np.abs(want) + 1e-6)
+
+
+@pytest.mark.parametrize("m", [1, 15, 16, 17, 32, 33, 63])
+def test_fused_swiglu_rows_do_not_depend_on_the_row_tiles(nq, device, m):
+    """One, two or four row tiles sum a row the same way: the bits of a 64-row call's rows."""
+
+    from nari_qwen3_tts_amd.layers import (linear_fp8_swiglu, pack_fp8_swiglu, quantize_fp8_rows,
+                                           quantize_fp8_weight_blocks)
+
+    g = torch.Generator(device=device)
+    g.manual_seed(300 + m)
+    xq, sx = quantize_fp8_rows(torch.randn(64, 2048, generator=g, device=device).to(torch.bfloat16))
+    wq, sw = quantize_fp8_weight_blocks((torch.randn(768, 2048, generator=g, device=device) * 0.02).to(torch.bfloat16))
+    packed = pack_fp8_swiglu(wq)
+    want = torch.empty(64, 384, dtype=torch.bfloat16, device=device)
+    linear_fp8_swiglu(xq, sx, packed, sw, want)
+    out = torch.full((64, 384), float("nan"), dtype=torch.bfloat16, device=device)
+    linear_fp8_swiglu(xq[:m], sx[:m], packed, sw, out[:m])
+    assert torch.equal(out[:m], want[:m])
+    assert bool(out[m:].isnan().all())

@@ -277,3 +277,22 @@ def test_fused_bf16_swiglu_falls_back_outside_its_shape(nq, device):
     assert torch.equal(out, linear_silu_mul(x, w))
     with pytest.raises(TypeError):
         linear_swiglu(x, pack_swiglu(w), out)
+
+
+@pytest.mark.parametrize("inter", [24, 48, 3072])
+@pytest.mark.parametrize("m", [1, 15, 16, 17, 32, 33, 64, 65])
+def test_fused_bf16_swiglu_rows_do_not_depend_on_the_row_tiles(nq, device, m, inter):
+    """Every row-tile and column-tile count sums a row the same way: the bits of a 128-row call's rows."""
+
+    from nari_qwen3_tts_amd.layers import linear_swiglu, pack_swiglu
+
+    g = torch.Generator(device=device)
+    g.manual_seed(31 * m + inter)
+    x = torch.randn(128, 1024, generator=g, device=device).to(torch.bfloat16)
+    packed = pack_swiglu((torch.randn(2 * inter, 1024, generator=g, device=device) * 0.05).to(torch.bfloat16))
+    want = torch.empty(128, inter, dtype=torch.bfloat16, device=device)
+    linear_swiglu(x, packed, want)
+    out = torch.full((128, inter), float("nan"), dtype=torch.bfloat16, device=device)
+    linear_swiglu(x[:m], packed, out[:m])
+    assert torch.equal(out[:m], want[:m])
+    assert bool(out[m:].isnan().all())
