@@ -1836,6 +1836,214 @@ dense_short_kernel(const uint16_t *__restrict__ q, int64_t q_s0, int64_t q_s1,
     }
 }
 
+// ---------------------------------------------------------------------------
+// Attention over at most 16 cached positions (the code predictor's frame), one
+// wave per (row, kv head).  Such a call is a chain of latencies, not work: a
+// workgroup of four waves that met at barriers, read the rotated q back from
+// memory and combined four online softmaxes took 4.9 us (one row) to 5.5 us
+// (64 rows) back to back in a graph, this one 3.6-3.7 and 4.0-4.1 (128-row frames spend 0.2 ms less in it).  Every load
+// of K, V and the planes is issued at entry; lane l holds a quarter (l % 4) of
+// the head's dims of position l / 4, so a score is one DPP quad sum; the 16
+// scores of a head go through LDS and each lane repeats its softmax (fp32
+// throughout); then lane pairs of dims gather V from LDS.
+
+constexpr int kShortLen = 16;
+
+template <int D, int G>
+struct ShortSmem {
+    __attribute__((aligned(16))) uint16_t q[G][D];
+    __attribute__((aligned(16))) uint16_t k[D];  // the new position's K (fused kernel)
+    __attribute__((aligned(16))) uint16_t v[kShortLen][D];
+    __attribute__((aligned(16))) float s[G][kShortLen];
+};
+
+// Positions p < stop of kv head h: this lane's quarter of position lane / 4.
+template <int D>
+__device__ __forceinline__ void short_load(const uint16_t *__restrict__ base, int64_t c_pos, int stop, int lane,
+                                           uint4 (&r)[D / 32]) {
+    const int pos = lane >> 2;
+    const uint16_t *p = base + pos * c_pos + (lane & 3) * (D / 4);
+#pragma unroll
+    for (int i = 0; i < D / 32; ++i)
+        r[i] = pos < stop ? *reinterpret_cast<const uint4 *>(p + i * 8) : make_uint4(0, 0, 0, 0);
+}
+
+// sm.q and sm.v (rows past len zero) are in LDS, kr holds the lane's K quarter; every lane of the wave calls.
+template <int D, int G>
+__device__ __forceinline__ void short_attend(ShortSmem<D, G> &sm, const uint4 (&kr)[D / 32], int len, int lane,
+                                             float scale_log2, uint16_t *__restrict__ out, int64_t o_s1) {
+    const int quarter = (lane & 3) * (D / 4);
+#pragma unroll
+    for (int j = 0; j < G; ++j) {
+        float dot = 0.f;
+#pragma unroll
+        for (int i = 0; i < D / 32; ++i) {
+            float a[8], b[8];
+            unpack8(*reinterpret_cast<const uint4 *>(&sm.q[j][quarter + i * 8]), a);
+            unpack8(kr[i], b);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) dot = fmaf(a[e], b[e], dot);
+        }
+        dot = group_sum<4>(dot);
+        if ((lane & 3) == 0) sm.s[j][lane >> 2] = (lane >> 2) < len ? dot * scale_log2 : -INFINITY;
+    }
+    __syncthreads();
+    constexpr int HALF = D / 2;
+    for (int t = lane; t < G * HALF; t += kWave) {
+        const int j = t / HALF, d = (t % HALF) * 2;
+        float w[kShortLen];
+#pragma unroll
+        for (int i = 0; i < kShortLen; i += 4) {
+            const float4 f = *reinterpret_cast<const float4 *>(&sm.s[j][i]);
+            w[i] = f.x;
+            w[i + 1] = f.y;
+            w[i + 2] = f.z;
+            w[i + 3] = f.w;
+        }
+        float mx = w[0];
+#pragma unroll
+        for (int i = 1; i < kShortLen; ++i) mx = fmaxf(mx, w[i]);
+        float l = 0.f, o0 = 0.f, o1 = 0.f;
+#pragma unroll
+        for (int i = 0; i < kShortLen; ++i) {  // positions past len: weight 0, V rows 0
+            const float e = __builtin_amdgcn_exp2f(w[i] - mx);
+            const uint32_t v = *reinterpret_cast<const uint32_t *>(&sm.v[i][d]);
+            l += e;
+            o0 = fmaf(e, __uint_as_float(v << 16), o0);
+            o1 = fmaf(e, __uint_as_float(v & 0xffff0000u), o1);
+        }
+        *reinterpret_cast<uint32_t *>(out + j * o_s1 + d) =
+            pack2_bf16(l > 0.f ? o0 / l : 0.f, l > 0.f ? o1 / l : 0.f);
+    }
+}
+
+// Stages the lane's V quarter of its position (zeros past the cached ones), except position `skip`.
+template <int D, int G>
+__device__ __forceinline__ void short_stage_v(ShortSmem<D, G> &sm, const uint4 (&vr)[D / 32], int skip, int lane) {
+    if ((lane >> 2) == skip) return;
+#pragma unroll
+    for (int i = 0; i < D / 32; ++i)
+        *reinterpret_cast<uint4 *>(&sm.v[lane >> 2][(lane & 3) * (D / 4) + i * 8]) = vr[i];
+}
+
+template <int D, int G>
+__global__ void __launch_bounds__(kWave)
+short_kernel(const uint16_t *__restrict__ q, int64_t q_s0, int64_t q_s1, const uint16_t *__restrict__ cache,
+             int64_t c_row, int64_t c_kind, int64_t c_pos, int64_t c_head, int valid_length, int num_kv_heads,
+             float scale_log2, uint16_t *__restrict__ out, int64_t o_s0, int64_t o_s1) {
+    __shared__ ShortSmem<D, G> sm;
+    const int lane = threadIdx.x;
+    const int row = blockIdx.x / num_kv_heads;
+    const int h = blockIdx.x - row * num_kv_heads;
+    const uint16_t *base = cache + row * c_row + h * c_head;
+    uint4 kr[D / 32], vr[D / 32];
+    short_load<D>(base, c_pos, valid_length, lane, kr);
+    short_load<D>(base + c_kind, c_pos, valid_length, lane, vr);
+    for (int t = lane; t < G * D / 8; t += kWave) {
+        const int j = t / (D / 8), d = t % (D / 8) * 8;
+        *reinterpret_cast<uint4 *>(&sm.q[j][d]) =
+            *reinterpret_cast<const uint4 *>(q + row * q_s0 + (h * G + j) * q_s1 + d);
+    }
+    short_stage_v(sm, vr, -1, lane);
+    __syncthreads();
+    short_attend(sm, kr, valid_length, lane, scale_log2, out + row * o_s0 + h * G * o_s1, o_s1);
+}
+
+// The same with the q/k norm + RoPE + K/V write in front, from the packed QKV
+// projection's split-K planes (summed in plane order and rounded to bf16; the
+// arithmetic of nq_qkv_partials_norm_rope_kv_write, so the same bits in q_out
+// and the cache).  A unit is a query head, the key head or the value head; a
+// wave takes 128 / D of them at a time, a lane the pair (i, i + D / 2).
+template <int D, int G>
+__global__ void __launch_bounds__(kWave)
+rope_short_kernel(const float *__restrict__ partials, int splits, int64_t plane, int64_t prow,
+                  const uint16_t *__restrict__ q_weight, const uint16_t *__restrict__ k_weight,
+                  const int64_t *__restrict__ positions, int64_t pos_stride, float eps, float log_theta,
+                  int round_to_input, uint16_t *__restrict__ q_out, int64_t q_s0, int64_t q_s1,
+                  uint16_t *__restrict__ cache, int64_t c_row, int64_t c_kind, int64_t c_pos, int64_t c_head,
+                  int cache_position, int num_kv_heads, float scale_log2, uint16_t *__restrict__ out, int64_t o_s0,
+                  int64_t o_s1) {
+    constexpr int HALF = D / 2;
+    constexpr int kAtOnce = kWave / HALF;
+    constexpr int kRounds = (G + 2 + kAtOnce - 1) / kAtOnce;
+    __shared__ ShortSmem<D, G> sm;
+    const int lane = threadIdx.x;
+    const int row = blockIdx.x / num_kv_heads;
+    const int h = blockIdx.x - row * num_kv_heads;
+    const int Hq = num_kv_heads * G;
+    const int pair = lane % HALF;
+    uint16_t *base = cache + row * c_row + h * c_head;
+    uint16_t *slot = base + cache_position * c_pos;
+
+    // the planes four at a time (all loads in flight together)
+    float x[kRounds][2];
+#pragma unroll
+    for (int r = 0; r < kRounds; ++r) x[r][0] = x[r][1] = 0.f;
+    const float *src[kRounds];
+#pragma unroll
+    for (int r = 0; r < kRounds; ++r) {
+        const int u = r * kAtOnce + lane / HALF;
+        const int head = u < G ? h * G + u : u == G ? Hq + h : Hq + num_kv_heads + h;
+        src[r] = partials + row * prow + static_cast<int64_t>(u < G + 2 ? head : h) * D + pair;
+    }
+    uint4 kr[D / 32], vr[D / 32];
+    const float position = static_cast<float>(positions[row * pos_stride]);
+    for (int i0 = 0; i0 < splits; i0 += 4) {
+        float a[kRounds][4][2];
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            if (i0 + v >= splits) break;
+#pragma unroll
+            for (int r = 0; r < kRounds; ++r) {
+                a[r][v][0] = src[r][(i0 + v) * plane];
+                a[r][v][1] = src[r][(i0 + v) * plane + HALF];
+            }
+        }
+        if (i0 == 0) {  // behind the first planes' loads, ahead of the wait for them
+            short_load<D>(base, c_pos, cache_position, lane, kr);
+            short_load<D>(base + c_kind, c_pos, cache_position, lane, vr);
+        }
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            if (i0 + v >= splits) break;
+#pragma unroll
+            for (int r = 0; r < kRounds; ++r) {
+                x[r][0] += a[r][v][0];
+                x[r][1] += a[r][v][1];
+            }
+        }
+    }
+    const float qw1 = bf16_to_f32(q_weight[pair]), qw2 = bf16_to_f32(q_weight[pair + HALF]);
+    const float kw1 = bf16_to_f32(k_weight[pair]), kw2 = bf16_to_f32(k_weight[pair + HALF]);
+#pragma unroll
+    for (int r = 0; r < kRounds; ++r) {
+        const int u = r * kAtOnce + lane / HALF;
+        const float x1 = bf16_to_f32(f32_to_bf16(x[r][0])), x2 = bf16_to_f32(f32_to_bf16(x[r][1]));
+        uint16_t o1, o2;
+        norm_rope_pair<D>(x1, x2, true, u < G ? qw1 : kw1, u < G ? qw2 : kw2, pair, eps, log_theta, position,
+                          round_to_input, o1, o2);
+        if (u < G) {
+            uint16_t *dst = q_out + row * q_s0 + (h * G + u) * q_s1;
+            dst[pair] = sm.q[u][pair] = o1;
+            dst[pair + HALF] = sm.q[u][pair + HALF] = o2;
+        } else if (u == G) {
+            slot[pair] = sm.k[pair] = o1;
+            slot[pair + HALF] = sm.k[pair + HALF] = o2;
+        } else if (u == G + 1) {
+            slot[c_kind + pair] = sm.v[cache_position][pair] = f32_to_bf16(x1);
+            slot[c_kind + pair + HALF] = sm.v[cache_position][pair + HALF] = f32_to_bf16(x2);
+        }
+    }
+    short_stage_v(sm, vr, cache_position, lane);
+    __syncthreads();
+    if ((lane >> 2) == cache_position) {
+#pragma unroll
+        for (int i = 0; i < D / 32; ++i)
+            kr[i] = *reinterpret_cast<const uint4 *>(&sm.k[(lane & 3) * (D / 4) + i * 8]);
+    }
+    short_attend(sm, kr, cache_position + 1, lane, scale_log2, out + row * o_s0 + h * G * o_s1, o_s1);
+}
+
 // Code-predictor layer attention with the q/k norm + RoPE + K/V write fused
 // in.  Workgroup (row, kv head h): waves 0 .. G-1 normalise and rotate query
 // heads h G + j from the packed QKV projection's split-K planes (summed in
@@ -2463,6 +2671,12 @@ int launch_dense(const uint16_t *q, int64_t q_s0, int64_t q_s1, const uint16_t *
                  int valid_length, int Hkv, float scale, uint16_t *out, int64_t o_s0, int64_t o_s1,
                  hipStream_t stream) {
     int64_t items = static_cast<int64_t>(rows) * Hkv;
+    if (valid_length <= kShortLen && items <= 0x7fffffff && (o_s0 % 2 | o_s1 % 2) == 0) {
+        hipLaunchKernelGGL((short_kernel<D, G>), dim3(static_cast<unsigned>(items)), dim3(kWave), 0, stream, q, q_s0,
+                           q_s1, cache, c_row, c_kind, c_pos, c_head, valid_length, Hkv, scale * kLog2e, out, o_s0,
+                           o_s1);
+        return NQ_LAUNCH_STATUS();
+    }
     int grid = static_cast<int>(items < 8192 ? items : 8192);
     hipLaunchKernelGGL((dense_short_kernel<D, G>), dim3(grid), dim3(kAttnThreads), 0, stream, q,
                        q_s0, q_s1, cache, c_row, c_kind, c_pos, c_head, rows, valid_length, Hkv,
@@ -2478,6 +2692,13 @@ int launch_dense_rope(const float *partials, int splits, int rows, const uint16_
                       int64_t o_s0, int64_t o_s1, hipStream_t stream) {
     const int64_t prow = static_cast<int64_t>(Hkv * G + 2 * Hkv) * D;
     const int64_t items = static_cast<int64_t>(rows) * Hkv;
+    if (cache_position < kShortLen && items <= 0x7fffffff && (o_s0 % 2 | o_s1 % 2) == 0) {
+        hipLaunchKernelGGL((rope_short_kernel<D, G>), dim3(static_cast<unsigned>(items)), dim3(kWave), 0, stream,
+                           partials, splits, static_cast<int64_t>(rows) * prow, prow, q_weight, k_weight, positions,
+                           pos_stride, eps, logf(rope_theta), round_to_input, q_out, q_s0, q_s1, cache, c_row, c_kind,
+                           c_pos, c_head, cache_position, Hkv, scale * kLog2e, out, o_s0, o_s1);
+        return NQ_LAUNCH_STATUS();
+    }
     const int grid = static_cast<int>(items < 8192 ? items : 8192);
     hipLaunchKernelGGL((dense_rope_short_kernel<D, G>), dim3(grid), dim3(kAttnThreads), 0, stream, partials, splits,
                        static_cast<int64_t>(rows) * prow, prow, q_weight, k_weight, positions, pos_stride, eps,

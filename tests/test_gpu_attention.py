@@ -268,6 +268,42 @@ def test_code_predictor_short_cache(nq, device, valid_length):
     assert mx <= MAX_ABS and mean <= MEAN_ABS
 
 
+@pytest.mark.parametrize("d,group", [(64, 1), (64, 2), (64, 8), (128, 1), (128, 2), (128, 4)])
+@pytest.mark.parametrize("position", [0, 1, 14, 15])
+def test_short_cache_head_shapes(nq, device, d, group, position):
+    """Every head shape of the one-wave short-cache attention against the oracle, uncached positions
+    holding NaN; and, for the groups the fused launch takes, q, cache and output bits equal to the
+    two launches'."""
+
+    from nari_qwen3_tts_amd import kernels as K
+
+    g = torch.Generator(device=device)
+    g.manual_seed(100 * d + 10 * group + position)
+    rows, hkv, splits = 5, 4, 3
+    hq = hkv * group
+    cache = torch.randn(rows, 2, 16, hkv, d, generator=g, device=device).to(torch.bfloat16)
+    cache[:, :, position + 1:] = float("nan")
+    q = torch.randn(rows, hq, d, generator=g, device=device).to(torch.bfloat16)
+    out = K.decode_attn_nhd_short_cache(q, cache[:, 0], cache[:, 1], position + 1)
+    want = o_att.short_cache_attention(to_np(q), to_np(cache[:, 0]), to_np(cache[:, 1]), position + 1)
+    mx, mean = attention_error(to_np(out), want)
+    assert mx <= MAX_ABS and mean <= MEAN_ABS
+    if group > 2:
+        return
+    planes = torch.randn(splits, rows, (hq + 2 * hkv) * d, generator=g, device=device)
+    w = [torch.randn(d, generator=g, device=device).to(torch.bfloat16) for _ in range(2)]
+    at = torch.full((rows,), position, dtype=torch.long, device=device)
+    caches, qs, outs = [cache.clone() for _ in range(2)], [torch.empty_like(q) for _ in range(2)], []
+    a = (planes.view(torch.uint8).flatten(), splits)
+    K.qkv_partials_norm_rope_dense_cache_(*a, qs[0], *w, at, 1e-6, 1e6, caches[0][:, 0], caches[0][:, 1], position)
+    outs.append(K.decode_attn_nhd_short_cache(qs[0], caches[0][:, 0], caches[0][:, 1], position + 1))
+    outs.append(torch.empty_like(q))
+    K.qkv_partials_rope_short_attention_(*a, qs[1], *w, at, 1e-6, 1e6, caches[1][:, 0], caches[1][:, 1], position,
+                                         outs[1])
+    for x, y in (caches, qs, outs):
+        assert torch.equal(x.view(torch.int16), y.view(torch.int16))
+
+
 def _fused_case(nq, device, seed, lengths, capture, pages, ps=16):
     rng = np.random.default_rng(seed)
     kv = make_kv(nq, device, layers=1, pages=pages, ps=ps, scratch=capture)
