@@ -710,6 +710,21 @@ int nq_codec_advance(const int32_t *offsets, int B, const int32_t *slots, int64_
 int nq_codec_pcm16(const float *x, int64_t n, float *wav, int16_t *pcm, void *stream);
 
 /*
+ * nq_codec_state_copy: the state tensors of `rows` streams into the first rows
+ * of a state pool (to_pool) or back.  Tensor kind k of a stream is a contiguous
+ * fp32 [A][B][inner] (shapes[3k..3k+2]); its pool row is [B][A][inner], rows
+ * contiguous from pool[k].  pool [kinds], shapes [kinds][3] and state
+ * [rows][kinds] are host arrays (device addresses; a zero state address stages
+ * zeros), read before the call returns; 16-byte aligned addresses where inner
+ * is a multiple of 4.  With to_pool, position (device int64, one per row at
+ * position_stride) fills frame_pos and context (device int64 [rows]) ctx_len;
+ * either may be NULL.
+ */
+int nq_codec_state_copy(int rows, int kinds, const int64_t *pool, const int32_t *shapes, const int64_t *state,
+                        int to_pool, const int64_t *position, int64_t position_stride, int64_t *frame_pos,
+                        const int64_t *context, int32_t *ctx_len, void *stream);
+
+/*
  * GEMM form of the wide convolutions.  nq_codec_im2col gathers the operand a
  * conv (or transconv) becomes one GEMM over: conv rows hold the K taps of the
  * (activated) input, history included, as a[t, k*Cin + ci]; transconv rows

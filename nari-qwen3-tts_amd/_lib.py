@@ -107,6 +107,7 @@ _SIGNATURES: dict[str, list] = {
                                   _I, _P, _L, _P],
     "nq_codec_advance": [_P, _I, _P, _P, _P, _I, _P],
     "nq_codec_pcm16": [_P, _L, _P, _P, _P],
+    "nq_codec_state_copy": [_I, _I, _P, _P, _P, _I, _P, _L, _P, _P, _P, _P],
     "nq_codec_im2col": [_P, _L, _L, _P, _I, _I, _P, _P, _I, _I, _I, _I, _P, _P, _P, _L, _P],
     "nq_codec_history_update": [_P, _L, _P, _I, _I, _P, _P, _I, _I, _P, _P, _P],
     "nq_codec_transconv_overlap": [_P, _I, _I, _I, _P, _P, _P, _I, _P, _L, _P],

@@ -202,6 +202,7 @@ class _StatePool:
         self.frame_pos = torch.zeros(slots, dtype=torch.long, device=device)
         self.ctx = torch.zeros(slots, dtype=torch.int32, device=device)
         self.free = list(range(slots))
+        self.kinds = None  # IncrementalCodecDecoder._state_kinds of this pool
 
     def reset(self, slot: int) -> None:
         for t in list(self.hist.values()) + list(self.overlap.values()):
@@ -391,70 +392,86 @@ class IncrementalCodecDecoder:
             self._shape_cache[key] = got
         return got
 
+    def _state_kinds(self, pool: "_StatePool"):
+        """Every tensor of a stream's state: its mapping and key in the reference's state object, its
+        shape there, and as ``nq_codec_state_copy`` takes them the pool addresses and the shapes
+        (the last two axes change places in the pool, around the head dim for K/V)."""
+
+        got = pool.kinds
+        if got is None:
+            c = self.config
+            hist_keys, over_keys = self.reference_keys()
+            kinds = [("conv_histories", hist_keys[n], (cin, pad), pool.hist[n], 1)
+                     for n, (cin, pad) in _history_shapes(c).items()]
+            kinds += [("transconv_overlaps", over_keys[n], (cout, s), pool.overlap[n], 1)
+                      for n, (cout, s) in _overlap_shapes(c).items()]
+            kv = (c.heads, c.retained_context, c.head_dim)
+            for li in range(c.layers):
+                kinds += [("transformer_keys", li, kv, pool.k[li], c.head_dim),
+                          ("transformer_values", li, kv, pool.v[li], c.head_dim)]
+            names = tuple(k[:3] for k in kinds)
+            address = np.array([k[3].data_ptr() for k in kinds], dtype=np.int64)
+            shapes = np.array([(*k[2][:2], k[4]) for k in kinds], dtype=np.int32)
+            # a new stream state is one allocation: each tensor's offset in it, 16-byte aligned
+            ends = np.cumsum([-(-int(np.prod(k[2])) // 4) * 4 for k in kinds])
+            got = pool.kinds = (names, address, shapes, (0, *ends[:-1].tolist()), int(ends[-1]))
+        return got
+
+    def _state_copy(self, pool: "_StatePool", rows: int, state: np.ndarray, to_pool: bool, position=None,
+                    context=None) -> None:
+        _, address, shapes, _, _ = self._state_kinds(pool)
+        _lib.call("nq_codec_state_copy", rows, len(address), address.ctypes.data, shapes.ctypes.data, state.ctypes.data,
+                  int(to_pool), _lib.ptr(position), 0 if position is None else position.stride(0),
+                  pool.frame_pos.data_ptr(), _lib.ptr(context), pool.ctx.data_ptr(), _lib.stream(self.device))
+
     def _stage_in(self, states, pool: "_StatePool", rows: int, frames: int, position_ids, context_lengths) -> None:
-        c = self.config
         dev = self.device
-        hist_keys, over_keys = self.reference_keys()
-
-        def gather(mapping: str, key, shape, dst_rows):
-            values = [getattr(st, mapping).get(key) for st in states]
-            for v in values:
-                if v is not None and tuple(v.shape) != shape:
-                    raise ValueError(f"invalid incremental state {key!r}: expected {shape}, got {tuple(v.shape)}")
-            if all(v is None for v in values):
-                dst_rows.zero_()
-                return
-            zero = None
-            rows_in = []
-            for v in values:
+        names = self._state_kinds(pool)[0]
+        state = np.zeros((rows, len(names)), dtype=np.int64)
+        held = []  # copies of tensors that are not contiguous fp32 on the device, until the launch is queued
+        for k, (mapping, key, shape) in enumerate(names):
+            for row, st in enumerate(states):
+                v = getattr(st, mapping).get(key)
                 if v is None:
-                    zero = torch.zeros(shape, dtype=torch.float32, device=dev) if zero is None else zero
-                    v = zero
-                rows_in.append(v.to(device=dev, dtype=torch.float32))
-            dst_rows.copy_(torch.stack(rows_in).transpose(1, 2))
-
-        for name, (cin, pad) in _history_shapes(c).items():
-            gather("conv_histories", hist_keys[name], (cin, pad), pool.hist[name][:rows])
-        for name, (cout, stride) in _overlap_shapes(c).items():
-            gather("transconv_overlaps", over_keys[name], (cout, stride), pool.overlap[name][:rows])
-        r = c.retained_context
-        for li in range(c.layers):
-            gather("transformer_keys", li, (c.heads, r, c.head_dim), pool.k[li, :rows])
-            gather("transformer_values", li, (c.heads, r, c.head_dim), pool.v[li, :rows])
+                    continue
+                if tuple(v.shape) != shape:
+                    raise ValueError(f"invalid incremental state {key!r}: expected {shape}, got {tuple(v.shape)}")
+                if v.dtype != torch.float32 or v.device != dev or not v.is_contiguous() or v.data_ptr() % 16:
+                    v = torch.empty(shape, dtype=torch.float32, device=dev).copy_(v)
+                    held.append(v)
+                state[row, k] = v.data_ptr()
+        position = context = None
         if position_ids is None:
             pool.frame_pos[:rows].copy_(torch.tensor([st.frame_position for st in states], dtype=torch.long))
         else:
             if tuple(position_ids.shape) != (rows, frames):
                 raise ValueError(f"incremental position_ids must have shape {(rows, frames)}, got "
                                  f"{tuple(position_ids.shape)}")
-            pool.frame_pos[:rows].copy_(position_ids[:, 0])
+            if position_ids.dtype == torch.long and position_ids.device == dev:
+                position = position_ids[:, 0]
+            else:
+                pool.frame_pos[:rows].copy_(position_ids[:, 0])
         if context_lengths is None:
             pool.ctx[:rows].copy_(torch.tensor([st.transformer_context_length for st in states], dtype=torch.int32))
         else:
             if tuple(context_lengths.shape) != (rows,):
                 raise ValueError(f"incremental context_lengths must have shape {(rows,)}, got "
                                  f"{tuple(context_lengths.shape)}")
-            pool.ctx[:rows].copy_(context_lengths)
+            if context_lengths.dtype == torch.long and context_lengths.device == dev and context_lengths.is_contiguous():
+                context = context_lengths
+            else:
+                pool.ctx[:rows].copy_(context_lengths)
+        self._state_copy(pool, rows, state, True, position, context)
 
     def _stage_out(self, states, pool: "_StatePool", rows: int, frames: int) -> None:
-        c = self.config
-        hist_keys, over_keys = self.reference_keys()
-        for name in _history_shapes(c):
-            new = pool.hist[name][:rows].transpose(1, 2).contiguous()
-            for st, row in zip(states, new.unbind(0)):
-                st.conv_histories[hist_keys[name]] = row
-        for name in _overlap_shapes(c):
-            new = pool.overlap[name][:rows].transpose(1, 2).contiguous()
-            for st, row in zip(states, new.unbind(0)):
-                st.transconv_overlaps[over_keys[name]] = row
-        for li in range(c.layers):
-            keys = pool.k[li, :rows].transpose(1, 2).contiguous()
-            values = pool.v[li, :rows].transpose(1, 2).contiguous()
-            for st, k, v in zip(states, keys.unbind(0), values.unbind(0)):
-                st.transformer_keys[li] = k
-                st.transformer_values[li] = v
-        r = c.retained_context
-        for st in states:
+        names, _, _, offsets, total = self._state_kinds(pool)
+        new = [torch.empty(total, dtype=torch.float32, device=self.device) for _ in range(rows)]
+        state = np.array([t.data_ptr() for t in new], dtype=np.int64)[:, None] + 4 * np.array(offsets, dtype=np.int64)
+        self._state_copy(pool, rows, state, False)
+        r = self.retained_context
+        for st, flat in zip(states, new):
+            for (mapping, key, shape), at in zip(names, offsets):
+                getattr(st, mapping)[key] = flat[at: at + math.prod(shape)].view(shape)
             st.frame_position += frames
             st.transformer_context_length = min(r, st.transformer_context_length + frames)
 

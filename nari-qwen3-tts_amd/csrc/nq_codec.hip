@@ -412,6 +412,64 @@ dwconv_kernel(const float *__restrict__ x, int64_t ldx, int64_t T, const int32_t
     }
 }
 
+// ---------------------------------------------------------------------------
+// Staging of per-stream state tensors (the reference's state objects) into a
+// state pool's rows and back, every tensor of up to kStateRows streams in one
+// launch.  A state tensor is [A][B][inner], its pool row [B][A][inner]; its
+// address travels in the kernel's arguments.  A stream has 39 such tensors of
+// 0.2 to 51 KB, so the cost is launches: stacking, transposing and copying
+// them one kind at a time took 116 launches and 273 us of a captured
+// one-stream step (1324 -> 1053 us with two).
+
+constexpr int kStateKinds = 40;
+constexpr int kStateRows = 9;
+constexpr int kStateThreads = 1024;
+
+struct StateKind {
+    float *pool;
+    int row_stride, a, b, inner;
+};
+struct StateArgs {
+    StateKind kind[kStateKinds];
+    float *state[kStateRows][kStateKinds];
+    const int64_t *position;  // fills frame_pos when given
+    int64_t position_stride;
+    int64_t *frame_pos;
+    const int64_t *context;  // fills ctx_len when given
+    int32_t *ctx_len;
+};
+static_assert(sizeof(StateArgs) <= 4096, "kernel arguments hold 4 KB");
+
+template <bool kToPool>
+__global__ void __launch_bounds__(kStateThreads) state_copy_kernel(const StateArgs args) {
+    const int row = blockIdx.y;
+    const StateKind k = args.kind[blockIdx.x];
+    float *state = args.state[row][blockIdx.x];
+    float *pool = k.pool + static_cast<int64_t>(row) * k.row_stride;
+    if (kToPool && blockIdx.x == 0 && threadIdx.x == 0) {
+        if (args.position) args.frame_pos[row] = args.position[row * args.position_stride];
+        if (args.context) args.ctx_len[row] = static_cast<int32_t>(args.context[row]);
+    }
+    const bool vec = k.inner % 4 == 0;  // the host checked that the addresses are 16-byte aligned then
+    const int inner = vec ? k.inner / 4 : k.inner;
+    const int n = k.a * k.b * inner;
+    for (int e = threadIdx.x; e < n; e += kStateThreads) {
+        // consecutive threads write consecutive elements
+        const int i = e % inner, rest = e / inner;
+        const int lo = kToPool ? rest % k.a : rest % k.b, hi = kToPool ? rest / k.a : rest / k.b;
+        const int from = (kToPool ? lo * k.b + hi : lo * k.a + hi) * inner + i;
+        if (vec) {
+            float4 *dst = reinterpret_cast<float4 *>(kToPool ? pool : state);
+            const float4 *src = reinterpret_cast<const float4 *>(kToPool ? state : pool);
+            dst[e] = src ? src[from] : make_float4(0.f, 0.f, 0.f, 0.f);
+        } else {
+            float *dst = kToPool ? pool : state;
+            const float *src = kToPool ? state : pool;
+            dst[e] = src ? src[from] : 0.f;
+        }
+    }
+}
+
 // new history = last pad rows of [history ; act(x)] per stream
 __global__ void __launch_bounds__(kCodecThreads)
 history_update_kernel(const float *__restrict__ x, int64_t ldx, const int32_t *__restrict__ off, int B, int u,
@@ -1448,6 +1506,55 @@ extern "C" int nq_codec_advance(const int32_t *offsets, int B, const int32_t *sl
     NQ_CHECK_ARG(offsets && slots && frame_pos && ctx_len && B > 0 && R >= 0);
     hipLaunchKernelGGL(advance_kernel, dim3((B + 63) / 64), dim3(64), 0, static_cast<hipStream_t>(stream), offsets, B,
                        slots, frame_pos, ctx_len, R);
+    return NQ_LAUNCH_STATUS();
+}
+
+extern "C" int nq_codec_state_copy(int rows, int kinds, const int64_t *pool, const int32_t *shapes,
+                                   const int64_t *state, int to_pool, const int64_t *position,
+                                   int64_t position_stride, int64_t *frame_pos, const int64_t *context,
+                                   int32_t *ctx_len, void *stream) {
+    using namespace nq;
+    NQ_CHECK_ARG(rows >= 1 && kinds >= 1 && pool && shapes && state);
+    NQ_CHECK_ARG((!position || (frame_pos && to_pool)) && (!context || (ctx_len && to_pool)));
+    for (int k = 0; k < kinds; ++k) {
+        const int64_t a = shapes[3 * k], b = shapes[3 * k + 1], inner = shapes[3 * k + 2];
+        NQ_CHECK_ARG(pool[k] && a >= 1 && b >= 1 && inner >= 1 && a * b * inner <= (1 << 24));
+        const int64_t mask = inner % 4 == 0 ? 15 : 3;
+        NQ_CHECK_ARG((pool[k] & mask) == 0);
+        for (int r = 0; r < rows; ++r) {
+            const int64_t at = state[static_cast<int64_t>(r) * kinds + k];
+            NQ_CHECK_ARG((at & mask) == 0 && (at || to_pool));
+        }
+    }
+    for (int r0 = 0; r0 < rows; r0 += kStateRows) {
+        const int nr = rows - r0 < kStateRows ? rows - r0 : kStateRows;
+        for (int k0 = 0; k0 < kinds; k0 += kStateKinds) {
+            const int nk = kinds - k0 < kStateKinds ? kinds - k0 : kStateKinds;
+            StateArgs args = {};
+            for (int k = 0; k < nk; ++k) {
+                const int32_t *sh = shapes + 3 * (k0 + k);
+                const int stride = sh[0] * sh[1] * sh[2];
+                args.kind[k] = {reinterpret_cast<float *>(pool[k0 + k]) + static_cast<int64_t>(r0) * stride, stride,
+                                sh[0], sh[1], sh[2]};
+                for (int r = 0; r < nr; ++r)
+                    args.state[r][k] = reinterpret_cast<float *>(state[static_cast<int64_t>(r0 + r) * kinds + k0 + k]);
+            }
+            if (position && k0 == 0) {
+                args.position = position + r0 * position_stride;
+                args.position_stride = position_stride;
+                args.frame_pos = frame_pos + r0;
+            }
+            if (context && k0 == 0) {
+                args.context = context + r0;
+                args.ctx_len = ctx_len + r0;
+            }
+            const dim3 grid(nk, nr), block(kStateThreads);
+            if (to_pool)
+                hipLaunchKernelGGL(state_copy_kernel<true>, grid, block, 0, static_cast<hipStream_t>(stream), args);
+            else
+                hipLaunchKernelGGL(state_copy_kernel<false>, grid, block, 0, static_cast<hipStream_t>(stream), args);
+        }
+    }
     return NQ_LAUNCH_STATUS();
 }
 

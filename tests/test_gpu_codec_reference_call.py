@@ -188,3 +188,37 @@ def test_pcm16_and_pinned_transfer_of_the_decoded_waveform(nq, device):
     assert pool.active == 0
     assert o_codec.pcm16(np.array([-2.0, -0.5, 0.0, 0.5, 2.0], np.float32)).tolist() == \
         pcm16(torch.tensor([-2.0, -0.5, 0.0, 0.5, 2.0], device=device)).tolist()
+
+
+@pytest.mark.parametrize("rows", [1, 9, 10, 19])
+def test_state_staging_takes_any_layout_and_missing_tensors(nq, device, rows):
+    """Rows on both sides of a launch's row count; states with missing tensors (zeros), and tensors that
+    are not contiguous, not fp32 or not on the device, decode as contiguous fp32 ones do."""
+
+    from nari_qwen3_tts_amd.codec import CodecConfig, CodecWeights, IncrementalCodecDecoder
+
+    cfg = CodecConfig()
+    dec = IncrementalCodecDecoder(CodecWeights(cfg, device, seed=81), max_streams=1)
+    g = torch.Generator().manual_seed(82)
+    codes = torch.randint(0, cfg.codebook_size, (rows, 16, 3), generator=g).to(device)
+    states = [IncrementalCodecState() for _ in range(rows)]
+    dec(codes, states)
+    other = [clone_state(s) for s in states]
+    for i, (a, b) in enumerate(zip(states, other)):
+        if i % 3 == 0:  # missing: zeros
+            del b.conv_histories["decoder.0"], b.transformer_keys[2]
+            a.conv_histories["decoder.0"] = torch.zeros_like(a.conv_histories["decoder.0"])
+            a.transformer_keys[2] = torch.zeros_like(a.transformer_keys[2])
+        b.conv_histories["pre_conv"] = b.conv_histories["pre_conv"].t().contiguous().t()
+        b.transformer_values[5] = b.transformer_values[5].double()
+        b.transconv_overlaps["decoder.1.transconv"] = b.transconv_overlaps["decoder.1.transconv"].cpu()
+    want, got = dec(codes, states), dec(codes, other)
+    assert torch.equal(got, want)
+    for a, b in zip(states, other):
+        assert a.frame_position == b.frame_position == 6
+        for name in MAPPINGS:
+            for key, value in getattr(a, name).items():
+                assert torch.equal(getattr(b, name)[key], value), (name, key)
+    with pytest.raises(ValueError, match="invalid incremental state"):
+        other[-1].conv_histories["pre_conv"] = torch.zeros(cfg.dim, 3, device=device)
+        dec(codes, other)
