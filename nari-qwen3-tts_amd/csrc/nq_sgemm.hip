@@ -272,6 +272,98 @@ int launch_sgemm(const float *x, int64_t x_s0, const int32_t *x_rows, int M, con
     return NQ_LAUNCH_STATUS();
 }
 
+// Few output tiles (a stream or a few of them): a workgroup owns one 16 x 16
+// tile and its sixteen waves deal the 32-k steps among themselves, each loading
+// its operands straight into registers (all in flight together, no staging, no
+// barrier), splitting them there and running its MFMAs; the partial tiles are
+// added in wave order through LDS.  The tiled kernel above walks K in 128-wide stages
+// with a barrier each on as few as 4 CUs: 4 rows of K = 512 (N = 512) take 3.6 us
+// here and 4.9 there, K = 1536 6.1 and 10.4, K = 3584 (N = 128) 11.1 and 21.4;
+// 100 rows of K = 1536 7.7 and 10.6.
+
+constexpr int kDeepWaves = 16;
+
+template <bool kSplit>
+__global__ void __launch_bounds__(kDeepWaves *kWave)
+sgemm_deep_kernel(const float *__restrict__ x, int64_t x_s0, const int32_t *__restrict__ x_rows, int M,
+                  const float *__restrict__ w, int64_t w_s0, int N, int K, const float *__restrict__ bias, int act,
+                  const float *res, int64_t r_s0, const float *__restrict__ scale, float *out, int64_t o_s0,
+                  int tiles_m, int units) {
+    constexpr int kUnroll = 3;  // steps whose loads are in flight
+    __shared__ floatx4_t red[kDeepWaves][kWave];
+    const int per = (units + 7) / 8;
+    const int t = static_cast<int>(blockIdx.x % 8) * per + static_cast<int>(blockIdx.x / 8);
+    if (t >= units) return;
+    const int m0 = (t % tiles_m) * 16, n0 = (t / tiles_m) * 16;
+    const int lane = threadIdx.x & (kWave - 1);
+    const int wave = threadIdx.x / kWave;
+    const int r16 = lane & 15, kq = lane >> 4;
+    int xr = m0 + r16 < M ? m0 + r16 : M - 1;
+    if (x_rows) xr = x_rows[xr];
+    const int nr = n0 + r16 < N ? n0 + r16 : N - 1;
+    const float *xp = x + static_cast<int64_t>(xr) * x_s0 + kq * 8;
+    const float *wp = w + static_cast<int64_t>(nr) * w_s0 + kq * 8;
+
+    floatx4_t acc = floatx4_t{0.f, 0.f, 0.f, 0.f};
+    const int steps = (K + 31) / 32;
+    for (int s0 = wave; s0 < steps; s0 += kDeepWaves * kUnroll) {
+        floatx4_t xv[kUnroll][2], wv[kUnroll][2];
+#pragma unroll
+        for (int u = 0; u < kUnroll; ++u) {
+            const int k0 = (s0 + u * kDeepWaves) * 32;
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const bool in = k0 + kq * 8 + h * 4 < K;  // K % 4 == 0: whole chunks
+                xv[u][h] = in ? *reinterpret_cast<const floatx4_t *>(xp + k0 + h * 4) : floatx4_t{0.f, 0.f, 0.f, 0.f};
+                wv[u][h] = in ? *reinterpret_cast<const floatx4_t *>(wp + k0 + h * 4) : floatx4_t{0.f, 0.f, 0.f, 0.f};
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < kUnroll; ++u) {
+            if constexpr (kSplit) {
+                uint2 h0, l0, h1, l1;
+                sg_split(wv[u][0], h0, l0);
+                sg_split(wv[u][1], h1, l1);
+                const bf16x8_t ah = __builtin_bit_cast(bf16x8_t, make_uint4(h0.x, h0.y, h1.x, h1.y));
+                const bf16x8_t al = __builtin_bit_cast(bf16x8_t, make_uint4(l0.x, l0.y, l1.x, l1.y));
+                sg_split(xv[u][0], h0, l0);
+                sg_split(xv[u][1], h1, l1);
+                const bf16x8_t bh = __builtin_bit_cast(bf16x8_t, make_uint4(h0.x, h0.y, h1.x, h1.y));
+                const bf16x8_t bl = __builtin_bit_cast(bf16x8_t, make_uint4(l0.x, l0.y, l1.x, l1.y));
+                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, bh, acc, 0, 0, 0);
+                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, bl, acc, 0, 0, 0);
+                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, bh, acc, 0, 0, 0);
+            } else {
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[u][h][e], xv[u][h][e], acc, 0, 0, 0);
+            }
+        }
+    }
+    red[wave][lane] = acc;
+    __syncthreads();
+    if (wave != 0) return;
+    const int row = m0 + r16, col = n0 + kq * 4;
+    if (row >= M || col >= N) return;
+    floatx4_t bv = floatx4_t{0.f, 0.f, 0.f, 0.f}, sv = floatx4_t{1.f, 1.f, 1.f, 1.f}, rv = bv;
+    if (bias) bv = *reinterpret_cast<const floatx4_t *>(bias + col);
+    if (scale) sv = *reinterpret_cast<const floatx4_t *>(scale + col);
+    if (res) rv = *reinterpret_cast<const floatx4_t *>(res + static_cast<int64_t>(row) * r_s0 + col);
+#pragma unroll
+    for (int i = 1; i < kDeepWaves; ++i) acc += red[i][lane];
+    floatx4_t v;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        float y = acc[e] + bv[e];
+        if (act) y = sg_gelu(y);
+        v[e] = y * sv[e];
+        if (res) v[e] = rv[e] + v[e];
+    }
+    *reinterpret_cast<floatx4_t *>(out + static_cast<int64_t>(row) * o_s0 + col) = v;
+}
+
 // Row-parallel RMSNorm / LayerNorm of fp32 rows (one wave per row, width % 4 == 0, width <= 1024):
 // RMS: x * rsqrt(mean(x^2) + eps) * w;  LayerNorm: (x - mean) * rsqrt(var + eps) * w + b.
 template <bool kLayer>
@@ -364,6 +456,15 @@ extern "C" int nq_sgemm(const float *x, int64_t x_s0, const int32_t *x_rows, con
 #define NQ_SG(MT, NT, WM, WN, KS, SPLIT)                                                                          \
     launch_sgemm<MT, NT, WM, WN, KS, SPLIT>(x, x_s0, x_rows, M, w, w_s0, N, K, bias, act, res, r_s0, scale, out, \
                                             o_s0, st)
+    // at most one 16 x 16 tile a CU: the waves split K.  More tiles read too much (a tile reads 64 bytes
+    // of operands a k for 256 products): at 288 - 512 tiles of K = 512 the tiled kernel takes 5.2 us and
+    // this one 6.7, at 224 and fewer 5.1 against 4.3
+    if (const int deep = units(16, 16); deep <= 256) {
+        const auto kernel = precision == NQ_MATMUL_HIGH ? sgemm_deep_kernel<true> : sgemm_deep_kernel<false>;
+        hipLaunchKernelGGL(kernel, dim3((deep + 7) / 8 * 8), dim3(kDeepWaves * kWave), 0, st, x, x_s0, x_rows, M, w,
+                           w_s0, N, K, bias, act, res, r_s0, scale, out, o_s0, (M + 15) / 16, deep);
+        return NQ_LAUNCH_STATUS();
+    }
     // 128 x 128 and 64 x 128 tiles over 16 and 8 waves of 32 x 32, 64 x 64 over 8 waves of 16 x 32: more
     // waves per CU hide the stage latency (the codec step's fp32 GEMMs 1.30 -> 1.21 ms against 4 waves per
     // tile).  The smaller tiles take more k per stage (fewer barriers and more bytes in flight per wave).

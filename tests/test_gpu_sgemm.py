@@ -91,6 +91,27 @@ def test_sgemm_epilogues(nq, device, m, n, k, epi, precision):
     assert bool((err <= tol * bound + 1e-6).all()), float((err - tol * bound).max())
 
 
+@pytest.mark.parametrize("precision", [HIGHEST, HIGH])
+@pytest.mark.parametrize("m,n,k", [(1, 4, 4), (4, 512, 512), (16, 16, 512), (17, 20, 516), (4, 128, 3584), (100, 512, 1532),
+                                   (256, 256, 544), (256, 260, 544)])
+def test_sgemm_few_tiles(nq, device, m, n, k, precision):
+    """Both sides of the 256-tile limit of the wave-split kernel, row, column and K tails, K shorter and
+    longer than the waves' first steps, every epilogue in place over a row gather."""
+
+    g = torch.Generator().manual_seed(m * 5 + n + k)
+    x, w = torch.randn(m, k, generator=g), torch.randn(n, k, generator=g) / k ** 0.5
+    b, sc, r = torch.randn(n, generator=g), torch.rand(n, generator=g) + 0.05, torch.randn(m, n, generator=g)
+    rows = torch.randint(0, m, (m,), generator=g, dtype=torch.int32)
+    rd = r.to(device)
+    got = _call(device, x.to(device), w.to(device), x_rows=rows.to(device), bias=b.to(device), act=1, scale=sc.to(device),
+                res=rd, out=rd, precision=precision)
+    xs = x[rows.long()].double()
+    want = r.double() + sc.double() * F.gelu(xs @ w.double().t() + b.double())
+    # GELU's slope is below 1.13
+    bound = 1.13 * (xs.abs() @ w.double().abs().t()) * sc.double()
+    assert bool(((got.cpu().double() - want).abs() <= BOUND[precision] * bound + 1e-6).all())
+
+
 @pytest.mark.parametrize("m,n,k", [(960, 1536, 512), (3840, 128, 3584)])
 def test_high_precision_takes_the_split_products(nq, device, m, n, k):
     g = torch.Generator().manual_seed(m * 3 + k)
