@@ -21,12 +21,19 @@ __device__ __forceinline__ float bf16_to_f32(uint16_t v) {
     return __uint_as_float(static_cast<uint32_t>(v) << 16);
 }
 
-// Round-to-nearest-even float -> bfloat16, quiet NaN preserved (matches torch).
+// Round-to-nearest-even float -> bfloat16, quiet NaN preserved (matches torch): gfx950's conversion
+// instruction, whose result is that of u + 0x7fff + bit 16 (and of the quieted NaN) for every one of the
+// 2^32 floats.  Spelled out in integers it was five instructions and a branch a value, and the short
+// kernels, which spend about 9 ns on fetching each 64 bytes of straight-line code, paid for all of them.
+typedef float cvt_f32x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 cvt_bf16x2 __attribute__((ext_vector_type(2)));
+
+__device__ __forceinline__ uint32_t pack2_bf16(float a, float b) {
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((cvt_f32x2){a, b}, cvt_bf16x2));
+}
+
 __device__ __forceinline__ uint16_t f32_to_bf16(float f) {
-    uint32_t u = __float_as_uint(f);
-    if ((u & 0x7fffffffu) > 0x7f800000u) return static_cast<uint16_t>((u >> 16) | 0x40u);
-    u += 0x7fffu + ((u >> 16) & 1u);
-    return static_cast<uint16_t>(u >> 16);
+    return __builtin_bit_cast(uint16_t, static_cast<__bf16>(f));
 }
 
 // Unpack 8 bf16 held in a 128-bit vector into floats.
@@ -39,10 +46,6 @@ __device__ __forceinline__ void unpack8(const uint4 &p, float (&x)[8]) {
     x[5] = __uint_as_float(p.z & 0xffff0000u);
     x[6] = __uint_as_float(p.w << 16);
     x[7] = __uint_as_float(p.w & 0xffff0000u);
-}
-
-__device__ __forceinline__ uint32_t pack2_bf16(float a, float b) {
-    return static_cast<uint32_t>(f32_to_bf16(a)) | (static_cast<uint32_t>(f32_to_bf16(b)) << 16);
 }
 
 // DPP lane permutations (gfx9 encodings): quad_perm [1,0,3,2], [2,3,0,1],
