@@ -233,44 +233,76 @@ tgemm_kernel(const uint16_t *__restrict__ x, int64_t x_s0, int M, const uint16_t
     }
 }
 
-// 128 x 128 tiles over 4 x 4 waves of 32 x 32 (2 x 2 MFMA tiles each): 68 registers, so the
-// sixteen waves of the one workgroup a CU holds (80 KB of LDS) are resident together.  Measured on
-// the 640-token prefill captures against 64 x 128 tiles of 2 x 2 waves at two workgroups per CU:
-// 20.75 against 21.57 ms per decision (2 x 4 waves of 32 x 64 at 128 x 128: 21.06 ms).
-constexpr int kTgShape[4] = {2, 2, 4, 4};
-constexpr int kTgMT = kTgShape[0], kTgNT = kTgShape[1], kTgWM = kTgShape[2], kTgWN = kTgShape[3];
-constexpr int kTgBM = 16 * kTgMT * kTgWM, kTgBN = 16 * kTgNT * kTgWN;
-constexpr int64_t kTgRound = 256;  // workgroups resident at once (one per CU)
+// Tile shapes of a launch: 128 x 128 over 4 x 4 waves of 32 x 32 (68 registers, 80 KB of LDS: one
+// workgroup of sixteen waves a CU), and 64 x 64 and 96 x 64 over 2 x 2 waves of 32 x 32 and 48 x 32,
+// three workgroups a CU.  Up to about 400 rows the large tiles leave CUs idle or rows padded, and more
+// K slices to fill them write more planes: QKV (N 4096, K 2048), o (2048, 2048) and down (2048, 6144)
+// with the add-RMSNorm took 11.3, 15.5 and 22.5 us at 192 rows and take 9.8 - 10.5, 13.0 and 18.6 in
+// 96 x 64 tiles; 10.2, 14.6 and 22.3 at 128 rows, and 8.3 - 9.3, 11.7 and 17.1 in 64 x 64.  At 448 rows
+// and more the large tiles read half the LDS bytes a product and win (QKV 15.9 us, small tiles 18).
+struct TgShape {
+    int bm, bn;
+    double stage, overlap;  // us a 64-wide K stage of a workgroup costs, and how many it costs alone beyond its share
+    double fixed;           // us of a launch beside its stages
+};
+constexpr TgShape kTgShapes[] = {{128, 128, 0.469, 0.0, 4.92}, {64, 64, 0.160, 0.8, 3.16}, {96, 64, 0.198, 0.8, 3.38}};
+constexpr int kTgBM = 128, kTgBN = 128;  // the large tile; every shape divides its columns
+constexpr double kTgPlane = 0.865e-6;    // us an element of a plane costs, written and read back
 
-// K slices of a launch.  One workgroup fits a CU, so the units run in rounds of 256 and a launch
-// costs about rounds x (slice length + a unit's fixed cost, in K columns): the slice
-// count minimising that (each slice a multiple of 64 columns and at least 256 of them), the fewest
-// slices on a tie.
-int tgemm_splits(int M, int N, int K) {
-    constexpr int64_t kUnitCost = 512;
-    const int64_t tiles = static_cast<int64_t>((M + kTgBM - 1) / kTgBM) * (N / kTgBN);
-    int best = 1;
-    int64_t best_cost = (tiles + kTgRound - 1) / kTgRound * (K + kUnitCost);
-    for (int s = 2; s <= 8; ++s) {
-        if (K % (s * kTgK) || K / s < 256) continue;
-        const int64_t cost = (tiles * s + kTgRound - 1) / kTgRound * (K / s + kUnitCost);
-        if (cost < best_cost) {
-            best_cost = cost;
-            best = s;
+struct TgPlan {
+    int shape, S;
+};
+
+// The shape and the number of K slices (each a multiple of 64 columns and at least 256 of them) with
+// the least time by a model fitted to 200 measured launches of 128 - 640 rows (within 5 % of them on
+// average): a CU's workgroups share it, so a launch takes the stages of the fullest CU.
+TgPlan tgemm_plan(int M, int N, int K) {
+    TgPlan best = {0, 1};
+    double best_cost = 1e30;
+    for (int shape = 0; shape < 3; ++shape) {
+        const TgShape &t = kTgShapes[shape];
+        const int64_t tiles = static_cast<int64_t>((M + t.bm - 1) / t.bm) * (N / t.bn);
+        for (int s = 1; s <= (shape == 0 ? 8 : 4); ++s) {
+            if (s > 1 && (K % (s * kTgK) || K / s < 256)) continue;
+            const double share = static_cast<double>((tiles * s + 255) / 256);
+            const double cost = t.stage * (share + t.overlap) * (K / s / kTgK) + t.fixed +
+                                kTgPlane * s * static_cast<double>(M) * N;
+            if (cost < best_cost) {
+                best_cost = cost;
+                best = {shape, s};
+            }
         }
     }
     return best;
+}
+int tgemm_splits(int M, int N, int K) { return tgemm_plan(M, N, K).S; }
+
+template <int MT, int NT, int WM, int WN, int kMode>
+int launch_tgemm_shape(const uint16_t *x, int64_t x_s0, int M, const uint16_t *w, int64_t w_s0, int N, int K, int S,
+                       uint16_t *out, int64_t o_s0, float *part, hipStream_t st) {
+    constexpr int BM = 16 * MT * WM, BN = 16 * NT * WN;
+    const int tiles_m = (M + BM - 1) / BM, tiles_n = N / BN;
+    const int units = tiles_m * tiles_n * S;
+    hipLaunchKernelGGL((tgemm_kernel<MT, NT, WM, WN, kMode>), dim3((units + 7) / 8 * 8), dim3(WM * WN * kWave), 0, st, x,
+                       x_s0, M, w, w_s0, N, K / S, out, o_s0, part, tiles_m, tiles_n, units);
+    return NQ_LAUNCH_STATUS();
 }
 
 template <int kMode>
 int launch_tgemm(const uint16_t *x, int64_t x_s0, int M, const uint16_t *w, int64_t w_s0, int N, int K, int S,
                  uint16_t *out, int64_t o_s0, float *part, hipStream_t st) {
-    const int tiles_m = (M + kTgBM - 1) / kTgBM, tiles_n = N / kTgBN;
-    const int units = tiles_m * tiles_n * S;
-    hipLaunchKernelGGL((tgemm_kernel<kTgMT, kTgNT, kTgWM, kTgWN, kMode>), dim3((units + 7) / 8 * 8),
-                       dim3(kTgWM * kTgWN * kWave), 0, st, x,
-                       x_s0, M, w, w_s0, N, K / S, out, o_s0, part, tiles_m, tiles_n, units);
-    return NQ_LAUNCH_STATUS();
+#define NQ_TG(MT, NT, WM, WN) \
+    launch_tgemm_shape<MT, NT, WM, WN, kMode>(x, x_s0, M, w, w_s0, N, K, S, out, o_s0, part, st)
+    if constexpr (kMode == kTgSwiglu) {
+        return NQ_TG(2, 2, 4, 4);
+    } else {
+        switch (tgemm_plan(M, N, K).shape) {
+            case 1: return NQ_TG(2, 2, 2, 2);
+            case 2: return NQ_TG(3, 2, 2, 2);
+            default: return NQ_TG(2, 2, 4, 4);
+        }
+    }
+#undef NQ_TG
 }
 
 }  // namespace
