@@ -50,7 +50,7 @@ from .layers import (
     tgemm_workspace_bytes,
 )
 from .errors import KVAllocationError
-from .sampling import sample_with_counter, sample_with_counter_from_planes, sample_with_uniforms
+from .sampling import sample_with_counter_from_planes, sample_with_uniforms
 
 
 @dataclass(frozen=True)
@@ -418,9 +418,8 @@ class TalkerPrefillStep:
     every token (``tgemm``: QKV as split-K planes feeding the q/k norm + RoPE + K/V write, o_proj
     and down through the add-RMSNorm that reduces their planes; FP8 gate/up + SwiGLU as
     ``tgemm_fp8_swiglu``); smaller buckets run the decode step's skinny GEMM with its fused
-    epilogues in pieces of at most CHUNK rows."""
+    epilogues (QKV planes feeding the q/k norm + RoPE + K/V write as well)."""
 
-    CHUNK = 128
     TILED_FROM = 128
 
     def __init__(self, weights: TalkerWeights, context, rows: int, tokens: int, *,
@@ -461,15 +460,15 @@ class TalkerPrefillStep:
         self.fp8 = weights.fp8_gate_up
         # the tiled prefill GEMMs from TILED_FROM tokens; below, the decode GEMM in one piece
         self.tiled = tokens >= self.TILED_FROM
-        piece = min(tokens, self.CHUNK)
+        piece = min(tokens, self.TILED_FROM)
         projections = (
-            (c.qkv_width, c.hidden, _lib.NQ_EPI_NONE),
+            (c.qkv_width, c.hidden, _lib.NQ_EPI_PARTIALS),
             (c.hidden, q_w, _lib.NQ_EPI_ADD_RMSNORM),
             (2 * c.intermediate, c.hidden, _lib.NQ_EPI_SILU_MUL),
             (c.hidden, c.intermediate, _lib.NQ_EPI_ADD_RMSNORM),
         )
         need = max(16, max(linear_workspace_bytes(piece, n, k, e) for n, k, e in projections),
-                   linear_workspace_bytes(rows, c.vocab, c.hidden, _lib.NQ_EPI_NONE))
+                   linear_workspace_bytes(rows, c.vocab, c.hidden, _lib.NQ_EPI_PARTIALS))
         if self.tiled:
             need = max(need, tgemm_workspace_bytes(tokens, c.qkv_width, c.hidden, _lib.NQ_EPI_PARTIALS),
                        tgemm_workspace_bytes(tokens, c.hidden, q_w, _lib.NQ_EPI_ADD_RMSNORM),
@@ -490,18 +489,12 @@ class TalkerPrefillStep:
         self._no_ids = torch.zeros((0, rows), dtype=torch.long, device=dev)
         self._no_tables = torch.zeros((0, 1, c.hidden), **bf)
 
-    def _pieces(self):
-        t = self.tokens_capacity
-        return [(r0, min(t, r0 + self.CHUNK)) for r0 in range(0, t, self.CHUNK)]
-
     def forward(self) -> torch.Tensor:
         c = self.w.config
         ctx = self.context
         t = self.tokens_capacity
         ws = self.linear_workspace
         q_w = c.num_qo_heads * c.head_dim
-        kv_w = c.num_kv_heads * c.head_dim
-        pieces = self._pieces()
         # materialize_prefill and the first input norm, one launch
         prefill_embed_rmsnorm(self.text_ids, self.w.text_embedding, self.codec_ids, self.w.codec_embedding,
                               self.codec_mask, self.w.layers[0].input_norm, c.rms_eps, self.residual, self.hidden,
@@ -530,24 +523,19 @@ class TalkerPrefillStep:
                 if trace is not None:
                     trace[index + 1].copy_(self.residual)
                 continue
-            for a, b in pieces:
-                linear(self.hidden[a:b], layer.qkv, out=self.qkv[a:b], workspace=ws)
+            # fewer tokens: the decode step's projections and fused epilogues, all tokens in one piece
+            splits = linear_partials(self.hidden, layer.qkv, ws)
             q = self.qkv[:, :q_w].view(t, c.num_qo_heads, c.head_dim)
-            k = self.qkv[:, q_w : q_w + kv_w].view(t, c.num_kv_heads, c.head_dim)
-            v = self.qkv[:, q_w + kv_w :].view(t, c.num_kv_heads, c.head_dim)
-            attended = ctx.attend(layer.attention, q, k, v).view(t, q_w)
-            for a, b in pieces:
-                if self.fp8:
-                    linear_add_rmsnorm_fp8(attended[a:b], layer.o, self.residual[a:b], layer.post_norm, c.rms_eps,
-                                           self.act_q[a:b], self.act_scales[a:b], ws)
-                    linear_fp8_swiglu(self.act_q[a:b], self.act_scales[a:b], layer.gate_up_packed,
-                                      layer.gate_up_scales, self.act[a:b], weight_q=layer.gate_up_q, workspace=ws)
-                else:
-                    linear_add_rmsnorm(attended[a:b], layer.o, self.residual[a:b], layer.post_norm, c.rms_eps,
-                                       self.hidden[a:b], ws)
-                    linear_silu_mul(self.hidden[a:b], layer.gate_up, out=self.act[a:b], workspace=ws)
-                linear_add_rmsnorm(self.act[a:b], layer.down, self.residual[a:b], nxt, c.rms_eps, self.hidden[a:b],
-                                   ws)
+            attended = ctx.attend_partials(layer.attention, ws, splits, q).view(t, q_w)
+            if self.fp8:
+                linear_add_rmsnorm_fp8(attended, layer.o, self.residual, layer.post_norm, c.rms_eps, self.act_q,
+                                       self.act_scales, ws)
+                linear_fp8_swiglu(self.act_q, self.act_scales, layer.gate_up_packed, layer.gate_up_scales, self.act,
+                                  weight_q=layer.gate_up_q, workspace=ws)
+            else:
+                linear_add_rmsnorm(attended, layer.o, self.residual, layer.post_norm, c.rms_eps, self.hidden, ws)
+                linear_silu_mul(self.hidden, layer.gate_up, out=self.act, workspace=ws)
+            linear_add_rmsnorm(self.act, layer.down, self.residual, nxt, c.rms_eps, self.hidden, ws)
             if trace is not None:
                 trace[index + 1].copy_(self.residual)
         ctx.advance_sequence_lengths()
@@ -559,10 +547,12 @@ class TalkerPrefillStep:
             torch.sub(qo[1 : self.rows + 1], 1, out=self.last)
         gather_sum_rows(self.last, self.hidden, self._no_ids, self._no_tables, self.last_hidden,
                         status=self.embed_status)
-        linear(self.last_hidden, self.w.codec_head, out=self.logits, workspace=ws)
-        sample_with_counter(self.logits, self.temperature, self.top_k, self.top_p, self.seed, self.offsets,
-                            repetition_penalty=self.penalty, seen_token_mask=self.seen, mask_from=c.codec_vocab,
-                            eos_id=c.eos_id, suppress_eos=self.suppress_eos, update_seen=True, out=self.tokens)
+        splits = linear_partials(self.last_hidden, self.w.codec_head, ws)
+        planes = ws[: splits * self.rows * c.vocab * 4].view(torch.float32).view(splits, self.rows, c.vocab)
+        sample_with_counter_from_planes(planes, self.temperature, self.top_k, self.top_p, self.seed, self.offsets,
+                                        logits_out=self.logits, repetition_penalty=self.penalty,
+                                        seen_token_mask=self.seen, mask_from=c.codec_vocab, eos_id=c.eos_id,
+                                        suppress_eos=self.suppress_eos, update_seen=True, out=self.tokens)
         TalkerDecodeStep._report(self)
         return self.tokens
 
