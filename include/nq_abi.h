@@ -560,6 +560,35 @@ int nq_fp8_pack_swiglu(const uint8_t *q, int64_t q_s0, int I, int K, uint8_t *pa
  */
 int nq_linear_swiglu(const uint16_t *x, int64_t x_s0, int M, const uint16_t *packed, int64_t w_s0, int I, int K,
                      uint16_t *out, int64_t o_s0, void *stream);
+
+/*
+ * Projections of a few rows (at most 16), and the add-RMSNorm before them done
+ * by their own workgroups.  nq_decode_linear leaves S = nq_decode_linear_splits
+ * fp32 planes [S][M][N] of X . W^T (-1 / NQ_ERR_UNSUPPORTED: not a shape it
+ * takes; N % 16 == 0, K % 32 == 0).  The norm forms take their rows from such
+ * planes of an earlier projection (in_planes [in_splits][M][K], at most 4):
+ * h = bf16(residual + bf16(sum)), x = rmsnorm(h) * norm_weight, the bits of
+ * nq_linear's NQ_EPI_ADD_RMSNORM; h goes to residual_out (another buffer than
+ * residual), x to x_out when given.  nq_decode_norm_linear writes one plane
+ * [1][M][N]; it and nq_decode_norm_swiglu / nq_decode_norm_fp8_swiglu (x, or its
+ * codes, through nq_linear_swiglu / nq_linear_fp8_swiglu) take K = 1024 (up to
+ * 8 rows) and K = 2048 (up to 4), the bf16 SwiGLU K = 1024 alone and the FP8
+ * one K = 2048 alone, else NQ_ERR_UNSUPPORTED.  The planes read and the planes
+ * written may not overlap.
+ */
+int nq_decode_linear_splits(int M, int N, int K);
+int nq_decode_linear(const uint16_t *x, int64_t x_s0, const uint16_t *w, int64_t w_s0, int M, int N, int K,
+                     float *planes, int64_t planes_bytes, void *stream);
+int nq_decode_norm_linear(const float *in_planes, int in_splits, const uint16_t *residual, uint16_t *residual_out,
+                          const uint16_t *norm_weight, float eps, uint16_t *x_out, const uint16_t *w, int64_t w_s0,
+                          int M, int N, int K, float *planes, int64_t planes_bytes, void *stream);
+int nq_decode_norm_swiglu(const float *in_planes, int in_splits, const uint16_t *residual, uint16_t *residual_out,
+                          const uint16_t *norm_weight, float eps, int M, const uint16_t *packed, int64_t w_s0, int I,
+                          int K, uint16_t *out, int64_t o_s0, void *stream);
+int nq_decode_norm_fp8_swiglu(const float *in_planes, int in_splits, const uint16_t *residual,
+                              uint16_t *residual_out, const uint16_t *norm_weight, float eps, int M,
+                              const uint8_t *packed, int64_t w_s0, const float *sw, int64_t sw_s0, int I, int K,
+                              uint16_t *out, int64_t o_s0, void *stream);
 int nq_linear_fp8_swiglu(const uint8_t *xq, int64_t x_s0, const float *sx, int64_t sx_s0, int M,
                          const uint8_t *packed, int64_t w_s0, const float *sw, int64_t sw_s0, int I, int K,
                          uint16_t *out, int64_t o_s0, void *stream);

@@ -41,6 +41,11 @@ import torch.nn.functional as F
 from . import _lib
 from .kernels import qkv_partials_rope_short_attention_
 from .layers import (
+    NormRows,
+    decode_linear,
+    decode_linear_splits,
+    decode_norm_linear,
+    decode_norm_swiglu,
     embed_add_rmsnorm,
     gather_sum_rows,
     linear,
@@ -227,6 +232,16 @@ class CodePredictorFrame:
             (c.vocab, c.hidden, _lib.NQ_EPI_PARTIALS),  # planes feed the sampler
         )
         need = max(linear_workspace_bytes(rows, n, k, e) for n, k, e in shapes)
+        # few rows: projections that normalise their rows themselves, over two alternating plane
+        # regions and two residual buffers (a kernel reads one of each and writes the other)
+        few = ((c.qkv_width, c.hidden), (c.hidden, c.num_qo_heads * c.head_dim), (c.hidden, c.intermediate),
+               (c.vocab, c.hidden))
+        self.few = rows <= self.FEW_ROWS and c.hidden == 1024 and c.intermediate % 16 == 0 and all(
+            decode_linear_splits(rows, n, k) > 0 for n, k in few)
+        if self.few:
+            self.h2 = torch.zeros(rows, c.hidden, **bf)
+            self._region = max(decode_linear_splits(rows, n, k) * rows * n * 4 for n, k in few)
+            need = max(need, 2 * self._region)
         self.workspace = torch.empty(max(need, 16), dtype=torch.uint8, device=dev)
         # optional [groups, layers + 2, rows, hidden] bf16 record of each pass: the residual stream
         # at the pass start and after every layer, then the normalised hidden state the head reads
@@ -236,6 +251,30 @@ class CodePredictorFrame:
         # otherwise a sampler with the reference's signature (logits, temperature, top_k, top_p, seed,
         # offset) -> tokens, called on each group's bf16 logits (read when the forward is recorded)
         self.sampler = None
+
+    # the most rows of 1024 that every workgroup of a projection normalises for itself
+    FEW_ROWS = 8
+
+    def _layers_few(self, cache_pos: int):
+        """The layers from self.h and its first input norm self.x with five launches each: QKV, attention,
+        o, gate/up + SwiGLU, down, the add-RMSNorms inside the projections after them.  Returns the final
+        norm's rows, for the head."""
+
+        c, n = self.w.config, self.rows
+        a, b = self.workspace[: self._region], self.workspace[self._region: 2 * self._region]
+        h, h2 = self.h, self.h2
+        positions = self.position_ids[:, cache_pos]
+        splits = decode_linear(self.x, self.w.layers[0].qkv, b)
+        for index, L in enumerate(self.w.layers):
+            if index:
+                splits = decode_norm_linear(NormRows(a, down, h2, h, L.input_norm, c.rms_eps), L.qkv, b)
+            cache = self.kv_cache[index]
+            qkv_partials_rope_short_attention_(b, splits, self.q, L.q_norm, L.k_norm, positions, c.rms_eps,
+                                               c.rope_theta, cache[:, 0], cache[:, 1], cache_pos, self.att)
+            splits = decode_linear(self.att.view(n, -1), L.o, a)
+            decode_norm_swiglu(NormRows(a, splits, h, h2, L.post_norm, c.rms_eps), L.gate_up_packed, self.act)
+            down = decode_linear(self.act, L.down, a)
+        return NormRows(a, down, h2, h, self.w.final_norm, c.rms_eps, self.x)
 
     def _layers(self, cache_pos: int, normed: bool = False) -> None:
         """The 5 layers at cache position ``cache_pos``; ``normed``: self.x already holds the first
@@ -272,23 +311,35 @@ class CodePredictorFrame:
         groups = c.num_code_groups
         # pass 0: the talker hidden state fills cache position 0
         linear(self.past_hidden, w.proj_w, out=self.h, workspace=ws, bias=w.proj_b)
-        self._layers(0)
+        few = self.few and self.trace is None and self.use_counter_rng and self.sampler is None
+        if few:
+            rmsnorm(self.h, w.layers[0].input_norm, c.rms_eps, out=self.x)
+            self._layers_few(0)
+        else:
+            self._layers(0)
         self.frames[:, 0].copy_(self.layer0_token)
         # the next input (a projected embedding row) and the first input norm in one launch
         first_norm = w.layers[0].input_norm
         embed_add_rmsnorm(self.layer0_token, w.projected_layer0, None, first_norm, c.rms_eps, self.h, self.x)
         for group in range(1, groups):
-            self._layers(group, normed=True)
             logits = self.logits[group - 1]
             token = self.tokens[group - 1]
+            head = w.lm_head[group - 1]
+            planes = ws  # the head's planes
+            if few:
+                planes = ws[self._region:]
+                splits = decode_norm_linear(self._layers_few(group), head, planes)
+            else:
+                self._layers(group, normed=True)
             if self.sampler is not None:
                 linear(self.x, w.lm_head[group - 1], out=logits, workspace=ws)
                 token.copy_(self.sampler(logits, self.temperature, self.top_k, self.top_p, self.seed,
                                          self.offsets[:, group - 1]))
             elif self.use_counter_rng:
                 # the head's split-K planes summed, rounded and drawn from in the sampling launch
-                splits = linear_partials(self.x, w.lm_head[group - 1], ws)
-                planes = ws[: splits * self.rows * c.vocab * 4].view(torch.float32).view(splits, self.rows, c.vocab)
+                if not few:
+                    splits = linear_partials(self.x, head, ws)
+                planes = planes[: splits * self.rows * c.vocab * 4].view(torch.float32).view(splits, self.rows, c.vocab)
                 sample_with_counter_from_planes(planes, self.temperature, self.top_k, self.top_p, self.seed,
                                                 self.offsets[:, group - 1], logits_out=logits, out=token)
             else:

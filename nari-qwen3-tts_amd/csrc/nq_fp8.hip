@@ -21,6 +21,7 @@
 // half the K splits.
 #include "nq_common.h"
 #include "nq_internal.h"
+#include "nq_norm_rows.h"
 
 namespace nq {
 
@@ -269,11 +270,11 @@ static_assert(kSwRows / 16 == kSwQuarters, "the wave of quarter q finishes 16-ro
 // count 9.5 in four.  At 8 rows the 25.2 MB of weights are 3.6 us of it at 7 TB/s of cache.
 // One or two column tiles a workgroup instead of three: 7.1 and 7.4 us at 8 rows, 10.2 and
 // 8.8 at 32.  The sums and bits of a row do not depend on MT.
-template <int K, int MT>
+template <int K, int MT, bool kNorm = false>
 __global__ void __launch_bounds__(kSwThreads)
 fp8_swiglu_kernel(const uint8_t *__restrict__ x, int64_t x_s0, const float *__restrict__ sx, int64_t sx_s0, int M,
                   const uint8_t *__restrict__ w, int64_t w_s0, const float *__restrict__ sw, int64_t sw_s0, int I,
-                  uint16_t *__restrict__ out, int64_t o_s0) {
+                  uint16_t *__restrict__ out, int64_t o_s0, NormRowsSrc norm) {
     constexpr int KB = K / 128;                    // K blocks
     constexpr int kRows = 16 * MT;
     constexpr int QS = K / kSwQuarters / 128;      // K blocks per quarter
@@ -303,21 +304,27 @@ fp8_swiglu_kernel(const uint8_t *__restrict__ x, int64_t x_s0, const float *__re
     // at the same moment.  Vector i of the thread is block vector rot(i).
     const int rot = (blockIdx.x * 258) % kVec;
     auto rot_of = [&](int i) { return i + rot < kVec ? i + rot : i + rot - kVec; };
-    uint4 xr[kPer];
+    uint4 xr[kNorm ? 1 : kPer];
+    float sr[kNorm ? 1 : kSxPer];
+    using Rows = NormRows<K, kSwThreads, kNorm ? 2 : 1>;  // kNorm: up to 4 rows are asked for
+    Rows rows_in;
+    if constexpr (kNorm) {
+        rows_in.load(norm, M);
+    } else {
 #pragma unroll
-    for (int u = 0; u < kPer; ++u) {
-        const int i = threadIdx.x + u * kSwThreads;
-        const int v = rot_of(i);
-        const int row = v / (K / 16), c = v % (K / 16);
-        xr[u] = (i < kVec && row < M) ? *reinterpret_cast<const uint4 *>(x + row * x_s0 + c * 16)
-                                      : make_uint4(0, 0, 0, 0);
-    }
-    float sr[kSxPer];
+        for (int u = 0; u < kPer; ++u) {
+            const int i = threadIdx.x + u * kSwThreads;
+            const int v = rot_of(i);
+            const int row = v / (K / 16), c = v % (K / 16);
+            xr[u] = (i < kVec && row < M) ? *reinterpret_cast<const uint4 *>(x + row * x_s0 + c * 16)
+                                          : make_uint4(0, 0, 0, 0);
+        }
 #pragma unroll
-    for (int u = 0; u < kSxPer; ++u) {
-        const int i = threadIdx.x + u * kSwThreads;
-        // element i of the [K block][row] table
-        sr[u] = (i < kSx && i % kRows < M) ? sx[(i % kRows) * sx_s0 + i / kRows] : 0.f;
+        for (int u = 0; u < kSxPer; ++u) {
+            const int i = threadIdx.x + u * kSwThreads;
+            // element i of the [K block][row] table
+            sr[u] = (i < kSx && i % kRows < M) ? sx[(i % kRows) * sx_s0 + i / kRows] : 0.f;
+        }
     }
     // 2. the wave's weights (16 packed rows over its K quarter) and scales:
     // gate rows 8t.. lie in 128-row block t / 16, up rows in (I + 8t) / 128
@@ -339,7 +346,19 @@ fp8_swiglu_kernel(const uint8_t *__restrict__ x, int64_t x_s0, const float *__re
     }
     // keep every weight load ahead of the wait for the X block
     __builtin_amdgcn_sched_barrier(0);
-    {
+    if constexpr (kNorm) {
+        // the normalised rows quantized as add_rmsnorm_kernel stores them: 16 threads hold a 128-column group
+        __shared__ float red[Rows::kRows * Rows::kParts];
+        rows_in.finish(norm, M, blockIdx.x == 0, red, [&](int row, int col, const uint4 &packed) {
+            float y[8], amax = 0.f;
+            unpack8(packed, y);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) amax = fmaxf(amax, fabsf(y[e]));
+            const float sc = row_group_scale(group_max<16>(amax));
+            *reinterpret_cast<uint2 *>(xs + Lds::stage_offset(row, col / 16) + (col & 8)) = e4m3_pack8(y, sc);
+            if ((threadIdx.x & 15) == 0) sxs[col / 128 * kRows + row] = sc;
+        });
+    } else {
         // adjacent vectors belong to the two LDS planes (whose starts share banks): each store
         // writes one plane, so its active lanes fill consecutive 16-byte chunks
 #pragma unroll
@@ -784,7 +803,25 @@ extern "C" int nq_linear_fp8_swiglu(const uint8_t *xq, int64_t x_s0, const float
                         : M <= 32 ? fp8_swiglu_kernel<kSwK, 2>
                                   : fp8_swiglu_kernel<kSwK, 4>;
     hipLaunchKernelGGL(kernel, dim3(I / (8 * kSwTiles)), dim3(kSwThreads), 0, static_cast<hipStream_t>(stream), xq,
-                       x_s0, sx, sx_s0, M, packed, w_s0, sw, sw_s0, I, out, o_s0);
+                       x_s0, sx, sx_s0, M, packed, w_s0, sw, sw_s0, I, out, o_s0, NormRowsSrc{});
+    return NQ_LAUNCH_STATUS();
+}
+
+extern "C" int nq_decode_norm_fp8_swiglu(const float *in_planes, int in_splits, const uint16_t *residual,
+                                         uint16_t *residual_out, const uint16_t *norm_weight, float eps, int M,
+                                         const uint8_t *packed, int64_t w_s0, const float *sw, int64_t sw_s0, int I,
+                                         int K, uint16_t *out, int64_t o_s0, void *stream) {
+    NQ_CHECK_ARG(packed && sw && out && M > 0 && I > 0 && K > 0);
+    NQ_CHECK_ARG(in_planes && residual && residual_out && norm_weight && residual != residual_out);
+    if (M > 4 || in_splits < 1 || in_splits > kNormRowsPlanes || K != kSwK || I % (8 * kSwTiles) != 0 || I % 128 != 0)
+        return NQ_ERR_UNSUPPORTED;
+    NQ_CHECK_ARG(al16(in_planes) && al16(residual) && al16(residual_out) && al16(norm_weight) && al16(packed));
+    NQ_CHECK_ARG(w_s0 >= K && w_s0 % 16 == 0 && sw_s0 >= K / 128 && o_s0 >= I && o_s0 % 2 == 0);
+    NQ_CHECK_ARG(reinterpret_cast<uintptr_t>(out) % 4 == 0);
+    const NormRowsSrc norm{in_planes, in_splits, residual, residual_out, norm_weight, eps, nullptr};
+    hipLaunchKernelGGL((fp8_swiglu_kernel<kSwK, 1, true>), dim3(I / (8 * kSwTiles)), dim3(kSwThreads), 0,
+                       static_cast<hipStream_t>(stream), nullptr, 0, nullptr, 0, M, packed, w_s0, sw, sw_s0, I, out,
+                       o_s0, norm);
     return NQ_LAUNCH_STATUS();
 }
 

@@ -17,6 +17,7 @@
 // single slice the bf16 result is written directly.
 #include "nq_common.h"
 #include "nq_internal.h"
+#include "nq_norm_rows.h"
 
 namespace nq {
 namespace {
@@ -297,10 +298,10 @@ void dispatch_gemm(const uint16_t *x, int64_t x_s0, int M, const uint16_t *w, in
 constexpr int kBsQuarters = 4;
 constexpr int kBsK = 1024;
 
-template <int K, int MT, int kTiles>
+template <int K, int MT, int kTiles, bool kNorm = false>
 __global__ void __launch_bounds__(kTiles * kBsQuarters * kWave)
 bf16_swiglu_kernel(const uint16_t *__restrict__ x, int64_t x_s0, int M, const uint16_t *__restrict__ w,
-                   int64_t w_s0, uint16_t *__restrict__ out, int64_t o_s0) {
+                   int64_t w_s0, uint16_t *__restrict__ out, int64_t o_s0, NormRowsSrc norm) {
     constexpr int kRows = 16 * MT;
     constexpr int kThreads = kTiles * kBsQuarters * kWave;
     constexpr int XP = x_pitch<K>();   // LDS row pitch (bf16)
@@ -327,14 +328,20 @@ bf16_swiglu_kernel(const uint16_t *__restrict__ x, int64_t x_s0, int M, const ui
     constexpr int kPer = (kVec + kThreads - 1) / kThreads;
     const int rot = (blockIdx.x * 258) % kVec;
     auto rot_of = [&](int i) { return i + rot < kVec ? i + rot : i + rot - kVec; };
-    uint4 xr[kPer];
+    uint4 xr[kNorm ? 1 : kPer];
+    using Rows = NormRows<K, kThreads, kNorm ? 2 : 1>;
+    Rows rows_in;
+    if constexpr (kNorm) {
+        rows_in.load(norm, M);
+    } else {
 #pragma unroll
-    for (int u = 0; u < kPer; ++u) {
-        const int i = threadIdx.x + u * kThreads;
-        const int v = rot_of(i);
-        const int row = v / (K / 8), c = v % (K / 8);
-        xr[u] = (i < kVec && row < rows) ? *reinterpret_cast<const uint4 *>(x + (row0 + row) * x_s0 + c * 8)
-                                         : make_uint4(0, 0, 0, 0);
+        for (int u = 0; u < kPer; ++u) {
+            const int i = threadIdx.x + u * kThreads;
+            const int v = rot_of(i);
+            const int row = v / (K / 8), c = v % (K / 8);
+            xr[u] = (i < kVec && row < rows) ? *reinterpret_cast<const uint4 *>(x + (row0 + row) * x_s0 + c * 8)
+                                             : make_uint4(0, 0, 0, 0);
+        }
     }
     // 2. the wave's weights: 16 packed rows over its K quarter
     uint4 wr[QS];
@@ -344,11 +351,17 @@ bf16_swiglu_kernel(const uint16_t *__restrict__ x, int64_t x_s0, int M, const ui
         for (int j = 0; j < QS; ++j) wr[j] = *reinterpret_cast<const uint4 *>(wrow + j * 32);
     }
     __builtin_amdgcn_sched_barrier(0);
+    if constexpr (kNorm) {
+        __shared__ float red[Rows::kRows * Rows::kParts];
+        rows_in.finish(norm, M, blockIdx.x == 0, red,
+                       [&](int row, int col, const uint4 &y) { *reinterpret_cast<uint4 *>(xs + row * XP + col) = y; });
+    } else {
 #pragma unroll
-    for (int u = 0; u < kPer; ++u) {
-        const int i = threadIdx.x + u * kThreads;
-        const int v = rot_of(i);
-        if (i < kVec) *reinterpret_cast<uint4 *>(xs + (v / (K / 8)) * XP + (v % (K / 8)) * 8) = xr[u];
+        for (int u = 0; u < kPer; ++u) {
+            const int i = threadIdx.x + u * kThreads;
+            const int v = rot_of(i);
+            if (i < kVec) *reinterpret_cast<uint4 *>(xs + (v / (K / 8)) * XP + (v % (K / 8)) * 8) = xr[u];
+        }
     }
     __syncthreads();
 
@@ -406,6 +419,118 @@ bf16_swiglu_kernel(const uint16_t *__restrict__ x, int64_t x_s0, int M, const ui
         a[e] = g / (1.0f + expf(-g)) * u;
     }
     *reinterpret_cast<uint32_t *>(out + (row0 + row) * o_s0 + tile * 8 + kq * 2) = pack2_bf16(a[0], a[1]);
+}
+
+
+// ---------------------------------------------------------------------------
+// Projections of a few rows (decode buckets up to 16 rows, a single 16-row
+// MFMA tile).  gemm_kernel's workgroup stages X[:, slice] and streams 64
+// columns of weights; here a workgroup owns 16 columns and its eight waves
+// split the K slice, each with its weights, and its own part of X, straight
+// from memory in MFMA operand shape, all loads in flight at entry, and the
+// partial tiles are added in wave order through LDS.  So a slice is long and
+// the planes are few, which lets the consumer do the add-RMSNorm itself
+// (kNorm: X is the normalised rows of a NormRowsSrc, whole K).  Back to back in a
+// graph, one row of 1024: QKV (N 2048) 2.3 us against gemm_kernel's 2.7, o (N
+// 1024) 2.3 against 2.4, down (K 3072) 3.0 against 2.9, and with the norm in
+// front QKV 2.6.  It pays by the launches it saves: a layer takes five instead of
+// seven.  That holds while a workgroup's share of the rows is small: with four
+// row vectors a thread the code predictor's frame takes 1640 us instead of 2100 at
+// one row, 1990 instead of 2160 at 8 and 2190 instead of 2180 at 12, the talker
+// step of four layers 169 instead of 190 us at one row, 195 instead of 201 at 4 and
+// 209 instead of 200 at 6; so two vectors, 8192 values, are the most it takes.
+
+constexpr int kSmallWaves = 8;
+constexpr int kSmallThreads = kSmallWaves * kWave;
+constexpr int kSmallRows = 16;
+constexpr int kSmallSteps = 12;        // 32-k steps a wave at most
+constexpr int kSmallVecs = 2;          // kNorm: row vectors a thread at most (8 columns each)
+
+template <int K_, bool kNorm, int kSteps>
+__global__ void __launch_bounds__(kSmallThreads)
+small_gemm_kernel(const uint16_t *__restrict__ x, int64_t x_s0, int M, const uint16_t *__restrict__ w, int64_t w_s0,
+                  int N, int slice_k, float *__restrict__ part, NormRowsSrc norm) {
+    using Rows = NormRows<kNorm ? K_ : 1024, kSmallThreads, kNorm ? kSmallVecs : 1>;
+    constexpr int XP = x_pitch<K_>();
+    constexpr int kRowsIn = Rows::kRows < kSmallRows ? Rows::kRows : kSmallRows;
+    __shared__ __attribute__((aligned(16))) uint16_t xs[kNorm ? kRowsIn * XP : 8];
+    __shared__ float4 red4[kSmallWaves][kWave];
+    const int lane = threadIdx.x & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int r16 = lane & 15, kq = lane >> 4;
+    const int col0 = blockIdx.x * 16;
+    const int k0 = blockIdx.y * slice_k;
+    const int steps = slice_k / 32;
+    const int each = (steps + kSmallWaves - 1) / kSmallWaves;
+    const int first = wave * each;
+    const int count = steps - first < each ? steps - first : each;  // <= 0: the wave has none
+    const int s0 = count > 0 ? first : 0;
+    const int xrow = r16 < M ? r16 : 0;  // rows past M repeat row 0; their sums are not stored
+
+    Rows rows_in;
+    if constexpr (kNorm) rows_in.load(norm, M);
+    uint4 xr[kNorm ? 1 : kSteps], wr[kSteps];
+    const uint16_t *wp = w + static_cast<int64_t>(col0 + r16) * w_s0 + k0 + s0 * 32 + kq * 8;
+    if constexpr (!kNorm) {
+        const uint16_t *xp = x + xrow * x_s0 + k0 + s0 * 32 + kq * 8;
+        // no branch between the loads (steps the wave has not got repeat its first, and count as zeros
+        // below): with one the compiler moves each load to its use, and they run one after the other
+#pragma unroll
+        for (int i = 0; i < kSteps; ++i) xr[i] = *reinterpret_cast<const uint4 *>(xp + (i < count ? i : 0) * 32);
+    }
+#pragma unroll
+    for (int i = 0; i < kSteps; ++i) wr[i] = *reinterpret_cast<const uint4 *>(wp + (i < count ? i : 0) * 32);
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (kNorm) {
+        rows_in.finish(norm, M, blockIdx.x == 0, reinterpret_cast<float *>(red4),
+                       [&](int row, int col, const uint4 &y) { *reinterpret_cast<uint4 *>(xs + row * XP + col) = y; });
+        __syncthreads();
+    }
+    floatx4_t acc = floatx4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < kSteps; ++i) {
+        uint4 b;
+        if constexpr (kNorm)
+            b = *reinterpret_cast<const uint4 *>(xs + xrow * XP + (s0 + (i < count ? i : 0)) * 32 + kq * 8);
+        else
+            b = xr[i];
+        if (i >= count) wr[i] = b = make_uint4(0, 0, 0, 0);  // not skipped: an MFMA runs whatever EXEC says
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(wr[i]), as_bf16x8(b), acc, 0, 0, 0);
+    }
+    red4[wave][lane] = make_float4(acc[0], acc[1], acc[2], acc[3]);
+    __syncthreads();
+    if (wave != 0 || r16 >= M) return;
+    float4 sum = red4[0][lane];
+#pragma unroll
+    for (int i = 1; i < kSmallWaves; ++i) {
+        const float4 v = red4[i][lane];
+        sum.x += v.x;
+        sum.y += v.y;
+        sum.z += v.z;
+        sum.w += v.w;
+    }
+    *reinterpret_cast<float4 *>(part + (static_cast<int64_t>(blockIdx.y) * M + r16) * N + col0 + kq * 4) = sum;
+}
+
+// K slices of a few-row projection: the fewest (1, 2, 4) whose workgroups fill the CUs, else the most.
+int small_slices(int M, int N, int K) {
+    if (M < 1 || M > kSmallRows || N % 16 != 0 || K % 32 != 0) return -1;
+    int best = -1;
+    for (int s = 1; s <= kNormRowsPlanes; s *= 2) {
+        if (K % (32 * s) != 0 || K / 32 / s > kSmallSteps * kSmallWaves) continue;
+        best = s;
+        if (N / 16 * s >= 256) break;
+    }
+    return best;
+}
+
+int check_norm_rows(const NormRowsSrc &n, int M, int K) {
+    NQ_CHECK_ARG(n.planes && n.residual_in && n.residual_out && n.weight && n.residual_in != n.residual_out);
+    if (n.S < 1 || n.S > kNormRowsPlanes || M * K > kSmallVecs * kSmallThreads * 8) return NQ_ERR_UNSUPPORTED;
+    NQ_CHECK_ARG(((reinterpret_cast<uintptr_t>(n.planes) | reinterpret_cast<uintptr_t>(n.residual_in) |
+                   reinterpret_cast<uintptr_t>(n.residual_out) | reinterpret_cast<uintptr_t>(n.weight) |
+                   reinterpret_cast<uintptr_t>(n.x_out)) & 15) == 0);
+    return NQ_OK;
 }
 
 }  // namespace
@@ -522,7 +647,7 @@ extern "C" int nq_linear_swiglu(const uint16_t *x, int64_t x_s0, int M, const ui
     hipLaunchKernelGGL((nq::bf16_swiglu_kernel<nq::kBsK, MT, TL>),                                       \
                        dim3(static_cast<unsigned>(I / (8 * TL)), static_cast<unsigned>(blocks)),          \
                        dim3(TL * nq::kBsQuarters * nq::kWave), 0, static_cast<hipStream_t>(stream), x, x_s0, \
-                       M, packed, w_s0, out, o_s0)
+                       M, packed, w_s0, out, o_s0, nq::NormRowsSrc{})
     if (mt == 1 && I % 16 == 0)
         NQ_BF16_SWIGLU(1, 2);
     else if (mt == 2 && I % 16 == 0)
@@ -532,5 +657,71 @@ extern "C" int nq_linear_swiglu(const uint16_t *x, int64_t x_s0, int M, const ui
     else
         NQ_BF16_SWIGLU(4, 3);
 #undef NQ_BF16_SWIGLU
+    return NQ_LAUNCH_STATUS();
+}
+
+extern "C" int nq_decode_linear_splits(int M, int N, int K) {
+    const int S = N > 0 && K > 0 ? nq::small_slices(M, N, K) : -1;
+    return S > 0 ? S : -1;
+}
+
+namespace {
+
+// the launch whose waves hold the fewest 32-k steps that cover the slice
+int launch_small(const uint16_t *x, int64_t x_s0, int M, const uint16_t *w, int64_t w_s0, int N, int K, int S,
+                 float *part, hipStream_t st) {
+    const int each = (K / S / 32 + nq::kSmallWaves - 1) / nq::kSmallWaves;
+    const auto kernel = each <= 2   ? nq::small_gemm_kernel<1024, false, 2>
+                        : each <= 4 ? nq::small_gemm_kernel<1024, false, 4>
+                        : each <= 8 ? nq::small_gemm_kernel<1024, false, 8>
+                                    : nq::small_gemm_kernel<1024, false, nq::kSmallSteps>;
+    hipLaunchKernelGGL(kernel, dim3(N / 16, S), dim3(nq::kSmallThreads), 0, st, x, x_s0, M, w, w_s0, N, K / S, part,
+                       nq::NormRowsSrc{});
+    return NQ_LAUNCH_STATUS();
+}
+
+}  // namespace
+
+extern "C" int nq_decode_linear(const uint16_t *x, int64_t x_s0, const uint16_t *w, int64_t w_s0, int M, int N, int K,
+                                float *planes, int64_t planes_bytes, void *stream) {
+    NQ_CHECK_ARG(x && w && planes && M > 0 && N > 0 && K > 0);
+    const int S = nq_decode_linear_splits(M, N, K);
+    if (S < 0) return NQ_ERR_UNSUPPORTED;
+    NQ_CHECK_ARG(x_s0 >= K && x_s0 % 8 == 0 && w_s0 >= K && w_s0 % 8 == 0);
+    NQ_CHECK_ARG(((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w) |
+                   reinterpret_cast<uintptr_t>(planes)) & 15) == 0);
+    NQ_CHECK_ARG(planes_bytes >= static_cast<int64_t>(S) * M * N * 4);
+    return launch_small(x, x_s0, M, w, w_s0, N, K, S, planes, static_cast<hipStream_t>(stream));
+}
+
+extern "C" int nq_decode_norm_linear(const float *in_planes, int in_splits, const uint16_t *residual,
+                                     uint16_t *residual_out, const uint16_t *norm_weight, float eps, uint16_t *x_out,
+                                     const uint16_t *w, int64_t w_s0, int M, int N, int K, float *planes,
+                                     int64_t planes_bytes, void *stream) {
+    NQ_CHECK_ARG(w && planes && M > 0 && N > 0 && K > 0);
+    if (M > nq::kSmallRows || N % 16 != 0 || (K != 1024 && K != 2048)) return NQ_ERR_UNSUPPORTED;
+    const nq::NormRowsSrc norm{in_planes, in_splits, residual, residual_out, norm_weight, eps, x_out};
+    if (const int rc = nq::check_norm_rows(norm, M, K)) return rc;
+    NQ_CHECK_ARG(w_s0 >= K && w_s0 % 8 == 0 && planes_bytes >= static_cast<int64_t>(M) * N * 4);
+    NQ_CHECK_ARG(((reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(planes)) & 15) == 0);
+    const auto kernel = K == 1024 ? nq::small_gemm_kernel<1024, true, 4> : nq::small_gemm_kernel<2048, true, 8>;
+    hipLaunchKernelGGL(kernel, dim3(N / 16), dim3(nq::kSmallThreads), 0, static_cast<hipStream_t>(stream), nullptr, 0,
+                       M, w, w_s0, N, K, planes, norm);
+    return NQ_LAUNCH_STATUS();
+}
+
+extern "C" int nq_decode_norm_swiglu(const float *in_planes, int in_splits, const uint16_t *residual,
+                                     uint16_t *residual_out, const uint16_t *norm_weight, float eps, int M,
+                                     const uint16_t *packed, int64_t w_s0, int I, int K, uint16_t *out, int64_t o_s0,
+                                     void *stream) {
+    NQ_CHECK_ARG(packed && out && M > 0 && I > 0 && K > 0);
+    if (M > nq::kSmallRows || K != nq::kBsK || I % 16 != 0) return NQ_ERR_UNSUPPORTED;
+    const nq::NormRowsSrc norm{in_planes, in_splits, residual, residual_out, norm_weight, eps, nullptr};
+    if (const int rc = nq::check_norm_rows(norm, M, K)) return rc;
+    NQ_CHECK_ARG(w_s0 >= K && w_s0 % 8 == 0 && reinterpret_cast<uintptr_t>(packed) % 16 == 0);
+    NQ_CHECK_ARG(o_s0 >= I && o_s0 % 2 == 0 && reinterpret_cast<uintptr_t>(out) % 4 == 0);
+    hipLaunchKernelGGL((nq::bf16_swiglu_kernel<nq::kBsK, 1, 2, true>), dim3(I / 16),
+                       dim3(2 * nq::kBsQuarters * nq::kWave), 0, static_cast<hipStream_t>(stream), nullptr, 0, M,
+                       packed, w_s0, out, o_s0, norm);
     return NQ_LAUNCH_STATUS();
 }

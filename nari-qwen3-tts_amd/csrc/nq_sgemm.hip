@@ -296,7 +296,7 @@ sgemm_deep_kernel(const float *__restrict__ x, int64_t x_s0, const int32_t *__re
     if (t >= units) return;
     const int m0 = (t % tiles_m) * 16, n0 = (t / tiles_m) * 16;
     const int lane = threadIdx.x & (kWave - 1);
-    const int wave = threadIdx.x / kWave;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);  // uniform: an MFMA ignores EXEC
     const int r16 = lane & 15, kq = lane >> 4;
     int xr = m0 + r16 < M ? m0 + r16 : M - 1;
     if (x_rows) xr = x_rows[xr];

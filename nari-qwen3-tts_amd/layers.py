@@ -450,6 +450,86 @@ def linear_silu_mul(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor | N
     return _linear(x, weight, _lib.NQ_EPI_SILU_MUL, out, weight.shape[0] // 2, workspace=workspace)
 
 
+class NormRows:
+    """Rows that a decode projection normalises itself (``nq_decode_norm_*``): residual + the split-K
+    planes an earlier ``decode_linear`` left, add-RMSNormed; the new residual goes to ``residual_out``,
+    the normalised rows to ``out`` when given (the linear form alone)."""
+
+    __slots__ = ("planes", "splits", "residual", "residual_out", "weight", "eps", "out")
+
+    def __init__(self, planes, splits: int, residual, residual_out, weight, eps: float, out=None) -> None:
+        for t, name in ((residual, "residual"), (residual_out, "residual_out"), (weight, "norm weight")):
+            _check(t, name)
+        if residual.shape != residual_out.shape or weight.shape != residual.shape[1:]:
+            raise ValueError("residuals and norm weight disagree")
+        if out is not None:
+            _check_out(out, residual, residual.shape)
+        if planes.numel() * planes.element_size() < splits * residual.numel() * 4:
+            raise ValueError("planes hold fewer partials than splits")
+        self.planes, self.splits, self.residual, self.residual_out = planes, splits, residual, residual_out
+        self.weight, self.eps, self.out = weight, float(eps), out
+
+    def args(self):
+        return (self.planes.data_ptr(), self.splits, self.residual.data_ptr(), self.residual_out.data_ptr(),
+                self.weight.data_ptr(), self.eps)
+
+
+def decode_linear_splits(rows: int, out_features: int, in_features: int) -> int:
+    """The planes ``decode_linear`` leaves for a shape; -1 where it does not take it."""
+
+    return int(_lib.load().nq_decode_linear_splits(int(rows), int(out_features), int(in_features)))
+
+
+def decode_linear(x: torch.Tensor, weight: torch.Tensor, planes: torch.Tensor) -> int:
+    """``linear_partials`` for at most 16 rows, with fewer planes; returns their number."""
+
+    rows, k = x.shape
+    if x.dtype != torch.bfloat16 or x.stride(1) != 1:
+        raise TypeError("linear needs bf16 tensors with unit inner stride")
+    w_ptr, w_s0, n = _weight_arg(weight, k)
+    _lib.require_device(x, weight, planes)
+    _lib.call("nq_decode_linear", x.data_ptr(), x.stride(0), w_ptr, w_s0, rows, n, k, planes.data_ptr(),
+              planes.numel() * planes.element_size(), _lib.stream(x.device))
+    return decode_linear_splits(rows, n, k)
+
+
+def decode_norm_linear(rows_in: NormRows, weight: torch.Tensor, planes: torch.Tensor) -> int:
+    """The projection of ``rows_in`` as one plane [1, rows, out] (returned: 1)."""
+
+    rows, k = rows_in.residual.shape
+    w_ptr, w_s0, n = _weight_arg(weight, k)
+    _lib.require_device(rows_in.planes, rows_in.residual, weight, planes)
+    _lib.call("nq_decode_norm_linear", *rows_in.args(), _lib.ptr(rows_in.out), w_ptr, w_s0, rows, n, k,
+              planes.data_ptr(), planes.numel() * planes.element_size(), _lib.stream(planes.device))
+    return 1
+
+
+def decode_norm_swiglu(rows_in: NormRows, packed: torch.Tensor, out: torch.Tensor,
+                       weight_scales: torch.Tensor | None = None) -> torch.Tensor:
+    """``linear_swiglu`` (bf16 ``packed``) or, quantizing the rows, ``linear_fp8_swiglu`` (FP8 ``packed``
+    and its block scales) of ``rows_in``."""
+
+    rows, k = rows_in.residual.shape
+    inter = packed.shape[0] // 2
+    if out.shape != (rows, inter) or out.dtype != torch.bfloat16 or out.stride(1) != 1:
+        raise ValueError(f"out must be bf16 [{rows}, {inter}] with unit inner stride")
+    if packed.shape[1] != k or packed.stride(1) != 1:
+        raise ValueError("packed gate/up rows must match the residual width")
+    _lib.require_device(rows_in.planes, rows_in.residual, packed, out, weight_scales)
+    if weight_scales is None:
+        if packed.dtype != torch.bfloat16:
+            raise TypeError("bf16 packed rows, or FP8 ones with their scales, expected")
+        _lib.call("nq_decode_norm_swiglu", *rows_in.args(), rows, packed.data_ptr(), packed.stride(0), inter, k,
+                  out.data_ptr(), out.stride(0), _lib.stream(out.device))
+        return out
+    if packed.dtype != FP8 or weight_scales.shape != (2 * inter // 128, k // 128):
+        raise TypeError("FP8 codes and matching scales expected")
+    _lib.call("nq_decode_norm_fp8_swiglu", *rows_in.args(), rows, packed.data_ptr(), packed.stride(0),
+              weight_scales.data_ptr(), weight_scales.stride(0), inter, k, out.data_ptr(), out.stride(0),
+              _lib.stream(out.device))
+    return out
+
+
 FP8 = torch.float8_e4m3fn
 
 
@@ -664,6 +744,11 @@ def linear_fp8_swiglu(q: torch.Tensor, scales: torch.Tensor, packed: torch.Tenso
 
 
 __all__ = [
+    "NormRows",
+    "decode_linear",
+    "decode_linear_splits",
+    "decode_norm_linear",
+    "decode_norm_swiglu",
     "linear_swiglu",
     "pack_swiglu",
     "FP8",

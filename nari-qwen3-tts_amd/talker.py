@@ -30,6 +30,11 @@ import torch
 from . import _lib
 from .layers import (
     FP8,
+    NormRows,
+    decode_linear,
+    decode_linear_splits,
+    decode_norm_linear,
+    decode_norm_swiglu,
     embed_add_rmsnorm,
     gather_sum_rows,
     linear,
@@ -330,6 +335,14 @@ class TalkerDecodeStep:
             self.act_q = torch.zeros(rows, c.hidden, dtype=FP8, device=dev)
             self.act_scales = torch.zeros(rows, c.hidden // 128, dtype=torch.float32, device=dev)
             need = max(need, linear_fp8_workspace_bytes(rows, 2 * c.intermediate, c.hidden, _lib.NQ_EPI_SILU_MUL))
+        # few rows: projections that normalise their rows themselves, over two alternating plane
+        # regions and two residual buffers (a kernel reads one of each and writes the other)
+        self.few = self.fp8 and rows <= self.FEW_ROWS and c.hidden == 2048 and c.intermediate % 384 == 0 and all(
+            decode_linear_splits(rows, n, k) > 0 for n, k in self._few_shapes(c))
+        if self.few:
+            self.residual2 = torch.zeros(rows, c.hidden, **bf)
+            self._region = max(decode_linear_splits(rows, n, k) * rows * n * 4 for n, k in self._few_shapes(c))
+            need = max(need, 2 * self._region)
         # split-K planes of the projections; may be shared by steps whose graphs never run at once
         if workspace is not None and workspace.numel() >= need:
             self.linear_workspace = workspace
@@ -342,6 +355,36 @@ class TalkerDecodeStep:
         self.embed_status = torch.zeros(1, dtype=torch.int32, device=dev)
         self.report = StepReport(rows, dev)
 
+    # the most rows of 2048 that every workgroup of a projection normalises for itself
+    FEW_ROWS = 4
+
+    @staticmethod
+    def _few_shapes(c: TalkerConfig):
+        return ((c.qkv_width, c.hidden), (c.hidden, c.num_qo_heads * c.head_dim), (c.hidden, c.intermediate),
+                (c.vocab, c.hidden))
+
+    def _forward_few(self) -> int:
+        """The layers with five launches each: QKV, attention, o, gate/up + SwiGLU, down, the add-RMSNorms
+        inside the projections after them; leaves the codec head's plane in the second region."""
+
+        c, ctx, n = self.w.config, self.context, self.rows
+        q_w = c.num_qo_heads * c.head_dim
+        a, b = self.linear_workspace[: self._region], self.linear_workspace[self._region: 2 * self._region]
+        h, h2 = self.residual, self.residual2
+        q = self.qkv[:, :q_w].view(n, c.num_qo_heads, c.head_dim)
+        splits = decode_linear(self.hidden, self.w.layers[0].qkv, b)
+        for index, layer in enumerate(self.w.layers):
+            ctx.select_layer(index)
+            if index:
+                splits = decode_norm_linear(NormRows(a, down, h2, h, layer.input_norm, c.rms_eps), layer.qkv, b)
+            attended = ctx.attend_partials(layer.attention, b, splits, q).view(n, q_w)
+            splits = decode_linear(attended, layer.o, a)
+            decode_norm_swiglu(NormRows(a, splits, h, h2, layer.post_norm, c.rms_eps), layer.gate_up_packed, self.act,
+                               layer.gate_up_scales)
+            down = decode_linear(self.act, layer.down, a)
+        return decode_norm_linear(NormRows(a, down, h2, h, self.w.final_norm, c.rms_eps, self.hidden),
+                                  self.w.codec_head, b)
+
     def forward(self) -> torch.Tensor:
         c = self.w.config
         ctx = self.context
@@ -350,6 +393,12 @@ class TalkerDecodeStep:
         embed_add_rmsnorm(self.text_ids, self.w.text_embedding, self.step_embed, self.w.layers[0].input_norm,
                           c.rms_eps, self.residual, self.hidden, status=self.embed_status)
         trace = self.trace
+        if self.few and trace is None and self.use_counter_rng:
+            splits = self._forward_few()
+            ctx.advance_sequence_lengths()
+            self._sample(self.linear_workspace[self._region:], splits)
+            self._report()
+            return self.tokens
         if trace is not None:
             trace[0].copy_(self.residual)
         q_w = c.num_qo_heads * c.head_dim
@@ -386,16 +435,19 @@ class TalkerDecodeStep:
                   self.embed_status.data_ptr(), self.tokens.data_ptr(), self.rows, c.eos_id, c.vocab,
                   self.report.device.data_ptr(), _lib.stream(self.device))
 
-    def _sample(self) -> None:
+    def _sample(self, planes: torch.Tensor | None = None, splits: int = 0) -> None:
+        """``planes``: the codec head's ``splits`` planes, when the layers left them already."""
+
         c = self.w.config
         n = self.rows
-        ws = self.linear_workspace
+        ws = self.linear_workspace if planes is None else planes
         options = dict(repetition_penalty=self.penalty, seen_token_mask=self.seen, mask_from=c.codec_vocab,
                        eos_id=c.eos_id, suppress_eos=self.suppress_eos, update_seen=True, out=self.tokens)
         if self.use_counter_rng:
             # codec head as split-K planes, summed, rounded and drawn from in the sampling launch
             # (the same logits and tokens as the projection followed by the sampler)
-            splits = linear_partials(self.hidden, self.w.codec_head, ws)
+            if planes is None:
+                splits = linear_partials(self.hidden, self.w.codec_head, ws)
             planes = ws[: splits * n * c.vocab * 4].view(torch.float32).view(splits, n, c.vocab)
             sample_with_counter_from_planes(planes, self.temperature, self.top_k, self.top_p, self.seed, self.offsets,
                                             logits_out=self.logits, **options)

@@ -217,3 +217,106 @@ def test_gather_sum_rows_and_gather_norm_equal_their_torch_steps(nq, device):
     want_h = torch.index_select(proj, 0, tok)
     assert torch.equal(h.view(torch.int16), want_h.view(torch.int16))
     assert torch.equal(x, rmsnorm(want_h, weight, 1e-6))
+
+
+@pytest.mark.parametrize("width,inter,rows", [(1024, 3072, 1), (1024, 48, 5), (1024, 3072, 8), (2048, 6144, 1),
+                                              (2048, 384, 3), (2048, 6144, 4)])
+@pytest.mark.parametrize("splits", [1, 2, 4])
+def test_decode_projections_that_normalise_their_rows(nq, device, width, inter, rows, splits):
+    """The residual, the normalised rows and the SwiGLU are those of the add-RMSNorm followed by the
+    projection, bit for bit; the projection itself within fp32 summation of the float64 product (K
+    terms of at most 2^-24 each, the waves' partial sums)."""
+
+    from nari_qwen3_tts_amd import layers as L
+
+    g = torch.Generator(device=device)
+    g.manual_seed(width + inter + 10 * rows + splits)
+
+    def bf(*shape, scale=1.0):
+        return (torch.randn(*shape, generator=g, device=device) * scale).to(torch.bfloat16)
+
+    planes = torch.randn(splits, rows, width, generator=g, device=device)
+    residual, norm = bf(rows, width), bf(width)
+    hidden = planes[0].clone()
+    for p in planes[1:]:
+        hidden += p
+    x, want_res = hidden.to(torch.bfloat16), residual.clone()
+    L.add_rmsnorm(x, want_res, norm, 1e-6)
+    new, out = torch.empty_like(residual), torch.empty_like(residual)
+    w = bf(80, width, scale=0.02)
+    got = torch.full((rows, 80), float("nan"), device=device)
+    assert L.decode_norm_linear(L.NormRows(planes, splits, residual, new, norm, 1e-6, out), w, got) == 1
+    assert torch.equal(new, want_res) and torch.equal(out, x)
+    exact = x.double() @ w.double().t()
+    bound = x.double().abs() @ w.double().abs().t()
+    assert bool(((got.double() - exact).abs() <= width * 2.0 ** -24 * bound).all())
+    gate_up = bf(2 * inter, width, scale=0.02)
+    act, want = (torch.empty(rows, inter, dtype=torch.bfloat16, device=device) for _ in range(2))
+    new.zero_()
+    rows_in = L.NormRows(planes, splits, residual, new, norm, 1e-6)
+    if width == 1024:
+        packed = L.pack_swiglu(gate_up)
+        L.decode_norm_swiglu(rows_in, packed, act)
+        L.linear_swiglu(x, packed, want, weight=gate_up)
+    else:
+        codes, scales = L.quantize_fp8_weight_blocks(gate_up)
+        packed = L.pack_fp8_swiglu(codes)
+        L.decode_norm_swiglu(rows_in, packed, act, scales)
+        L.linear_fp8_swiglu(*L.quantize_fp8_rows(x), packed, scales, want)
+    assert torch.equal(act, want) and torch.equal(new, want_res)
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 16, 32), (3, 64, 96), (4, 2048, 2048), (4, 2048, 6144), (8, 1024, 3072), (16, 48, 864),
+                                   (16, 4096, 1024)])
+def test_decode_linear_planes(nq, device, m, n, k):
+    """Few-row projections with wave counts that do not divide the steps, against float64; what it does
+    not take is refused."""
+
+    from nari_qwen3_tts_amd import layers as L
+
+    g = torch.Generator(device=device)
+    g.manual_seed(m + n + k)
+    x = torch.randn(m, k, generator=g, device=device).to(torch.bfloat16)
+    w = torch.randn(n, k, generator=g, device=device).to(torch.bfloat16)
+    planes = torch.full((4 * m * n,), float("nan"), device=device)
+    splits = L.decode_linear(x, w, planes)
+    got = planes[: splits * m * n].view(splits, m, n).double().sum(0)
+    bound = x.double().abs() @ w.double().abs().t()
+    assert bool(((got - x.double() @ w.double().t()).abs() <= k * 2.0 ** -24 * bound).all())
+    assert bool(planes[splits * m * n:].isnan().all())
+    assert L.decode_linear_splits(17, n, k) == L.decode_linear_splits(m, n + 8, k) == -1
+    with pytest.raises(ValueError):
+        L.decode_linear(x, w, planes[: splits * m * n - 1])
+
+
+@pytest.mark.parametrize("rows", [1, 4])
+def test_few_row_decode_step_equals_the_general_one(nq, device, rows):
+    """The step whose projections normalise their rows against the step with its own norm launches:
+    logits, hidden state, residual and written K/V within bf16 rounding of sums in another order."""
+
+    from helpers import DecodeKey, adopt_random, make_kv
+    from nari_qwen3_tts_amd.talker import TalkerConfig, TalkerDecodeStep, TalkerWeights
+
+    cfg = TalkerConfig(num_layers=2)
+    weights = TalkerWeights(cfg, device, seed=9)
+    outs = []
+    for few in (True, False):
+        rng = np.random.default_rng(17)
+        kv = make_kv(nq, device, layers=2, pages=256)
+        gen = torch.Generator(device=device)
+        gen.manual_seed(4)
+        kv.storage.copy_(torch.randn(kv.storage.shape, generator=gen, device=device))
+        rids = adopt_random(kv, rng, rng.integers(5, 200, size=rows))
+        ctx = kv.create_decode(DecodeKey(rows), slot=0)
+        step = TalkerDecodeStep(weights, ctx, rows, use_counter_rng=True)
+        assert step.few
+        step.few = few
+        step.step_embed.copy_(torch.randn(rows, cfg.hidden, generator=gen, device=device))
+        step.temperature.fill_(0.9)
+        kv.prepare_decode(ctx, DecodeKey(rows), tuple(rids))
+        step.forward()
+        torch.cuda.synchronize()
+        outs.append([t.float() for t in (step.logits, step.hidden, step.residual, kv.storage)])
+    for a, b in zip(*outs):
+        # two layers: an FP8 code that falls to the other side moves a value by a sixteenth
+        assert float((a - b).norm() / b.norm()) <= 1e-2
