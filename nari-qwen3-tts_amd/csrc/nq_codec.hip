@@ -16,7 +16,6 @@
 // A conv or transconv reads the old state, then a second small kernel writes
 // the new state (in place: each thread owns one (stream, channel) column and
 // walks it forward, so no element is overwritten before it is read).
-#include <type_traits>
 
 #include "nq_common.h"
 
@@ -24,7 +23,10 @@ namespace nq {
 namespace {
 
 constexpr int kCodecThreads = 256;
-constexpr int kHistoryPerThread = 16;  // history_update_kernel covers pad * C <= 256 * 16
+constexpr int kCus = 256;  // compute units of the chip
+// history_update_kernel covers pad * C <= 1024 * 4
+constexpr int kHistoryThreads = 1024;
+constexpr int kHistoryPerThread = 4;
 
 // stream of stage row t: the largest b with off[b] * u <= t
 __device__ __forceinline__ int stream_of(const int32_t *__restrict__ off, int B, int64_t t, int u) {
@@ -36,6 +38,51 @@ __device__ __forceinline__ int stream_of(const int32_t *__restrict__ off, int B,
     }
     return lo;
 }
+
+// Tile `tile` of the streams' rows cut into tiles of at most `rows` rows that never cross a stream (tiles
+// counted through the streams in order): every row before the tile's first one that a causal tap can
+// read is then a row of the same stream or of its history.  The lanes of a wave count 64 streams at a
+// time.  Like stream_of, the last stream reaches to row T.  False past the last tile; uniform over the
+// workgroup.  At most T / rows + B tiles exist.
+struct StreamTile {
+    int b;          // stream
+    int64_t first;  // its first row
+    int64_t n;      // its rows
+    int64_t l0;     // the tile's first row within it
+};
+__device__ __forceinline__ bool stream_tile(const int32_t *__restrict__ off, int B, int u, int64_t T, int rows,
+                                            int tile, StreamTile &s) {
+    const int lane = threadIdx.x & (kWave - 1);
+    int before = 0;
+    for (int b0 = 0; b0 < B; b0 += kWave) {
+        const int b = b0 + lane;
+        const int lo = off[b < B ? b : B], hi = off[b < B ? b + 1 : B];
+        const int64_t end = b + 1 < B && static_cast<int64_t>(hi) * u < T ? static_cast<int64_t>(hi) * u : T;
+        const int64_t n = end - static_cast<int64_t>(lo) * u;
+        const int count = b < B && n > 0 ? static_cast<int>((n + rows - 1) / rows) : 0;
+        int upto = count;
+#pragma unroll
+        for (int d = 1; d < kWave; d *= 2) {
+            const int other = __shfl_up(upto, d, kWave);
+            if (lane >= d) upto += other;
+        }
+        const uint64_t past = __ballot(before + upto > tile);
+        if (past) {
+            const int at = __builtin_ctzll(past);
+            s.b = b0 + at;
+            s.first = static_cast<int64_t>(__builtin_amdgcn_readlane(lo, at)) * u;
+            const int64_t next = static_cast<int64_t>(__builtin_amdgcn_readlane(hi, at)) * u;
+            s.n = (s.b + 1 < B && next < T ? next : T) - s.first;
+            const int skipped = before + __builtin_amdgcn_readlane(upto - count, at);
+            s.l0 = static_cast<int64_t>(tile - skipped) * rows;
+            return true;
+        }
+        before += __builtin_amdgcn_readlane(upto, kWave - 1);
+    }
+    return false;
+}
+
+int stream_tiles_bound(int64_t T, int B, int rows) { return static_cast<int>(T / rows + (B < T ? B : T)); }
 
 // SnakeBeta x + sin(a x)^2 / b with a = exp(alpha), b = exp(beta) (per channel)
 __device__ __forceinline__ float snake(float x, float a, float inv_b) {
@@ -154,33 +201,35 @@ conv_kernel(const float *__restrict__ x, int64_t ldx, int64_t T, const int32_t *
     }
 }
 
-// Narrow causal Conv1d (Cin, Cout <= 64): each thread computes every output
-// channel of R rows (rows t, t + 256, ..., of the workgroup's 256 R), so each
-// weight read from LDS feeds R rows.  The workgroup stages its 256 R rows plus
-// the `pad` rows before them, activated once, in LDS (row pitch Cin + 1, so the
-// 64 rows a wave reads at one channel hit distinct banks) with the weights as
-// [ci][k][co].  A tap whose input time is >= 0 reads the staged row (it lies in
-// the same stream); a tap before the stream's first fresh row reads the
-// stream's history from global memory.  The thread finds its first row's
-// stream by binary search and steps forward for its later rows.  Outputs (and
-// the residual) move as float4 when the row strides allow it.
+// Narrow causal Conv1d (Cin, Cout <= 64): a workgroup owns 256 R rows of one stream, each thread every
+// output channel of R of them (rows t, t + 256, ...), so each weight read from LDS feeds R rows.  The
+// rows, and the `pad` rows before them (from the stream's history where they lie before its first
+// fresh row), are staged in LDS, the fresh ones activated once (row pitch Cin + 1, so the 64 rows a wave
+// reads at one channel hit distinct banks), with the weights as [ci][k][co]; every tap then reads LDS.
+// Outputs (and the residual) move as float4 when the row strides allow it.
 //
-// kUnit: the decoder's whole residual unit in one launch (Cin == Cout == C):
+// kUnit: the decoder's whole residual unit in one launch (Cin == Cout == CO, seven taps):
 // out = res + conv1x1(snake2(conv(snake1(x)) + bias)) + bias2, with res the
 // input x itself.  The 1x1 convolution runs in registers on the thread's
 // conv outputs (its weights [ci][co] in LDS), in the order of the separate
 // 1x1 launch, so the bits are those of the two launches; the intermediate
 // tensor never reaches memory.
+//
+// With tiles cut from the concatenated rows of all streams, a wave near a stream's start read every tap
+// through generic pointers: one stream's 8000 rows of 8 channels took 14.7 us and take 10.1, 38 and
+// 1.8 M rows 16 and 52 us (10.5 and 51), where the multiply-adds and the activation bound it.  A single
+// output channel (the decoder's last convolution) computes one, not eight: 1.8 M rows 36 -> 24 us.
 template <int CO, int R, bool kUnit = false>
 __global__ void __launch_bounds__(kCodecThreads)
 conv_small_kernel(const float *__restrict__ x, int64_t ldx, int64_t T, const int32_t *__restrict__ off, int B, int u,
                   const int32_t *__restrict__ slots, const float *__restrict__ hist, const float *__restrict__ w,
-                  const float *__restrict__ bias, int Cin, int Cout, int K, int dil, Act act,
+                  const float *__restrict__ bias, int cin, int Cout, int taps, int dil, Act act,
                   const float *__restrict__ res, int64_t ldres, float *__restrict__ out, int64_t ldo,
                   const float *__restrict__ w2 = nullptr, const float *__restrict__ bias2 = nullptr,
                   Act act2 = Act{nullptr, nullptr}) {
     constexpr int ROWS = kCodecThreads * R;
     extern __shared__ float lds[];
+    const int Cin = kUnit ? CO : cin, K = kUnit ? kConvKMax : taps;
     const int pad = (K - 1) * dil;
     const int pitch = Cin + 1;
     float *xs = lds;                                            // [(ROWS + pad) * pitch]
@@ -190,7 +239,13 @@ conv_small_kernel(const float *__restrict__ x, int64_t ldx, int64_t T, const int
     float *w2s = sb + Cin + (kUnit ? (4 - (Cin * K * CO + 2 * Cin) % 4) % 4 : 0);  // [Cin][CO], 16-byte aligned
     float *sa2 = w2s + Cin * CO;                                // [Cin]
     float *sb2 = sa2 + Cin;                                     // [Cin]
-    const int64_t row0 = static_cast<int64_t>(blockIdx.x) * ROWS;
+    StreamTile st;
+    if (!stream_tile(off, B, u, T, ROWS, static_cast<int>(blockIdx.x), st)) return;
+    x += st.first * ldx;
+    if (res) res += st.first * ldres;
+    out += st.first * ldo;
+    // row -1 lies before h
+    const float *h = pad ? hist + (static_cast<int64_t>(slots[st.b]) * pad + pad) * Cin : nullptr;
     for (int e = threadIdx.x; e < Cin * K * CO; e += kCodecThreads) {
         const int co = e % CO;
         const int ck = e / CO;
@@ -204,7 +259,7 @@ conv_small_kernel(const float *__restrict__ x, int64_t ldx, int64_t T, const int
     if constexpr (kUnit) {
         for (int e = threadIdx.x; e < Cin * CO; e += kCodecThreads) {
             const int co = e % CO, ci = e / CO;
-            w2s[e] = co < Cout ? w2[static_cast<int64_t>(co) * Cin + ci] : 0.f;
+            w2s[e] = w2[static_cast<int64_t>(co) * Cin + ci];
         }
         if (act2.alpha && threadIdx.x < Cin) {
             sa2[threadIdx.x] = act2.a_of(threadIdx.x);
@@ -212,29 +267,35 @@ conv_small_kernel(const float *__restrict__ x, int64_t ldx, int64_t T, const int
         }
     }
     __syncthreads();
-    if ((Cin & 3) == 0 && (ldx & 3) == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0) {
-        // 128-bit loads, eight per thread in flight before any is activated and stored
+    // staged row rr is row l0 - pad + rr of the stream (the last one again past its end: those feed no
+    // stored output)
+    auto source = [&](int rr, int64_t &l) {
+        l = st.l0 - pad + rr;
+        if (l >= st.n) l = st.n - 1;
+        return l < 0 ? h + l * Cin : x + l * ldx;
+    };
+    if ((Cin & 3) == 0 && (ldx & 3) == 0 &&
+        ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(h)) & 15) == 0) {
+        // 128-bit loads, kBatch per thread in flight before any is activated and stored
+        constexpr int kBatch = R == 1 ? 4 : 8;
         const int vpr = Cin / 4;
         const int nvec = (ROWS + pad) * vpr;
-        for (int e0 = threadIdx.x; e0 < nvec; e0 += 8 * kCodecThreads) {
-            float4 v[8];
+        for (int e0 = threadIdx.x; e0 < nvec; e0 += kBatch * kCodecThreads) {
+            float4 v[kBatch];
 #pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const int e = e0 + i * kCodecThreads;
+            for (int i = 0; i < kBatch; ++i) {
+                const int e = e0 + i * kCodecThreads < nvec ? e0 + i * kCodecThreads : nvec - 1;
                 const int rr = e / vpr;
-                const int64_t g = row0 - pad + rr;
-                v[i] = (e < nvec && g >= 0 && g < T)
-                           ? *reinterpret_cast<const float4 *>(x + g * ldx + (e - rr * vpr) * 4)
-                           : make_float4(0.f, 0.f, 0.f, 0.f);
+                int64_t l;
+                v[i] = *reinterpret_cast<const float4 *>(source(rr, l) + (e - rr * vpr) * 4);
             }
 #pragma unroll
-            for (int i = 0; i < 8; ++i) {
+            for (int i = 0; i < kBatch; ++i) {
                 const int e = e0 + i * kCodecThreads;
                 if (e >= nvec) break;
                 const int rr = e / vpr, c = (e - rr * vpr) * 4;
-                const int64_t g = row0 - pad + rr;
                 float f[4] = {v[i].x, v[i].y, v[i].z, v[i].w};
-                if (act.alpha && g >= 0 && g < T) {
+                if (act.alpha && st.l0 - pad + rr >= 0) {
 #pragma unroll
                     for (int q = 0; q < 4; ++q) f[q] = snake(f[q], sa[c + q], sb[c + q]);
                 }
@@ -245,83 +306,54 @@ conv_small_kernel(const float *__restrict__ x, int64_t ldx, int64_t T, const int
     } else {
         for (int e = threadIdx.x; e < (ROWS + pad) * Cin; e += kCodecThreads) {
             const int rr = e / Cin, c = e - rr * Cin;
-            const int64_t g = row0 - pad + rr;
-            float v = 0.f;
-            if (g >= 0 && g < T) {
-                v = x[g * ldx + c];
-                if (act.alpha) v = snake(v, sa[c], sb[c]);
-            }
+            int64_t l;
+            float v = source(rr, l)[c];
+            if (act.alpha && l >= 0) v = snake(v, sa[c], sb[c]);
             xs[rr * pitch + c] = v;
         }
     }
     __syncthreads();
-    const int64_t first = row0 + threadIdx.x;
-    // the residual unit meets a second barrier below, so its threads past the end stay (they only
-    // skip the stores)
-    if (!kUnit && first >= T) return;
-    // streams of the thread's rows (non-decreasing)
-    int sb_[R];
-    int64_t local[R];
-    {
-        int b = stream_of(off, B, first, u);
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            const int64_t row = first + static_cast<int64_t>(r) * kCodecThreads;
-            while (b + 1 < B && static_cast<int64_t>(off[b + 1]) * u <= row) ++b;
-            sb_[r] = b;
-            local[r] = row - static_cast<int64_t>(off[b]) * u;
-        }
-    }
     float acc[R][CO];
 #pragma unroll
     for (int r = 0; r < R; ++r)
 #pragma unroll
         for (int j = 0; j < CO; ++j) acc[r][j] = 0.f;
-    // taps read the staged rows through LDS addressing when every row of the wave has
-    // its whole receptive field in the stream's fresh rows (the common case), else through
-    // generic pointers that may point into the history
-    bool staged = true;
-#pragma unroll
-    for (int r = 0; r < R; ++r) staged = staged && local[r] >= pad;
     // one tap's multiply-adds over the input channels: the rows' inputs xr[r][ci], the weights at wk
     // ([ci][k][co] with row pitch kw floats)
-    auto channel_loop = [&](const float *const (&xr)[R], const float *wk, int kw, int cin) {
-        for (int ci = 0; ci < cin; ++ci) {
+    auto channel_loop = [&](const float *const (&xr)[R], const float *wk, int kw) {
+        for (int ci = 0; ci < Cin; ++ci) {
             float xv[R];
 #pragma unroll
             for (int r = 0; r < R; ++r) xv[r] = xr[r][ci];
-            const float4 *w4 = reinterpret_cast<const float4 *>(wk + ci * kw);
+            if constexpr (CO % 4 == 0) {
+                const float4 *w4 = reinterpret_cast<const float4 *>(wk + ci * kw);
 #pragma unroll
-            for (int j = 0; j < CO / 4; ++j) {
-                const float4 ww = w4[j];
+                for (int j = 0; j < CO / 4; ++j) {
+                    const float4 ww = w4[j];
 #pragma unroll
-                for (int r = 0; r < R; ++r) {
-                    acc[r][4 * j] += xv[r] * ww.x;
-                    acc[r][4 * j + 1] += xv[r] * ww.y;
-                    acc[r][4 * j + 2] += xv[r] * ww.z;
-                    acc[r][4 * j + 3] += xv[r] * ww.w;
+                    for (int r = 0; r < R; ++r) {
+                        acc[r][4 * j] += xv[r] * ww.x;
+                        acc[r][4 * j + 1] += xv[r] * ww.y;
+                        acc[r][4 * j + 2] += xv[r] * ww.z;
+                        acc[r][4 * j + 3] += xv[r] * ww.w;
+                    }
+                }
+            } else {
+#pragma unroll
+                for (int j = 0; j < CO; ++j) {
+                    const float ww = wk[ci * kw + j];
+#pragma unroll
+                    for (int r = 0; r < R; ++r) acc[r][j] += xv[r] * ww;
                 }
             }
         }
     };
-    auto taps = [&](auto lds_only) {
-        for (int k = 0; k < K; ++k) {
-            const int back = (K - 1 - k) * dil;
-            const float *xr[R];
+    for (int k = 0; k < K; ++k) {
+        const float *xr[R];
 #pragma unroll
-            for (int r = 0; r < R; ++r) {
-                const int64_t src = local[r] - back;
-                if constexpr (decltype(lds_only)::value)
-                    xr[r] = xs + (threadIdx.x + r * kCodecThreads + pad - back) * pitch;
-                else
-                    xr[r] = src >= 0 ? xs + (threadIdx.x + r * kCodecThreads + pad - back) * pitch
-                                     : hist + (static_cast<int64_t>(slots[sb_[r]]) * pad + pad + src) * Cin;
-            }
-            channel_loop(xr, wsm + k * CO, K * CO, Cin);
-        }
-    };
-    if (__all(staged)) taps(std::true_type{});
-    else taps(std::false_type{});
+        for (int r = 0; r < R; ++r) xr[r] = xs + (threadIdx.x + r * kCodecThreads + k * dil) * pitch;
+        channel_loop(xr, wsm + k * CO, K * CO);
+    }
     if constexpr (kUnit) {
         // the 1x1 convolution of snake2(conv + bias): each thread parks its rows' activated conv
         // outputs in its own rows of the (now free) staging area and reads them back per channel
@@ -338,15 +370,15 @@ conv_small_kernel(const float *__restrict__ x, int64_t ldx, int64_t T, const int
             }
             yr[r] = yw;
         }
-        channel_loop(yr, w2s, CO, Cin);
+        channel_loop(yr, w2s, CO);
         bias = bias2;
     }
-    const bool vec = Cout == CO && (ldo & 3) == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0 &&
+    const bool vec = CO % 4 == 0 && Cout == CO && (ldo & 3) == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0 &&
                      (!res || ((ldres & 3) == 0 && (reinterpret_cast<uintptr_t>(res) & 15) == 0));
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-        const int64_t row = first + static_cast<int64_t>(r) * kCodecThreads;
-        if (row >= T) break;
+        const int64_t row = st.l0 + threadIdx.x + r * kCodecThreads;
+        if (row >= st.n) break;
         if (vec) {
 #pragma unroll
             for (int j = 0; j < CO / 4; ++j) {
@@ -378,13 +410,20 @@ conv_small_kernel(const float *__restrict__ x, int64_t ldx, int64_t T, const int
     }
 }
 
-constexpr int conv_small_rows(int CO) { return CO <= 16 ? 2 : 1; }
-
-size_t conv_small_lds(int Cin, int K, int dil, int CO, bool unit = false) {
-    const size_t rows = static_cast<size_t>(kCodecThreads) * conv_small_rows(CO);
+size_t conv_small_lds(int Cin, int K, int dil, int CO, int R, bool unit = false) {
+    const size_t rows = static_cast<size_t>(kCodecThreads) * R;
     const size_t unit_floats = unit ? 3 + static_cast<size_t>(Cin) * CO + 2 * Cin : 0;
     return ((rows + (K - 1) * dil) * (Cin + 1) + 3 + static_cast<size_t>(Cin) * K * CO + 2 * Cin + unit_floats) *
            sizeof(float);
+}
+
+constexpr size_t kConvLds = 150 * 1024;
+
+// Rows per thread of the narrow convolution: two while the tiles then still fill the chip, one below a
+// 256-row tile per CU, where the time is one tile's chain (8000 rows of 8 channels 10.1 us against 12.5;
+// 192,000 rows 25.1 against 15.0).  More than 16 channels take one (their sums fill the registers).
+int conv_small_rows(int CO, int64_t T, int B) {
+    return CO <= 16 && stream_tiles_bound(T, B, kCodecThreads) > kCus ? 2 : 1;
 }
 
 // depthwise causal Conv1d (groups == C): one thread per (row, channel)
@@ -470,8 +509,9 @@ __global__ void __launch_bounds__(kStateThreads) state_copy_kernel(const StateAr
     }
 }
 
-// new history = last pad rows of [history ; act(x)] per stream
-__global__ void __launch_bounds__(kCodecThreads)
+// new history = last pad rows of [history ; act(x)] per stream.  1024 threads of four elements: with 256
+// of sixteen the unrolled activations were 11 KB of code, whose fetch a launch of one workgroup waits for.
+__global__ void __launch_bounds__(kHistoryThreads)
 history_update_kernel(const float *__restrict__ x, int64_t ldx, const int32_t *__restrict__ off, int B, int u,
                       const int32_t *__restrict__ slots, float *__restrict__ hist, int C, int pad, Act act) {
     // one workgroup per stream: every (j, c) of its [pad, C] history is read first (the entries that
@@ -486,7 +526,7 @@ history_update_kernel(const float *__restrict__ x, int64_t ldx, const int32_t *_
     float v[kPer];
 #pragma unroll
     for (int i = 0; i < kPer; ++i) {
-        const int e = threadIdx.x + i * kCodecThreads;
+        const int e = threadIdx.x + i * kHistoryThreads;
         v[i] = 0.f;
         if (e < n) {
             const int j = e / C, c = e - j * C;
@@ -496,7 +536,7 @@ history_update_kernel(const float *__restrict__ x, int64_t ldx, const int32_t *_
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < kPer; ++i) {
-        const int e = threadIdx.x + i * kCodecThreads;
+        const int e = threadIdx.x + i * kHistoryThreads;
         if (e < n) h[e] = v[i];
     }
 }
@@ -996,7 +1036,7 @@ pcm16_kernel(const float *__restrict__ x, int64_t n, float *__restrict__ wav, in
 }
 
 // ---------------------------------------------------------------------------
-// A decoder residual unit of C = 8, 16 or 32 channels on MFMA, for the decoder's
+// A decoder residual unit of C = 16 or 32 channels on MFMA, for the decoder's
 // "high" float32 matmul precision (the reference's convolutions run on cuDNN with
 // its TF32 default): out = x + conv1x1(snake2(conv7(snake1(x)) + b1)) + b2 as two
 // implicit GEMMs with bf16x3 split products and fp32 sums, each operand v = hi +
@@ -1009,31 +1049,29 @@ pcm16_kernel(const float *__restrict__ x, int64_t n, float *__restrict__ wav, in
 // consecutive k are 8 consecutive channels of one input row, staged split in LDS
 // as [row][C hi | C lo] with a 16-byte row pad, 8 rows of a lane group then
 // cover distinct banks), so a lane ends with 4 consecutive output channels of
-// one row.  Rows within (K-1) dil of their stream's start take those taps from
-// the stream's history (the wave takes that path only when one of its rows
-// needs it).  The activated 7-tap outputs go split, one 16-row tile at a time,
+// one row.  The activated 7-tap outputs go split, one 16-row tile at a time,
 // through the wave's own LDS rows into the B operand of the 1x1 convolution.  A
-// workgroup of 4 waves owns 4 x 16 x unit_tiles<C>() output rows.
+// workgroup of 4 waves owns 4 x 16 x MT output rows of one stream, and the
+// (K-1) dil rows before them come from the stream's history where they lie
+// before its first fresh row.
+//
+// What bounds it is the chain of one workgroup (weights, rows, activation, products), so the weights are
+// read as each thread's 28 consecutive floats (as scattered fragment elements every lane of a load met
+// its own cache line) and a tile stays within a stream: with tiles over the concatenated rows the rows
+// near a stream's start searched their stream and read its history tap by tap, and one such wave held
+// its workgroup up.  32 channels at dilation 9: 400 rows of one stream 24.8 -> 11.6 us, 89,600 rows of 32
+// streams 50.7 -> 25.4; 16 channels: 1600 rows 14.5 -> 8.6, 358,400 rows 38.9 -> 27.0.
 
 typedef __bf16 cu_bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 cu_bf16x2 __attribute__((ext_vector_type(2)));
 typedef float cu_floatx2 __attribute__((ext_vector_type(2)));
 typedef float cu_floatx4 __attribute__((ext_vector_type(4)));
+typedef float cu_weights4 __attribute__((ext_vector_type(4), aligned(4)));  // four floats at any float's address
 
 constexpr int kUnitThreads = 256;
 constexpr int kUnitTaps = 7;
 
-// 16-row tiles per wave (256 output rows per workgroup): 8 and 16 tiles for 8 and 16 channels measured
-// 130 / 48 us against 85 / 39 us per launch, the workgroup's chain being latency-bound
-constexpr int kUnitStreamsLds = 1024;  // stream offsets searched in LDS (more streams: in global memory)
-template <int C>
-constexpr int unit_tiles() {
-    return 4;
-}
-template <int C>
-constexpr int unit_rows() {
-    return kUnitThreads / kWave * unit_tiles<C>() * 16;  // output rows per workgroup
-}
+constexpr int unit_rows(int MT) { return kUnitThreads / kWave * MT * 16; }  // output rows per workgroup
 
 __device__ __forceinline__ uint32_t cu_pack(float a, float b) {
     return __builtin_bit_cast(uint32_t, __builtin_convertvector((cu_floatx2){a, b}, cu_bf16x2));
@@ -1045,6 +1083,12 @@ __device__ __forceinline__ void cu_split2(float a, float b, uint32_t &hi, uint32
     lo = cu_pack(a - __uint_as_float(hi << 16), b - __uint_as_float(hi & 0xffff0000u));
 }
 
+// hi / lo words of four values
+__device__ __forceinline__ void cu_split4(float a, float b, float c, float d, uint2 &hi, uint2 &lo) {
+    cu_split2(a, b, hi.x, lo.x);
+    cu_split2(c, d, hi.y, lo.y);
+}
+
 __device__ __forceinline__ cu_bf16x8 cu_frag(const uint4 &v) { return __builtin_bit_cast(cu_bf16x8, v); }
 
 template <int C>
@@ -1053,110 +1097,112 @@ constexpr int unit_ksteps() {
 }
 
 template <int C>
-size_t unit_mfma_lds(int pad) {
-    constexpr int NT = C <= 16 ? 1 : 2;
+size_t unit_mfma_lds(int pad, int MT) {
+    constexpr int NT = C / 16;
     constexpr int RB = 4 * C + 16;
     return static_cast<size_t>(unit_ksteps<C>() * NT * 2 * kWave + NT * 2 * kWave) * 16 +
-           static_cast<size_t>(unit_rows<C>() + pad) * RB + static_cast<size_t>(kUnitThreads / kWave) * 16 * RB;
+           static_cast<size_t>(unit_rows(MT) + pad) * RB + static_cast<size_t>(kUnitThreads / kWave) * 16 * RB;
 }
 
-template <int C>
+template <int C, int MT>
 __global__ void __launch_bounds__(kUnitThreads)
 unit_mfma_kernel(const float *__restrict__ x, int64_t ldx, int64_t T, const int32_t *__restrict__ off, int B, int u,
                  const int32_t *__restrict__ slots, const float *__restrict__ hist, int dil,
                  const float *__restrict__ w1, const float *__restrict__ b1, Act act1,
                  const float *__restrict__ w2, const float *__restrict__ b2, Act act2,
                  float *__restrict__ out, int64_t ldo) {
-    static_assert(C == 8 || C == 16 || C == 32, "8, 16 or 32 channels");
-    constexpr int NT = C <= 16 ? 1 : 2;     // 16-wide output-channel tiles
+    static_assert(C == 16 || C == 32, "16 or 32 channels");
+    constexpr int NT = C / 16;               // 16-wide output-channel tiles
     constexpr int KS = unit_ksteps<C>();     // 32-k steps of the 7-tap convolution
     constexpr int RB = 4 * C + 16;           // LDS row bytes
     constexpr int VPR = C / 4;               // float4 per input row
-    constexpr int MT = unit_tiles<C>();      // 16-row tiles per wave
-    constexpr int ROWS = unit_rows<C>();     // output rows per workgroup
+    constexpr int ROWS = unit_rows(MT);      // output rows per workgroup
+    constexpr int kBatch = MT == 1 ? 4 : 8;  // 128-bit loads in flight per thread
     extern __shared__ __attribute__((aligned(16))) char ulds[];
     __shared__ float sp[4][32];              // snake1 a, 1/b; snake2 a, 1/b
-    __shared__ int32_t soff[kUnitStreamsLds + 1];
     uint4 *wf1 = reinterpret_cast<uint4 *>(ulds);      // [KS][NT][hi, lo][64 lanes]
     uint4 *wf2 = wf1 + KS * NT * 2 * kWave;            // [NT][hi, lo][64 lanes]
     char *xs = reinterpret_cast<char *>(wf2 + NT * 2 * kWave);
     const int pad = (kUnitTaps - 1) * dil;
     char *ys = xs + (ROWS + pad) * RB;                 // [wave][16 rows][RB]
     const int tid = threadIdx.x;
-    const int64_t row0 = static_cast<int64_t>(blockIdx.x) * ROWS;
 
-    // 1. the input rows row0 - pad .. row0 + ROWS - 1, activated and split (rows outside [0, T) zero), in
-    // batches of eight 128-bit loads per thread; the first batch is issued before the weight table is
-    // built, so that its round trip overlaps the table's
-    const int nvec = (ROWS + pad) * VPR;
-    auto load_batch = [&](int e0, float4 (&v)[8]) {
+    // 1. thread t < C^2 / 4 holds the weights of output channel t / (C / 4) and four consecutive input
+    // channels: 28 consecutive floats of w1, four of w2; requested before the tile is known
+    const bool has_w = tid < C * C / 4;
+    cu_weights4 wr[kUnitTaps], wr2 = {};
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int e = e0 + i * kUnitThreads;
+    for (int i = 0; i < kUnitTaps; ++i)
+        wr[i] = *reinterpret_cast<const cu_weights4 *>(w1 + (has_w ? tid : 0) * 4 * kUnitTaps + 4 * i);
+    wr2 = *reinterpret_cast<const cu_weights4 *>(w2 + (has_w ? tid : 0) * 4);
+    StreamTile st;
+    if (!stream_tile(off, B, u, T, ROWS, static_cast<int>(blockIdx.x), st)) return;
+    x += st.first * ldx;
+    out += st.first * ldo;
+    const float *h = hist + (static_cast<int64_t>(slots[st.b]) * pad + pad) * C;  // row -1 lies before it
+
+    // 2. the input rows l0 - pad .. l0 + ROWS - 1 of the stream (the last one again past its end: those
+    // feed no stored output); the first batch is in flight while the weights are laid out
+    const int nvec = (ROWS + pad) * VPR;
+    auto load_batch = [&](int e0, float4 (&v)[kBatch]) {
+#pragma unroll
+        for (int i = 0; i < kBatch; ++i) {
+            const int e = e0 + i * kUnitThreads < nvec ? e0 + i * kUnitThreads : nvec - 1;
             const int rr = e / VPR;
-            const int64_t g = row0 - pad + rr;
-            v[i] = (e < nvec && g >= 0 && g < T)
-                       ? *reinterpret_cast<const float4 *>(x + g * ldx + (e - rr * VPR) * 4)
-                       : make_float4(0.f, 0.f, 0.f, 0.f);
+            int64_t l = st.l0 - pad + rr;
+            if (l >= st.n) l = st.n - 1;
+            const float *row = l < 0 ? h + l * C : x + l * ldx;
+            v[i] = *reinterpret_cast<const float4 *>(row + (e - rr * VPR) * 4);
         }
     };
-    auto store_batch = [&](int e0, const float4 (&v)[8]) {
+    auto store_batch = [&](int e0, const float4 (&v)[kBatch]) {
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
+        for (int i = 0; i < kBatch; ++i) {
             const int e = e0 + i * kUnitThreads;
             if (e >= nvec) break;
             const int rr = e / VPR, c4 = (e - rr * VPR) * 4;
-            const int64_t g = row0 - pad + rr;
             float f[4] = {v[i].x, v[i].y, v[i].z, v[i].w};
-            if (act1.alpha && g >= 0 && g < T) {
+            if (act1.alpha && st.l0 - pad + rr >= 0) {
 #pragma unroll
                 for (int q = 0; q < 4; ++q) f[q] = snake(f[q], sp[0][c4 + q], sp[1][c4 + q]);
             }
-            uint32_t h0, l0, h1, l1;
-            cu_split2(f[0], f[1], h0, l0);
-            cu_split2(f[2], f[3], h1, l1);
-            *reinterpret_cast<uint2 *>(xs + rr * RB + 2 * c4) = make_uint2(h0, h1);
-            *reinterpret_cast<uint2 *>(xs + rr * RB + 2 * C + 2 * c4) = make_uint2(l0, l1);
+            uint2 hi, lo;
+            cu_split4(f[0], f[1], f[2], f[3], hi, lo);
+            *reinterpret_cast<uint2 *>(xs + rr * RB + 2 * c4) = hi;
+            *reinterpret_cast<uint2 *>(xs + rr * RB + 2 * C + 2 * c4) = lo;
         }
     };
-    float4 vb[8];
+    float4 vb[kBatch];
     load_batch(tid, vb);
 
-    // 2. the weights as split MFMA A fragments: lane (r16, kq) of step j holds W[co = 16 nt + r16][k = 32 j + 8 kq .. + 7]
-    for (int e = tid; e < KS * NT * kWave; e += kUnitThreads) {
-        const int ln = e % kWave, nt = (e / kWave) % NT, j = e / (kWave * NT);
-        const int co = nt * 16 + (ln & 15), k0 = 32 * j + 8 * (ln >> 4);
-        uint32_t hi[4], lo[4];
+    // 3. the weights as split MFMA A fragments: lane (r16, kq) of step j holds W[co = 16 nt + r16][k = 32 j + 8 kq .. + 7]
+    if (has_w) {
+        const int co = tid / (C / 4), ci = tid % (C / 4) * 4;
+        // the half fragment of the four channels at k: hi words, and lo words one fragment on
+        auto put = [&](uint4 *frag, int lane, int ci_in, const uint2 &hi, const uint2 &lo) {
+            uint2 *at = reinterpret_cast<uint2 *>(frag + lane) + (ci_in >> 2);
+            at[0] = hi;
+            at[2 * kWave] = lo;
+        };
 #pragma unroll
-        for (int p = 0; p < 4; ++p) {
-            float v2[2];
+        for (int tap = 0; tap < KS * 32 / C; ++tap) {
+            uint2 hi = make_uint2(0, 0), lo = make_uint2(0, 0);
+            if (tap < kUnitTaps) {
+                float f[4];
 #pragma unroll
-            for (int q = 0; q < 2; ++q) {
-                const int kk = k0 + 2 * p + q, tap = kk / C, ci = kk - (kk / C) * C;
-                v2[q] = (co < C && tap < kUnitTaps) ? w1[(static_cast<int64_t>(co) * C + ci) * kUnitTaps + tap] : 0.f;
+                for (int p = 0; p < 4; ++p) f[p] = wr[(p * kUnitTaps + tap) / 4][(p * kUnitTaps + tap) % 4];
+                cu_split4(f[0], f[1], f[2], f[3], hi, lo);
             }
-            cu_split2(v2[0], v2[1], hi[p], lo[p]);
+            const int k = (tap * C) % 32 + ci;
+            put(wf1 + ((tap * C / 32 * NT + co / 16) * 2) * kWave, (k >> 3) * 16 + (co & 15), k & 7, hi, lo);
         }
-        wf1[((j * NT + nt) * 2) * kWave + ln] = make_uint4(hi[0], hi[1], hi[2], hi[3]);
-        wf1[((j * NT + nt) * 2 + 1) * kWave + ln] = make_uint4(lo[0], lo[1], lo[2], lo[3]);
+        uint2 hi, lo;
+        cu_split4(wr2[0], wr2[1], wr2[2], wr2[3], hi, lo);
+        put(wf2 + (co / 16 * 2) * kWave, (ci >> 3) * 16 + (co & 15), ci & 7, hi, lo);
+        if constexpr (C == 16)  // k 16 .. 31 of the 1x1 convolution
+            put(wf2 + (co / 16 * 2) * kWave, ((ci + 16) >> 3) * 16 + (co & 15), ci & 7, make_uint2(0, 0),
+                make_uint2(0, 0));
     }
-    for (int e = tid; e < NT * kWave; e += kUnitThreads) {
-        const int ln = e % kWave, nt = e / kWave;
-        const int co = nt * 16 + (ln & 15), ci0 = 8 * (ln >> 4);
-        uint32_t hi[4], lo[4];
-#pragma unroll
-        for (int p = 0; p < 4; ++p) {
-            const int ci = ci0 + 2 * p;
-            const float a = (co < C && ci < C) ? w2[co * C + ci] : 0.f;
-            const float b = (co < C && ci + 1 < C) ? w2[co * C + ci + 1] : 0.f;
-            cu_split2(a, b, hi[p], lo[p]);
-        }
-        wf2[(nt * 2) * kWave + ln] = make_uint4(hi[0], hi[1], hi[2], hi[3]);
-        wf2[(nt * 2 + 1) * kWave + ln] = make_uint4(lo[0], lo[1], lo[2], lo[3]);
-    }
-    const bool off_lds = B <= kUnitStreamsLds;
-    if (off_lds)
-        for (int i = tid; i <= B; i += kUnitThreads) soff[i] = off[i];
     if (tid < C) {
         sp[0][tid] = act1.alpha ? act1.a_of(tid) : 0.f;
         sp[1][tid] = act1.alpha ? act1.inv_b_of(tid) : 0.f;
@@ -1164,46 +1210,26 @@ unit_mfma_kernel(const float *__restrict__ x, int64_t ldx, int64_t T, const int3
         sp[3][tid] = act2.alpha ? act2.inv_b_of(tid) : 0.f;
     }
 
-    __syncthreads();  // the snake parameters and stream offsets
+    __syncthreads();  // the snake parameters
     store_batch(tid, vb);
-    for (int e0 = tid + 8 * kUnitThreads; e0 < nvec; e0 += 8 * kUnitThreads) {
+    for (int e0 = tid + kBatch * kUnitThreads; e0 < nvec; e0 += kBatch * kUnitThreads) {
         load_batch(e0, vb);
         store_batch(e0, vb);
     }
     __syncthreads();
 
-    // 3. the 7-tap convolution: wave w owns rows row0 + (MT w + m) 16 + r16, m < MT
+    // 4. the 7-tap convolution: wave w owns rows l0 + (MT w + m) 16 + r16, m < MT
     const int lane = tid & (kWave - 1), wave = tid / kWave;
     const int r16 = lane & 15, kq = lane >> 4;
-    // the lane's row of tile m is row0 + (MT w + m) 16 + r16; its offset from its stream's first row
-    // (pad when far enough: the rows of a workgroup lie in few streams, so the search runs once per tile)
-    const int32_t *offs = off_lds ? soff : off;
-    int local[MT];
-    bool near_start = false;
-#pragma unroll
-    for (int m = 0; m < MT; ++m) {
-        const int64_t t = row0 + (wave * MT + m) * 16 + r16;
-        local[m] = pad;
-        if (t < T) {
-            const int b = stream_of(offs, B, t, u);
-            const int64_t l = t - static_cast<int64_t>(offs[b]) * u;
-            local[m] = l < pad ? static_cast<int>(l) : pad;
-            near_start = near_start || l < pad;
-        }
-    }
     // the residual rows of the epilogue, loaded now so that their round trip overlaps the MFMAs
     float4 xres[MT][NT];
 #pragma unroll
     for (int m = 0; m < MT; ++m) {
-        const int64_t t = row0 + (wave * MT + m) * 16 + r16;
+        const int64_t l = st.l0 + (wave * MT + m) * 16 + r16;
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt) {
-            const int co = nt * 16 + 4 * kq;
-            xres[m][nt] = (co < C && t < T) ? *reinterpret_cast<const float4 *>(x + t * ldx + co)
-                                            : make_float4(0.f, 0.f, 0.f, 0.f);
-        }
+        for (int nt = 0; nt < NT; ++nt)
+            xres[m][nt] = *reinterpret_cast<const float4 *>(x + (l < st.n ? l : st.n - 1) * ldx + nt * 16 + 4 * kq);
     }
-    const bool slow = __any(near_start);
     cu_floatx4 acc[MT][NT];
 #pragma unroll
     for (int m = 0; m < MT; ++m)
@@ -1222,20 +1248,8 @@ unit_mfma_kernel(const float *__restrict__ x, int64_t ldx, int64_t T, const int3
 #pragma unroll
         for (int m = 0; m < MT; ++m) {
             const char *rp = xs + ((wave * MT + m) * 16 + r16 + pad - back) * RB + 2 * cb;
-            uint4 bh = *reinterpret_cast<const uint4 *>(rp);
-            uint4 bl = *reinterpret_cast<const uint4 *>(rp + 2 * C);
-            if (slow && tap < kUnitTaps && local[m] - back < 0) {
-                // a row within pad of its stream's start: this tap reads the stream's history
-                const int b = stream_of(offs, B, row0 + (wave * MT + m) * 16 + r16, u);
-                const float *hp =
-                    hist + (static_cast<int64_t>(slots[b]) * pad + pad + local[m] - back) * C + cb;
-                const float4 h0 = *reinterpret_cast<const float4 *>(hp);
-                const float4 h1 = *reinterpret_cast<const float4 *>(hp + 4);
-                cu_split2(h0.x, h0.y, bh.x, bl.x);
-                cu_split2(h0.z, h0.w, bh.y, bl.y);
-                cu_split2(h1.x, h1.y, bh.z, bl.z);
-                cu_split2(h1.z, h1.w, bh.w, bl.w);
-            }
+            const uint4 bh = *reinterpret_cast<const uint4 *>(rp);
+            const uint4 bl = *reinterpret_cast<const uint4 *>(rp + 2 * C);
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt) {
                 acc[m][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al[nt], cu_frag(bh), acc[m][nt], 0, 0, 0);
@@ -1245,7 +1259,7 @@ unit_mfma_kernel(const float *__restrict__ x, int64_t ldx, int64_t T, const int3
         }
     }
 
-    // 4. per tile: y = snake2(conv + b1), split into the wave's own 16 LDS rows (lane (r16, kq) holds
+    // 5. per tile: y = snake2(conv + b1), split into the wave's own 16 LDS rows (lane (r16, kq) holds
     // y[row r16][co = 16 nt + 4 kq .. + 3]), read back as the B operand of the 1x1 convolution (lane
     // (r16, kq) = y[row r16][ci = 8 kq .. + 7]), then the residual
     char *yw = ys + wave * 16 * RB;
@@ -1260,19 +1274,17 @@ unit_mfma_kernel(const float *__restrict__ x, int64_t ldx, int64_t T, const int3
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) {
             const int co = nt * 16 + 4 * kq;
-            if (co >= C) continue;
             float y[4];
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 y[e] = acc[m][nt][e] + (b1 ? b1[co + e] : 0.f);
                 if (act2.alpha) y[e] = snake(y[e], sp[2][co + e], sp[3][co + e]);
             }
-            uint32_t h0, l0, h1, l1;
-            cu_split2(y[0], y[1], h0, l0);
-            cu_split2(y[2], y[3], h1, l1);
+            uint2 hi, lo;
+            cu_split4(y[0], y[1], y[2], y[3], hi, lo);
             char *rp = yw + r16 * RB + 2 * co;
-            *reinterpret_cast<uint2 *>(rp) = make_uint2(h0, h1);
-            *reinterpret_cast<uint2 *>(rp + 2 * C) = make_uint2(l0, l1);
+            *reinterpret_cast<uint2 *>(rp) = hi;
+            *reinterpret_cast<uint2 *>(rp + 2 * C) = lo;
         }
         __builtin_amdgcn_wave_barrier();  // the wave reads back what its own lanes wrote (LDS keeps its order)
         uint4 bh = make_uint4(0, 0, 0, 0), bl = make_uint4(0, 0, 0, 0);
@@ -1282,24 +1294,35 @@ unit_mfma_kernel(const float *__restrict__ x, int64_t ldx, int64_t T, const int3
             bl = *reinterpret_cast<const uint4 *>(rp + 2 * C);
         }
         __builtin_amdgcn_wave_barrier();  // every lane has read the tile before the next one is written
-        const int64_t t = row0 + (wave * MT + m) * 16 + r16;
+        const int64_t l = st.l0 + (wave * MT + m) * 16 + r16;
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) {
             cu_floatx4 d = cu_floatx4{0.f, 0.f, 0.f, 0.f};
             d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a2l[nt], cu_frag(bh), d, 0, 0, 0);
             d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a2h[nt], cu_frag(bl), d, 0, 0, 0);
             d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a2h[nt], cu_frag(bh), d, 0, 0, 0);
+            if (l >= st.n) continue;
             const int co = nt * 16 + 4 * kq;
-            if (co >= C || t >= T) continue;
             const float4 xr = xres[m][nt];
             float4 o;
             o.x = xr.x + d[0] + (b2 ? b2[co] : 0.f);
             o.y = xr.y + d[1] + (b2 ? b2[co + 1] : 0.f);
             o.z = xr.z + d[2] + (b2 ? b2[co + 2] : 0.f);
             o.w = xr.w + d[3] + (b2 ? b2[co + 3] : 0.f);
-            *reinterpret_cast<float4 *>(out + t * ldo + co) = o;
+            *reinterpret_cast<float4 *>(out + l * ldo + co) = o;
         }
     }
+}
+
+// 16-row tiles per wave.  One while the 64-row workgroups fit on the chip at once (32 channels: 58 KB of
+// LDS, two per CU; 16 channels: 25 KB, where four per CU is the measured line): the shortest chain.  Past
+// that the rows before a tile, staged again by the next, and the weights weigh more: 32 channels at
+// dilation 9, 89,600 rows: 28.1 / 25.4 / 35.4 us with 1 / 2 / 4 tiles (9600 rows: 12.1 / 14.7 / 20.2);
+// 16 channels, 358,400 rows: 30.5 / 27.7 / 27.0 (38,400 rows: 10.4 / 11.4 / 12.7).
+int unit_tiles(int C, int64_t T, int B) {
+    const int64_t small = stream_tiles_bound(T, B, unit_rows(1));
+    if (C == 16) return small <= 4 * kCus ? 1 : 4;
+    return small <= 2 * kCus ? 1 : 2;
 }
 
 int grid_for(int64_t n) {
@@ -1333,23 +1356,27 @@ extern "C" int nq_codec_causal_conv(const float *x, int64_t ldx, int64_t T, cons
     NQ_CHECK_ARG(ldx >= Cin && ldo >= Cout && (!residual || ldres >= Cout));
     const int pad = (K - 1) * dilation;
     NQ_CHECK_ARG(pad == 0 || history);
-    if (pad * Cin > kCodecThreads * kHistoryPerThread) return NQ_ERR_UNSUPPORTED;
+    if (pad * Cin > kHistoryThreads * kHistoryPerThread) return NQ_ERR_UNSUPPORTED;
     if (T == 0) return NQ_OK;
     hipStream_t st = static_cast<hipStream_t>(stream);
     const Act act{act_alpha, act_beta};
-    const int co_pad = Cout <= 8 ? 8 : Cout <= 16 ? 16 : Cout <= 32 ? 32 : 64;
-    if (groups == 1 && Cin <= 64 && Cout <= 64 && conv_small_lds(Cin, K, dilation, co_pad) <= 150 * 1024) {
-        const size_t lds = conv_small_lds(Cin, K, dilation, co_pad);
-        const int64_t rows = static_cast<int64_t>(kCodecThreads) * conv_small_rows(co_pad);
-        const dim3 grid(static_cast<unsigned>((T + rows - 1) / rows));
-#define NQ_SMALL(CO)                                                                                              \
-        hipLaunchKernelGGL((conv_small_kernel<CO, conv_small_rows(CO)>), grid, dim3(kCodecThreads), lds, st, x, ldx, \
-                           T, offsets, B, u, slots, history, w, bias, Cin, Cout, K, dilation, act, residual, ldres,   \
-                           out, ldo)
-        if (co_pad == 8) NQ_SMALL(8);
-        else if (co_pad == 16) NQ_SMALL(16);
-        else if (co_pad == 32) NQ_SMALL(32);
-        else NQ_SMALL(64);
+    const int co_pad = Cout == 1 ? 1 : Cout <= 8 ? 8 : Cout <= 16 ? 16 : Cout <= 32 ? 32 : 64;
+    const int R = conv_small_rows(co_pad, T, B);
+    const int most = co_pad <= 16 ? 2 : 1;  // rows per thread the rule may choose
+    if (groups == 1 && Cin <= 64 && Cout <= 64 && conv_small_lds(Cin, K, dilation, co_pad, most) <= kConvLds) {
+        const size_t lds = conv_small_lds(Cin, K, dilation, co_pad, R);
+        const dim3 grid(static_cast<unsigned>(stream_tiles_bound(T, B, kCodecThreads * R)));
+#define NQ_SMALL(CO, R)                                                                                              \
+        hipLaunchKernelGGL((conv_small_kernel<CO, R>), grid, dim3(kCodecThreads), lds, st, x, ldx, T, offsets, B, u, \
+                           slots, history, w, bias, Cin, Cout, K, dilation, act, residual, ldres, out, ldo)
+        if (co_pad == 1 && R == 1) NQ_SMALL(1, 1);
+        else if (co_pad == 1) NQ_SMALL(1, 2);
+        else if (co_pad == 8 && R == 1) NQ_SMALL(8, 1);
+        else if (co_pad == 8) NQ_SMALL(8, 2);
+        else if (co_pad == 16 && R == 1) NQ_SMALL(16, 1);
+        else if (co_pad == 16) NQ_SMALL(16, 2);
+        else if (co_pad == 32) NQ_SMALL(32, 1);
+        else NQ_SMALL(64, 1);
 #undef NQ_SMALL
     } else if (groups == 1) {
         const int cg = Cout <= 16 ? 1 : Cout <= 32 ? 2 : 4;
@@ -1370,7 +1397,7 @@ extern "C" int nq_codec_causal_conv(const float *x, int64_t ldx, int64_t T, cons
     }
     if (hipGetLastError() != hipSuccess) return NQ_ERR_LAUNCH;
     if (pad > 0) {
-        hipLaunchKernelGGL(history_update_kernel, dim3(B), dim3(kCodecThreads),
+        hipLaunchKernelGGL(history_update_kernel, dim3(B), dim3(kHistoryThreads),
                            0, st, x, ldx, offsets, B, u, slots, history, Cin, pad, groups == 1 ? act : Act{nullptr, nullptr});
     }
     return NQ_LAUNCH_STATUS();
@@ -1385,7 +1412,7 @@ extern "C" int nq_codec_residual_unit(const float *x, int64_t ldx, int64_t T, co
     NQ_CHECK_ARG(C > 0 && K >= 2 && K <= kConvKMax && dilation >= 1 && ldx >= C && ldo >= C && out != x);
     NQ_CHECK_ARG(precision == NQ_MATMUL_HIGHEST || precision == NQ_MATMUL_HIGH);
     if (K != kConvKMax) return NQ_ERR_UNSUPPORTED;  // the fused kernels are built for 7 taps
-    if ((K - 1) * dilation * C > kCodecThreads * kHistoryPerThread) return NQ_ERR_UNSUPPORTED;
+    if ((K - 1) * dilation * C > kHistoryThreads * kHistoryPerThread) return NQ_ERR_UNSUPPORTED;
     NQ_CHECK_ARG((a1_alpha == nullptr) == (a1_beta == nullptr) && (a2_alpha == nullptr) == (a2_beta == nullptr));
     const int co_pad = C <= 8 ? 8 : C <= 16 ? 16 : 32;
     if (C > 32 || C != co_pad) return NQ_ERR_UNSUPPORTED;
@@ -1397,36 +1424,37 @@ extern "C" int nq_codec_residual_unit(const float *x, int64_t ldx, int64_t T, co
     if (split && (ldx % 4 || ldo % 4 || ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(out) |
                                           reinterpret_cast<uintptr_t>(history)) & 15)))
         return NQ_ERR_UNSUPPORTED;
-    const size_t lds = split ? (C == 8 ? unit_mfma_lds<8>(pad) : C == 16 ? unit_mfma_lds<16>(pad)
-                                                                          : unit_mfma_lds<32>(pad))
-                             : conv_small_lds(C, K, dilation, co_pad, true);
-    if (lds > 150 * 1024) return NQ_ERR_UNSUPPORTED;
+    const int R = conv_small_rows(co_pad, T, B), MT = unit_tiles(C, T, B);
+    const size_t lds = split ? (C == 16 ? unit_mfma_lds<16>(pad, MT) : unit_mfma_lds<32>(pad, MT))
+                             : conv_small_lds(C, K, dilation, co_pad, R, true);
+    if (lds > kConvLds) return NQ_ERR_UNSUPPORTED;
     if (T == 0) return NQ_OK;
     hipStream_t st = static_cast<hipStream_t>(stream);
     const Act act1{a1_alpha, a1_beta}, act2{a2_alpha, a2_beta};
     if (split) {
-#define NQ_UNIT(CC)                                                                                                  \
-        hipLaunchKernelGGL(unit_mfma_kernel<CC>, dim3(static_cast<unsigned>((T + unit_rows<CC>() - 1) / unit_rows<CC>())), \
-                           dim3(kUnitThreads), lds, st, x, ldx, T, offsets, B, u, slots, history, dilation, w1, b1,     \
-                           act1, w2, b2, act2, out, ldo)
-        if (C == 8) NQ_UNIT(8);
-        else if (C == 16) NQ_UNIT(16);
-        else NQ_UNIT(32);
+        const dim3 grid(static_cast<unsigned>(stream_tiles_bound(T, B, unit_rows(MT))));
+#define NQ_UNIT(CC, MT)                                                                                         \
+        hipLaunchKernelGGL((unit_mfma_kernel<CC, MT>), grid, dim3(kUnitThreads), lds, st, x, ldx, T, offsets, B, u, \
+                           slots, history, dilation, w1, b1, act1, w2, b2, act2, out, ldo)
+        if (C == 16 && MT == 1) NQ_UNIT(16, 1);
+        else if (C == 16) NQ_UNIT(16, 4);
+        else if (MT == 1) NQ_UNIT(32, 1);
+        else NQ_UNIT(32, 2);
 #undef NQ_UNIT
     } else {
-        const int64_t rows = static_cast<int64_t>(kCodecThreads) * conv_small_rows(co_pad);
-        const dim3 grid(static_cast<unsigned>((T + rows - 1) / rows));
-#define NQ_UNIT(CO)                                                                                                 \
-        hipLaunchKernelGGL((conv_small_kernel<CO, conv_small_rows(CO), true>), grid, dim3(kCodecThreads), lds, st, x, \
-                           ldx, T, offsets, B, u, slots, history, w1, b1, C, C, K, dilation, act1, x, ldx, out, ldo, \
-                           w2, b2, act2)
-        if (co_pad == 8) NQ_UNIT(8);
-        else if (co_pad == 16) NQ_UNIT(16);
-        else NQ_UNIT(32);
+        const dim3 grid(static_cast<unsigned>(stream_tiles_bound(T, B, kCodecThreads * R)));
+#define NQ_UNIT(CO, R)                                                                                               \
+        hipLaunchKernelGGL((conv_small_kernel<CO, R, true>), grid, dim3(kCodecThreads), lds, st, x, ldx, T, offsets, \
+                           B, u, slots, history, w1, b1, C, C, K, dilation, act1, x, ldx, out, ldo, w2, b2, act2)
+        if (co_pad == 8 && R == 1) NQ_UNIT(8, 1);
+        else if (co_pad == 8) NQ_UNIT(8, 2);
+        else if (co_pad == 16 && R == 1) NQ_UNIT(16, 1);
+        else if (co_pad == 16) NQ_UNIT(16, 2);
+        else NQ_UNIT(32, 1);
 #undef NQ_UNIT
     }
     if (hipGetLastError() != hipSuccess) return NQ_ERR_LAUNCH;
-    hipLaunchKernelGGL(history_update_kernel, dim3(B), dim3(kCodecThreads), 0, st,
+    hipLaunchKernelGGL(history_update_kernel, dim3(B), dim3(kHistoryThreads), 0, st,
                        x, ldx, offsets, B, u, slots, history, C, (K - 1) * dilation, act1);
     return NQ_LAUNCH_STATUS();
 }
@@ -1599,8 +1627,8 @@ extern "C" int nq_codec_history_update(const float *x, int64_t ldx, const int32_
                                        const float *act_beta, void *stream) {
     NQ_CHECK_ARG(x && offsets && slots && history && B > 0 && u > 0 && C > 0 && pad > 0 && ldx >= C);
     NQ_CHECK_ARG((act_alpha == nullptr) == (act_beta == nullptr));
-    if (pad * C > nq::kCodecThreads * nq::kHistoryPerThread) return NQ_ERR_UNSUPPORTED;
-    hipLaunchKernelGGL(history_update_kernel, dim3(B), dim3(kCodecThreads), 0,
+    if (pad * C > nq::kHistoryThreads * nq::kHistoryPerThread) return NQ_ERR_UNSUPPORTED;
+    hipLaunchKernelGGL(history_update_kernel, dim3(B), dim3(kHistoryThreads), 0,
                        static_cast<hipStream_t>(stream), x, ldx, offsets, B, u, slots, history, C, pad,
                        Act{act_alpha, act_beta});
     return NQ_LAUNCH_STATUS();

@@ -303,3 +303,59 @@ def test_window_attention_kernel_against_the_oracle(nq, device, D, H, window):
         np.testing.assert_allclose(got_sk[s, valid:], keys[len(keys) - R :][valid:], atol=1e-4, rtol=1e-4,
                                    err_msg=f"retained keys, stream {b}")
         np.testing.assert_array_equal(got_sv[s, valid:], vals[len(vals) - R :][valid:])
+
+
+# streams' rows around the tiles' edges (16, 64 and 256 rows, with histories longer than a stream), more streams
+# than a wave counts at a time, and enough rows for the shapes that large calls take
+TILE_STREAMS = {
+    "edges": [1, 15, 16, 17, 0, 63, 64, 65, 255, 256, 257, 2, 513],
+    "many": [(37 * i) % 131 for i in range(150)],
+    "large": [70000, 3, 300, 0, 1000],
+}
+
+
+@pytest.mark.parametrize("streams", list(TILE_STREAMS))
+@pytest.mark.parametrize("channels", [8, 16, 32])
+def test_convolution_tiles_keep_to_their_stream(nq, device, channels, streams):
+    """Narrow convolutions (the residual unit at both precisions, and one to a single output channel) on integer
+    operands, whose sums are exact in fp32 and whose operands split exactly: equal to each stream's own
+    convolution of [history ; rows] on the host, and the histories are its last rows."""
+    from nari_qwen3_tts_amd import _lib
+
+    rows, c, k, dilation = TILE_STREAMS[streams], channels, 7, 9
+    B, T, pad = len(rows), sum(rows), (k - 1) * dilation
+    g = torch.Generator().manual_seed(c + B)
+    r = lambda *shape, lim=3: torch.randint(-lim, lim + 1, shape, generator=g).float()  # noqa: E731
+    x, hist0 = r(T, c), r(B + 1, pad, c)
+    w1, b1, w2, b2, w3 = r(c, c, k, lim=1), r(c), r(c, c, 1, lim=1), r(c), r(1, c, k)
+    slots = torch.randperm(B + 1, generator=g)[:B].int()
+    off = torch.tensor(np.concatenate([[0], np.cumsum(rows)]), dtype=torch.int32)
+    conv = torch.nn.functional.conv1d
+    want, want1, want_hist = [], [], hist0.clone()
+    for b in range(B):
+        xb = x[off[b] : off[b + 1]]
+        cat = torch.cat([hist0[slots[b]], xb])
+        want_hist[slots[b]] = cat[len(cat) - pad :]
+        if rows[b]:
+            y = conv(cat.t()[None], w1, b1, dilation=dilation)
+            want.append((conv(y, w2, b2)[0]).t() + xb)
+            want1.append(conv(cat.t()[None], w3, dilation=dilation)[0].t())
+    want, want1 = torch.cat(want), torch.cat(want1)
+
+    d = {n: t.to(device) for n, t in dict(x=x, w1=w1, b1=b1, w2=w2, b2=b2, w3=w3, off=off, slots=slots).items()}
+    st = _lib.stream(device)
+    for precision in (0, 1):
+        hist, got = hist0.to(device), torch.full((T, c), float("nan"), device=device)
+        _lib.call("nq_codec_residual_unit", d["x"].data_ptr(), c, T, d["off"].data_ptr(), B, 1, d["slots"].data_ptr(),
+                  hist.data_ptr(), c, k, dilation, d["w1"].data_ptr(), d["b1"].data_ptr(), None, None,
+                  d["w2"].data_ptr(), d["b2"].data_ptr(), None, None, got.data_ptr(), c, precision, st)
+        torch.cuda.synchronize()
+        assert torch.equal(got.cpu(), want)
+        assert torch.equal(hist.cpu(), want_hist)
+    hist, got = hist0.to(device), torch.full((T, 1), float("nan"), device=device)
+    _lib.call("nq_codec_causal_conv", d["x"].data_ptr(), c, T, d["off"].data_ptr(), B, 1, d["slots"].data_ptr(),
+              hist.data_ptr(), d["w3"].data_ptr(), None, c, 1, k, dilation, 1, None, None, None, 0, got.data_ptr(), 1,
+              st)
+    torch.cuda.synchronize()
+    assert torch.equal(got.cpu(), want1)
+    assert torch.equal(hist.cpu(), want_hist)
