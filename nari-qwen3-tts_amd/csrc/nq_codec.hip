@@ -797,19 +797,22 @@ overlap_fixup_kernel(const int32_t *__restrict__ off, int B, int u_in, int s, co
 // i0 - R + kappa < 0, else fresh frame f = i0 - R + kappa, rotated here (and
 // written back in place, so a later block reads it rotated) unless an earlier
 // block already did.  K, V and the rotated q of a block are staged in LDS
-// (rows of D + 4 floats); query lane j then reads key row j + s for window
-// step s, so the 64 lanes read 64 consecutive rows and a 16-byte read covers
-// every bank once.  The four waves split the channels: wave w forms partial
-// scores over its D/4 channels, the partials meet in LDS, every wave finishes
-// the softmax of its lanes and accumulates P V over its own channels.  After
-// the last block the new retained rows (the last R positions) are written from
+// (rows of D + 4 floats).  Eight queries then go at a time, a thread each
+// (query j, window step s), which reads key row j + s: 32 lanes read 32
+// consecutive rows, and a 16-byte read spreads over the banks.  A query's
+// scores lie in half a wave, which finds its softmax with shuffles and takes
+// its channels for P V.  What bounds a launch is this chain, and the code it
+// is written in: with a query a lane and the window's steps unrolled (25 KB
+// of code, four lanes of 64 at work on a four-frame chunk) a launch took
+// 17 us at one stream of four frames and 18.5 us at 32 of 12 - 48, and takes
+// 8.5 and 18.0.  After the last block the new retained rows (the last R positions) are written from
 // LDS: the state is read (staged) before this workgroup overwrites it, and no
 // other workgroup touches this (stream, head).
 
 constexpr int kWinThreads = 256;
-constexpr int kWinWaves = kWinThreads / kWave;
-constexpr int kWinQ = 64;     // queries per block (one per lane)
+constexpr int kWinQ = 64;     // queries per block
 constexpr int kWinMax = 32;   // window (R + 1) the kernel takes
+constexpr int kWinGroup = kWinThreads / kWinMax;  // queries whose (query, step) pairs are one per thread
 
 template <int D>
 __global__ void __launch_bounds__(kWinThreads)
@@ -819,18 +822,16 @@ window_block_kernel(const float *__restrict__ q, float *__restrict__ k, const fl
                     const int64_t *__restrict__ frame_pos, const int32_t *__restrict__ ctx_len, float *state_k,
                     float *state_v, int64_t state_slot_stride, int R, float scale, float *__restrict__ out,
                     int64_t ldo) {
-    static_assert(D % 16 == 0 && D <= 64, "four waves of D / 4 channels, 4-channel chunks");
+    static_assert(D % 16 == 0 && D <= 64, "rows of 4-channel chunks, whole rows a pass");
     constexpr int P = D + 4;                // LDS row pitch (floats)
     constexpr int LPR = D / 4;              // lanes (4-channel chunks) per row
     constexpr int RPP = kWinThreads / LPR;  // rows staged per pass
-    constexpr int DW = D / kWinWaves;       // channels per wave
-    constexpr int CW = DW / 4;              // chunks per wave
     constexpr int HALF = D / 2;             // rotated pairs
     static_assert(kWinThreads % HALF == 0, "a thread makes the angles of one pair");
     __shared__ __attribute__((aligned(16))) float ks[(kWinMax - 1 + kWinQ) * P];
     __shared__ __attribute__((aligned(16))) float vs[(kWinMax - 1 + kWinQ) * P];
     __shared__ __attribute__((aligned(16))) float qs[kWinQ * P];
-    __shared__ float ps[kWinWaves * kWinMax * kWinQ];
+    __shared__ float ps[kWinThreads];
     __shared__ __attribute__((aligned(16))) float cosines[kWinQ * HALF];
     __shared__ __attribute__((aligned(16))) float sines[kWinQ * HALF];
 
@@ -842,7 +843,6 @@ window_block_kernel(const float *__restrict__ q, float *__restrict__ k, const fl
     const int ctx = ctx_len[slot];
     const int64_t P0 = frame_pos[slot];
     const int W = R + 1;
-    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
     const int c = threadIdx.x % LPR;  // the thread's 4-channel chunk when staging
     float *sk = state_k + static_cast<int64_t>(slot) * state_slot_stride + h * D;
     float *sv = state_v + static_cast<int64_t>(slot) * state_slot_stride + h * D;
@@ -853,8 +853,8 @@ window_block_kernel(const float *__restrict__ q, float *__restrict__ k, const fl
     // (channels d and d + D / 2, inv_freq of pair d = theta^(-2d/D)), as the reference rotates them.
     // The block's cosines and sines are made once, in LDS, while its loads are in flight, and serve
     // q and k: with a sincosf in each of the unrolled rows the kernel was a long straight line of
-    // code, and fetching it cost as much as its work: 32 streams of 12 - 48 frames decode in 1845 us where they
-    // took 1871 (20.7 us of each of eight launches).
+    // code, and fetching it cost as much as its work: 32 streams of 12 - 48
+    // frames decode in 1845 us where they took 1871 (20.7 us of each of eight launches).
     const bool first = c < LPR / 2;
     const int pair4 = 4 * (first ? c : c - LPR / 2);  // the chunk's first pair
     const float pair_freq = expf(-log_theta * (2.0f * static_cast<float>(threadIdx.x % HALF) / static_cast<float>(D)));
@@ -936,71 +936,51 @@ window_block_kernel(const float *__restrict__ q, float *__restrict__ k, const fl
         }
         __syncthreads();
 
-        // partial scores over wave w's channels: lane j = query i0 + j, window step s = key row j + s
-        const int j = lane;
-        const bool live = j < nq;
-        float4 qv[CW];
-#pragma unroll
-        for (int u = 0; u < CW; ++u)
-            qv[u] = live ? *reinterpret_cast<const float4 *>(qs + j * P + wave * DW + 4 * u) : make_float4(0, 0, 0, 0);
-#pragma unroll
-        for (int s = 0; s < kWinMax; ++s) {
-            if (s >= W) break;
-            float dot = 0.f;
-            if (live) {
-                const float *kr = ks + (j + s) * P + wave * DW;
-#pragma unroll
-                for (int u = 0; u < CW; ++u) {
-                    const float4 kk = *reinterpret_cast<const float4 *>(kr + 4 * u);
-                    dot += qv[u].x * kk.x + qv[u].y * kk.y + qv[u].z * kk.z + qv[u].w * kk.w;
+        // eight queries at a time, one thread per (query, window step): half a wave holds a query's
+        // scores, and its lanes then take the query's channels
+        for (int j0 = 0; j0 < nq; j0 += kWinGroup) {
+            const int j = j0 + threadIdx.x / kWinMax, s = threadIdx.x % kWinMax;
+            const int lowest = max(0, R - i0 - j - ctx);  // the first window step that holds a key
+            const bool valid = j < nq && s >= lowest && s < W;
+            float score = -INFINITY;
+            if (valid) {
+                const float *qr = qs + j * P, *kr = ks + (j + s) * P;
+                score = 0.f;
+#pragma unroll 4
+                for (int u = 0; u < D; u += 4) {
+                    const float4 qq = *reinterpret_cast<const float4 *>(qr + u);
+                    const float4 kk = *reinterpret_cast<const float4 *>(kr + u);
+                    score += qq.x * kk.x + qq.y * kk.y + qq.z * kk.z + qq.w * kk.w;
                 }
+                score *= scale;
             }
-            ps[(wave * kWinMax + s) * kWinQ + j] = dot;
-        }
-        __syncthreads();
-
-        // softmax of the lane's window (in every wave, for its own channels of P V)
-        float sc[kWinMax];
-        float mx = -INFINITY;
+            float mx = score;
 #pragma unroll
-        for (int s = 0; s < kWinMax; ++s) {
-            sc[s] = -INFINITY;
-            const int fi = i0 + j - R + s;  // the key's fresh index (< 0: retained slot R + fi)
-            if (s < W && live && (fi >= 0 || R + fi >= R - ctx)) {
-                float full = 0.f;
+            for (int m = kWinMax / 2; m; m >>= 1) mx = fmaxf(mx, __shfl_xor(mx, m, kWave));
+            const float pr = valid ? expf(score - mx) : 0.f;
+            float l = pr;
 #pragma unroll
-                for (int w = 0; w < kWinWaves; ++w) full += ps[(w * kWinMax + s) * kWinQ + j];
-                sc[s] = full * scale;
-                mx = fmaxf(mx, sc[s]);
-            }
-        }
-        float l = 0.f;
-        float acc[DW];
+            for (int m = kWinMax / 2; m; m >>= 1) l += __shfl_xor(l, m, kWave);
+            ps[threadIdx.x] = pr;  // read by the same half wave, whose LDS accesses complete in order
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            constexpr int CPL = D > kWinMax ? D / kWinMax : 1;  // channels per lane
+            if (j < nq && s * CPL < D) {
+                const float *pj = ps + threadIdx.x - s;
+                float acc[CPL] = {};
+#pragma unroll 4
+                for (int i = lowest; i < W; ++i) {
+                    const float *vr = vs + (j + i) * P + s * CPL;
 #pragma unroll
-        for (int d = 0; d < DW; ++d) acc[d] = 0.f;
-#pragma unroll
-        for (int s = 0; s < kWinMax; ++s) {
-            if (sc[s] != -INFINITY) {
-                const float pr = expf(sc[s] - mx);
-                l += pr;
-                const float *vr = vs + (j + s) * P + wave * DW;
-#pragma unroll
-                for (int u = 0; u < CW; ++u) {
-                    const float4 vv = *reinterpret_cast<const float4 *>(vr + 4 * u);
-                    acc[4 * u] += pr * vv.x;
-                    acc[4 * u + 1] += pr * vv.y;
-                    acc[4 * u + 2] += pr * vv.z;
-                    acc[4 * u + 3] += pr * vv.w;
+                    for (int e = 0; e < CPL; ++e) acc[e] += pj[i] * vr[e];
                 }
-            }
-        }
-        if (live) {
-            float *op = out + (t0 + i0 + j) * ldo + h * D + wave * DW;
-            const float il = 1.0f / l;
+                float *op = out + (t0 + i0 + j) * ldo + h * D + s * CPL;
+                const float il = 1.0f / l;
 #pragma unroll
-            for (int u = 0; u < CW; ++u)
-                *reinterpret_cast<float4 *>(op + 4 * u) =
-                    make_float4(acc[4 * u] * il, acc[4 * u + 1] * il, acc[4 * u + 2] * il, acc[4 * u + 3] * il);
+                for (int e = 0; e < CPL; ++e) op[e] = acc[e] * il;
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
         }
         if (i0 + kWinQ < F) __syncthreads();  // the block's LDS rows are read before the next block restages them
     }

@@ -359,3 +359,38 @@ def test_convolution_tiles_keep_to_their_stream(nq, device, channels, streams):
     torch.cuda.synchronize()
     assert torch.equal(got.cpu(), want1)
     assert torch.equal(hist.cpu(), want_hist)
+
+
+@pytest.mark.parametrize("frames", [1, 7, 8, 9, 71, 72, 73])
+@pytest.mark.parametrize("D", [16, 32, 64])
+def test_window_attention_of_few_queries(nq, device, D, frames):
+    """Blocks of up to eight queries take one thread per (query, window step), longer ones one lane per query:
+    chunks around that line (and whose last block lies around it), with five of the retained rows valid and the
+    others infinite or NaN, within 1e-4 of the oracle: an angle below 128 rounds at 2^-18, which moves a score of
+    at most |q| |k| / sqrt(D) = 8 by at most 2 * 8 * 2^-18 = 6e-5, and outputs of unit size by as much."""
+    from nari_qwen3_tts_amd import _lib
+
+    H, window, ctx, pos0 = 3, 32, 5, 40
+    R, HD = window - 1, H * D
+    g = torch.Generator().manual_seed(D + frames)
+    qkv = torch.randn(frames, 3 * HD, generator=g)
+    norm = torch.ones(D)
+    sk, sv = torch.randn(1, R, H, D, generator=g), torch.randn(1, R, H, D, generator=g)
+    state_k, state_v = sk.clone(), sv.clone()
+    state_k[:, : R - ctx], state_v[:, : R - ctx] = float("nan"), float("inf")
+    d_qkv, d_norm, d_sk, d_sv = (t.to(device) for t in (qkv, norm, state_k, state_v))
+    d_off, d_slots = (torch.tensor(v, dtype=torch.int32, device=device) for v in ([0, frames], [0]))
+    d_pos, d_ctx = (torch.tensor([v], dtype=dt, device=device) for v, dt in ((pos0, torch.int64), (ctx, torch.int32)))
+    out = torch.full((frames, HD), float("nan"), device=device)
+    q, k, v = d_qkv[:, :HD], d_qkv[:, HD : 2 * HD], d_qkv[:, 2 * HD :]
+    _lib.call("nq_codec_window_attention", q.data_ptr(), k.data_ptr(), v.data_ptr(), d_qkv.stride(0), frames, H, D,
+              d_norm.data_ptr(), d_norm.data_ptr(), 1e-6, 10000.0, d_off.data_ptr(), 1, d_slots.data_ptr(),
+              d_pos.data_ptr(), d_ctx.data_ptr(), d_sk.data_ptr(), d_sv.data_ptr(), d_sk.stride(0), R, window,
+              out.data_ptr(), out.stride(0), _lib.stream(device))
+    torch.cuda.synchronize()
+    rows = qkv.numpy().reshape(frames, 3, H, D)
+    pos = pos0 + np.arange(frames)
+    qr, kr = (o_codec.rope(o_codec.rmsnorm(rows[:, i], norm.numpy(), 1e-6), pos, 10000.0) for i in (0, 1))
+    want = o_codec.window_attention(qr, np.concatenate([sk[0].numpy(), kr]),
+                                    np.concatenate([sv[0].numpy(), rows[:, 2]]), pos0, ctx, window)
+    np.testing.assert_allclose(out.cpu().numpy().reshape(frames, H, D), want, atol=1e-4, rtol=1e-4)
