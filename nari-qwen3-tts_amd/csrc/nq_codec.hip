@@ -619,9 +619,14 @@ transconv_kernel(const float *__restrict__ x, int64_t ldx, int64_t T_out, const 
 // Narrow causal transposed Conv1d (Cout <= 16, stride s): output row r reads input
 // rows r / s and r / s - 1 (the stream's rows are aligned to s at this stage).
 // The workgroup stages the (at most 256 / s + 3) input rows its 256 output rows read,
-// activated once, in LDS (row pitch Cin + 1) with the weights as [ci][co][2s];
+// activated once, in LDS (row pitch Cin + 1) with the weights as [ci][2s][co];
 // the first output rows of a stream add its carried overlap instead of an
 // earlier input row.  Outputs move as float4 when the row stride allows it.
+// With one or a few streams the staging is the time, so its loads are in
+// flight together; with many the weights' LDS reads, so they lie with the
+// output channels together and are read four at a time: 32 -> 16 channels, s =
+// 4: 1600 rows 28 -> 15 us, 363,000 rows 48.7 -> 31.6; 16 -> 8, s = 5: 8000
+// rows 10.3 -> 7.5, 1.8 M rows 57 -> 45.
 template <int CO>
 __global__ void __launch_bounds__(kCodecThreads)
 transconv_small_kernel(const float *__restrict__ x, int64_t ldx, int64_t T_out, const int32_t *__restrict__ off,
@@ -633,7 +638,7 @@ transconv_small_kernel(const float *__restrict__ x, int64_t ldx, int64_t T_out, 
     const int pitch = Cin + 1;
     const int n_max = kCodecThreads / s + 3;  // >= the staged rows for every stride
     float *xs = lds;                                    // [n_max * pitch]
-    float *tw = xs + (n_max * pitch + 3) / 4 * 4;       // [Cin][CO][2s]
+    float *tw = xs + (n_max * pitch + 3) / 4 * 4;       // [Cin][2s][CO], 16-byte aligned
     float *sa = tw + Cin * CO * ks;                     // [Cin]
     float *sb = sa + Cin;                               // [Cin]
     const int64_t T_in = T_out / s;
@@ -641,26 +646,59 @@ transconv_small_kernel(const float *__restrict__ x, int64_t ldx, int64_t T_out, 
     const int64_t last = row0 + kCodecThreads - 1 < T_out ? row0 + kCodecThreads - 1 : T_out - 1;
     const int64_t in0 = row0 / s - 1;  // staged input row 0 (may be -1)
     const int n_in = static_cast<int>(last / s - in0 + 1);
-    for (int e = threadIdx.x; e < Cin * CO * ks; e += kCodecThreads) {
-        const int ci = e / (CO * ks);
-        const int rem = e - ci * CO * ks;
-        const int co = rem / ks, k = rem - co * ks;
-        tw[e] = co < Cout ? w[(static_cast<int64_t>(ci) * Cout + co) * ks + k] : 0.f;
+    // eight weights, and four 128-bit pieces of the rows, requested before the first is stored
+    const int nw = Cin * Cout * ks;
+    for (int e0 = threadIdx.x; e0 < nw; e0 += 8 * kCodecThreads) {
+        float v[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] = w[e0 + i * kCodecThreads < nw ? e0 + i * kCodecThreads : nw - 1];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const int e = e0 + i * kCodecThreads;
+            if (e >= nw) break;
+            const int cc = e / ks, k = e - cc * ks;
+            const int ci = Cout == CO ? cc / CO : cc / Cout;
+            tw[(ci * ks + k) * CO + cc - ci * Cout] = v[i];
+        }
     }
     if (act.alpha && threadIdx.x < Cin) {
         sa[threadIdx.x] = act.a_of(threadIdx.x);
         sb[threadIdx.x] = act.inv_b_of(threadIdx.x);
     }
     __syncthreads();
-    for (int e = threadIdx.x; e < n_in * Cin; e += kCodecThreads) {
-        const int rr = e / Cin, c = e - rr * Cin;
-        const int64_t g = in0 + rr;
-        float v = 0.f;
-        if (g >= 0 && g < T_in) {
-            v = x[g * ldx + c];
-            if (act.alpha) v = snake(v, sa[c], sb[c]);
+    if ((Cin & 3) == 0 && (ldx & 3) == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0) {
+        const int vpr = Cin / 4, nvec = n_in * vpr;
+        for (int e0 = threadIdx.x; e0 < nvec; e0 += 4 * kCodecThreads) {
+            float4 v[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int e = e0 + i * kCodecThreads < nvec ? e0 + i * kCodecThreads : nvec - 1;
+                const int rr = e / vpr;
+                const int64_t g = in0 + rr < 0 ? 0 : in0 + rr < T_in ? in0 + rr : T_in - 1;
+                v[i] = *reinterpret_cast<const float4 *>(x + g * ldx + (e - rr * vpr) * 4);
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int e = e0 + i * kCodecThreads;
+                if (e >= nvec) break;
+                const int rr = e / vpr, c = (e - rr * vpr) * 4;
+                const float f[4] = {v[i].x, v[i].y, v[i].z, v[i].w};
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    xs[rr * pitch + c + q] = act.alpha ? snake(f[q], sa[c + q], sb[c + q]) : f[q];
+            }
         }
-        xs[rr * pitch + c] = v;
+    } else {
+        for (int e = threadIdx.x; e < n_in * Cin; e += kCodecThreads) {
+            const int rr = e / Cin, c = e - rr * Cin;
+            const int64_t g = in0 + rr;
+            float v = 0.f;
+            if (g >= 0 && g < T_in) {
+                v = x[g * ldx + c];
+                if (act.alpha) v = snake(v, sa[c], sb[c]);
+            }
+            xs[rr * pitch + c] = v;
+        }
     }
     __syncthreads();
     const int64_t row = row0 + threadIdx.x;
@@ -677,9 +715,16 @@ transconv_small_kernel(const float *__restrict__ x, int64_t ldx, int64_t T_out, 
     for (int q = 0; q < CO; ++q) acc[q] = 0.f;
     for (int ci = 0; ci < Cin; ++ci) {
         const float a1 = x1[ci], a0 = first ? 0.f : x0[ci];
-        const float *wr = tw + ci * CO * ks;
+        const float4 *w1 = reinterpret_cast<const float4 *>(tw + (ci * ks + j) * CO);
+        const float4 *w0 = w1 + s * (CO / 4);
 #pragma unroll
-        for (int q = 0; q < CO; ++q) acc[q] += a1 * wr[q * ks + j] + a0 * wr[q * ks + j + s];
+        for (int q = 0; q < CO / 4; ++q) {
+            const float4 u1 = w1[q], u0 = w0[q];
+            acc[4 * q] += a1 * u1.x + a0 * u0.x;
+            acc[4 * q + 1] += a1 * u1.y + a0 * u0.y;
+            acc[4 * q + 2] += a1 * u1.z + a0 * u0.z;
+            acc[4 * q + 3] += a1 * u1.w + a0 * u0.w;
+        }
     }
     const float *ov = overlap + (static_cast<int64_t>(slots[b]) * s + j) * Cout;
     float y[CO];

@@ -394,3 +394,34 @@ def test_window_attention_of_few_queries(nq, device, D, frames):
     want = o_codec.window_attention(qr, np.concatenate([sk[0].numpy(), kr]),
                                     np.concatenate([sv[0].numpy(), rows[:, 2]]), pos0, ctx, window)
     np.testing.assert_allclose(out.cpu().numpy().reshape(frames, H, D), want, atol=1e-4, rtol=1e-4)
+
+
+@pytest.mark.parametrize("cin,cout,stride", [(32, 16, 4), (16, 8, 5), (12, 5, 3), (7, 16, 2), (16, 1, 1)])
+def test_narrow_transposed_convolution(nq, device, cin, cout, stride):
+    """nq_codec_causal_transconv with at most 16 output channels (whole and partial channel groups, rows with and
+    without 128-bit pieces, several workgroups): integer operands, exact in fp32, against each stream's own transposed
+    convolution on the host, with the overlap it carries in and out."""
+    from nari_qwen3_tts_amd import _lib
+
+    rows = [1, 3, 0, 64, 200, 65]
+    B, T = len(rows), sum(rows)
+    g = torch.Generator().manual_seed(cin + cout)
+    r = lambda *shape, lim=3: torch.randint(-lim, lim + 1, shape, generator=g).float()  # noqa: E731
+    x, w, bias, overlap0 = r(T, cin), r(cin, cout, 2 * stride), r(cout), r(B + 1, stride, cout)
+    slots = torch.randperm(B + 1, generator=g)[:B].int()
+    off = torch.tensor(np.concatenate([[0], np.cumsum(rows)]), dtype=torch.int32)
+    want, want_overlap = [], overlap0.clone()
+    for b in range(B):
+        if rows[b]:
+            y = torch.nn.functional.conv_transpose1d(x[off[b] : off[b + 1]].t()[None], w, stride=stride)[0].t().clone()
+            y[:stride] += overlap0[slots[b]]
+            want.append(y[: rows[b] * stride] + bias)
+            want_overlap[slots[b]] = y[rows[b] * stride :]
+    d = {n: t.to(device) for n, t in dict(x=x, w=w, bias=bias, off=off, slots=slots, overlap=overlap0).items()}
+    got = torch.full((T * stride, cout), float("nan"), device=device)
+    _lib.call("nq_codec_causal_transconv", d["x"].data_ptr(), cin, T, d["off"].data_ptr(), B, 1, stride,
+              d["slots"].data_ptr(), d["overlap"].data_ptr(), d["w"].data_ptr(), d["bias"].data_ptr(), cin, cout, None,
+              None, got.data_ptr(), cout, _lib.stream(device))
+    torch.cuda.synchronize()
+    assert torch.equal(got.cpu(), torch.cat(want))
+    assert torch.equal(d["overlap"].cpu(), want_overlap)
