@@ -241,6 +241,24 @@ int nq_cp_rope_short_attention(const float *partials, int splits, int rows, cons
                                int64_t o_s0, int64_t o_s1, void *stream);
 
 /*
+ * The same attention with the projection of its output behind it, for a few
+ * rows (at most 8): planes [S][rows][N] receives att . W^T as S =
+ * nq_cp_rope_short_linear_splits fp32 planes, one per pair of kv heads, and
+ * the caches the new position; the rotated q and the attention go nowhere
+ * else.  Two query heads of 64 per kv head, 2, 4, 6 or 8 kv heads, N % 128 == 0
+ * and cache_position < 16, else -1 / NQ_ERR_UNSUPPORTED.  The planes hold the bits of
+ * nq_cp_rope_short_attention and then nq_decode_linear where that cuts K into
+ * the same slices.  planes may not overlap partials.
+ */
+int nq_cp_rope_short_linear_splits(int rows, int num_qo_heads, int num_kv_heads, int head_dim, int N);
+int nq_cp_rope_short_linear(const float *partials, int splits, int rows, const uint16_t *q_weight,
+                            const uint16_t *k_weight, const int64_t *positions, int64_t pos_stride, float eps,
+                            float rope_theta, int round_to_input, uint16_t *cache, int64_t c_row, int64_t c_kind,
+                            int64_t c_pos, int64_t c_head, int cache_position, int num_qo_heads, int num_kv_heads,
+                            int head_dim, float sm_scale, const uint16_t *w, int64_t w_s0, int N, float *planes,
+                            int64_t planes_bytes, void *stream);
+
+/*
  * Fused per-head RMSNorm + rotate-half RoPE of q and k (in place), with K and
  * V written into the cache.
  * Replaces paired_qk_norm_rope_paged_cache_ (model/kernels.py:15-160) and,

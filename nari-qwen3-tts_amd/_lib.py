@@ -90,6 +90,9 @@ _SIGNATURES: dict[str, list] = {
     "nq_fp8_pack_swiglu": [_P, _L, _I, _I, _P, _L, _P],
     "nq_linear_swiglu": [_P, _L, _I, _P, _L, _I, _I, _P, _L, _P],
     "nq_linear_fp8_swiglu": [_P, _L, _P, _L, _I, _P, _L, _P, _L, _I, _I, _P, _L, _P],
+    "nq_cp_rope_short_linear_splits": [_I, _I, _I, _I, _I],
+    "nq_cp_rope_short_linear": [_P, _I, _I, _P, _P, _P, _L, _F, _F, _I, _P, _L, _L, _L, _L, _I, _I, _I, _I, _F, _P, _L,
+                                _I, _P, _L, _P],
     "nq_decode_linear_splits": [_I, _I, _I],
     "nq_decode_linear": [_P, _L, _P, _L, _I, _I, _I, _P, _L, _P],
     "nq_decode_norm_linear": [_P, _I, _P, _P, _P, _F, _P, _P, _L, _I, _I, _I, _P, _L, _P],

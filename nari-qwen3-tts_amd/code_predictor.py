@@ -39,7 +39,11 @@ import torch
 import torch.nn.functional as F
 
 from . import _lib
-from .kernels import qkv_partials_rope_short_attention_
+from .kernels import (
+    qkv_partials_rope_short_attention_,
+    qkv_partials_rope_short_linear_,
+    rope_short_linear_splits,
+)
 from .layers import (
     NormRows,
     decode_linear,
@@ -234,13 +238,14 @@ class CodePredictorFrame:
         need = max(linear_workspace_bytes(rows, n, k, e) for n, k, e in shapes)
         # few rows: projections that normalise their rows themselves, over two alternating plane
         # regions and two residual buffers (a kernel reads one of each and writes the other)
-        few = ((c.qkv_width, c.hidden), (c.hidden, c.num_qo_heads * c.head_dim), (c.hidden, c.intermediate),
-               (c.vocab, c.hidden))
+        few = ((c.qkv_width, c.hidden), (c.hidden, c.intermediate), (c.vocab, c.hidden))
+        o_splits = rope_short_linear_splits(rows, c.num_qo_heads, c.num_kv_heads, c.head_dim, c.hidden)
         self.few = rows <= self.FEW_ROWS and c.hidden == 1024 and c.intermediate % 16 == 0 and all(
-            decode_linear_splits(rows, n, k) > 0 for n, k in few)
+            decode_linear_splits(rows, n, k) > 0 for n, k in few) and o_splits > 0
         if self.few:
             self.h2 = torch.zeros(rows, c.hidden, **bf)
-            self._region = max(decode_linear_splits(rows, n, k) * rows * n * 4 for n, k in few)
+            self._region = max([decode_linear_splits(rows, n, k) * rows * n * 4 for n, k in few]
+                               + [o_splits * rows * c.hidden * 4])
             need = max(need, 2 * self._region)
         self.workspace = torch.empty(max(need, 16), dtype=torch.uint8, device=dev)
         # optional [groups, layers + 2, rows, hidden] bf16 record of each pass: the residual stream
@@ -256,11 +261,11 @@ class CodePredictorFrame:
     FEW_ROWS = 8
 
     def _layers_few(self, cache_pos: int):
-        """The layers from self.h and its first input norm self.x with five launches each: QKV, attention,
-        o, gate/up + SwiGLU, down, the add-RMSNorms inside the projections after them.  Returns the final
-        norm's rows, for the head."""
+        """The layers from self.h and its first input norm self.x with four launches each: QKV, attention
+        and o, gate/up + SwiGLU, down, the add-RMSNorms inside the projections after them.  Returns the
+        final norm's rows, for the head."""
 
-        c, n = self.w.config, self.rows
+        c = self.w.config
         a, b = self.workspace[: self._region], self.workspace[self._region: 2 * self._region]
         h, h2 = self.h, self.h2
         positions = self.position_ids[:, cache_pos]
@@ -269,9 +274,8 @@ class CodePredictorFrame:
             if index:
                 splits = decode_norm_linear(NormRows(a, down, h2, h, L.input_norm, c.rms_eps), L.qkv, b)
             cache = self.kv_cache[index]
-            qkv_partials_rope_short_attention_(b, splits, self.q, L.q_norm, L.k_norm, positions, c.rms_eps,
-                                               c.rope_theta, cache[:, 0], cache[:, 1], cache_pos, self.att)
-            splits = decode_linear(self.att.view(n, -1), L.o, a)
+            splits = qkv_partials_rope_short_linear_(b, splits, L.q_norm, L.k_norm, positions, c.rms_eps, c.rope_theta,
+                                                     cache[:, 0], cache[:, 1], cache_pos, L.o, a)
             decode_norm_swiglu(NormRows(a, splits, h, h2, L.post_norm, c.rms_eps), L.gate_up_packed, self.act)
             down = decode_linear(self.act, L.down, a)
         return NormRows(a, down, h2, h, self.w.final_norm, c.rms_eps, self.x)

@@ -1849,6 +1849,12 @@ dense_short_kernel(const uint16_t *__restrict__ q, int64_t q_s0, int64_t q_s1,
 
 constexpr int kShortLen = 16;
 
+// LDS written by one lane of a wave, read by another: a wave's LDS accesses complete in order
+__device__ __forceinline__ void short_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 template <int D, int G>
 struct ShortSmem {
     __attribute__((aligned(16))) uint16_t q[G][D];
@@ -1887,7 +1893,7 @@ __device__ __forceinline__ void short_attend(ShortSmem<D, G> &sm, const uint4 (&
         dot = group_sum<4>(dot);
         if ((lane & 3) == 0) sm.s[j][lane >> 2] = (lane >> 2) < len ? dot * scale_log2 : -INFINITY;
     }
-    __syncthreads();
+    short_sync();
     constexpr int HALF = D / 2;
     for (int t = lane; t < G * HALF; t += kWave) {
         const int j = t / HALF, d = (t % HALF) * 2;
@@ -1945,7 +1951,7 @@ short_kernel(const uint16_t *__restrict__ q, int64_t q_s0, int64_t q_s1, const u
             *reinterpret_cast<const uint4 *>(q + row * q_s0 + (h * G + j) * q_s1 + d);
     }
     short_stage_v(sm, vr, -1, lane);
-    __syncthreads();
+    short_sync();
     short_attend(sm, kr, valid_length, lane, scale_log2, out + row * o_s0 + h * G * o_s1, o_s1);
 }
 
@@ -1954,26 +1960,36 @@ short_kernel(const uint16_t *__restrict__ q, int64_t q_s0, int64_t q_s1, const u
 // arithmetic of nq_qkv_partials_norm_rope_kv_write, so the same bits in q_out
 // and the cache).  A unit is a query head, the key head or the value head; a
 // wave takes 128 / D of them at a time, a lane the pair (i, i + D / 2).
-template <int D, int G>
-__global__ void __launch_bounds__(kWave)
-rope_short_kernel(const float *__restrict__ partials, int splits, int64_t plane, int64_t prow,
-                  const uint16_t *__restrict__ q_weight, const uint16_t *__restrict__ k_weight,
-                  const int64_t *__restrict__ positions, int64_t pos_stride, float eps, float log_theta,
-                  int round_to_input, uint16_t *__restrict__ q_out, int64_t q_s0, int64_t q_s1,
-                  uint16_t *__restrict__ cache, int64_t c_row, int64_t c_kind, int64_t c_pos, int64_t c_head,
-                  int cache_position, int num_kv_heads, float scale_log2, uint16_t *__restrict__ out, int64_t o_s0,
-                  int64_t o_s1) {
+struct ShortRope {
+    const float *partials;  // [splits][rows][prow]
+    int splits;
+    int64_t plane, prow;
+    const uint16_t *q_weight, *k_weight;
+    const int64_t *positions;
+    int64_t pos_stride;
+    float eps, log_theta;
+    int round_to_input;
+    uint16_t *q_out;  // or null
+    int64_t q_s0, q_s1;
+    uint16_t *cache;
+    int64_t c_row, c_kind, c_pos, c_head;
+    int cache_position, num_kv_heads;
+    float scale_log2;
+};
+
+// One wave: row `row`, kv head `h`; `write`: q_out (where given) and the cache's new position are written.
+// `after` issues loads of the caller's behind these, which return first.
+template <int D, int G, typename After>
+__device__ __forceinline__ void rope_short_row(const ShortRope &s_, ShortSmem<D, G> &sm, int row, int h, int lane,
+                                               bool write, uint16_t *__restrict__ out, int64_t o_s1, After after) {
     constexpr int HALF = D / 2;
     constexpr int kAtOnce = kWave / HALF;
     constexpr int kRounds = (G + 2 + kAtOnce - 1) / kAtOnce;
-    __shared__ ShortSmem<D, G> sm;
-    const int lane = threadIdx.x;
-    const int row = blockIdx.x / num_kv_heads;
-    const int h = blockIdx.x - row * num_kv_heads;
-    const int Hq = num_kv_heads * G;
+    const int Hq = s_.num_kv_heads * G;
     const int pair = lane % HALF;
-    uint16_t *base = cache + row * c_row + h * c_head;
-    uint16_t *slot = base + cache_position * c_pos;
+    const int cache_position = s_.cache_position;
+    uint16_t *base = s_.cache + row * s_.c_row + h * s_.c_head;
+    uint16_t *slot = base + cache_position * s_.c_pos;
 
     // the planes four at a time (all loads in flight together)
     float x[kRounds][2];
@@ -1983,29 +1999,33 @@ rope_short_kernel(const float *__restrict__ partials, int splits, int64_t plane,
 #pragma unroll
     for (int r = 0; r < kRounds; ++r) {
         const int u = r * kAtOnce + lane / HALF;
-        const int head = u < G ? h * G + u : u == G ? Hq + h : Hq + num_kv_heads + h;
-        src[r] = partials + row * prow + static_cast<int64_t>(u < G + 2 ? head : h) * D + pair;
+        const int head = u < G ? h * G + u : u == G ? Hq + h : Hq + s_.num_kv_heads + h;
+        src[r] = s_.partials + row * s_.prow + static_cast<int64_t>(u < G + 2 ? head : h) * D + pair;
     }
     uint4 kr[D / 32], vr[D / 32];
-    const float position = static_cast<float>(positions[row * pos_stride]);
-    for (int i0 = 0; i0 < splits; i0 += 4) {
+    const float position = static_cast<float>(s_.positions[row * s_.pos_stride]);
+    const float qw1 = bf16_to_f32(s_.q_weight[pair]), qw2 = bf16_to_f32(s_.q_weight[pair + HALF]);
+    const float kw1 = bf16_to_f32(s_.k_weight[pair]), kw2 = bf16_to_f32(s_.k_weight[pair + HALF]);
+    for (int i0 = 0; i0 < s_.splits; i0 += 4) {
         float a[kRounds][4][2];
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-            if (i0 + v >= splits) break;
+            if (i0 + v >= s_.splits) break;
 #pragma unroll
             for (int r = 0; r < kRounds; ++r) {
-                a[r][v][0] = src[r][(i0 + v) * plane];
-                a[r][v][1] = src[r][(i0 + v) * plane + HALF];
+                a[r][v][0] = src[r][(i0 + v) * s_.plane];
+                a[r][v][1] = src[r][(i0 + v) * s_.plane + HALF];
             }
         }
         if (i0 == 0) {  // behind the first planes' loads, ahead of the wait for them
-            short_load<D>(base, c_pos, cache_position, lane, kr);
-            short_load<D>(base + c_kind, c_pos, cache_position, lane, vr);
+            short_load<D>(base, s_.c_pos, cache_position, lane, kr);
+            short_load<D>(base + s_.c_kind, s_.c_pos, cache_position, lane, vr);
+            after();
+            __builtin_amdgcn_sched_barrier(0);
         }
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-            if (i0 + v >= splits) break;
+            if (i0 + v >= s_.splits) break;
 #pragma unroll
             for (int r = 0; r < kRounds; ++r) {
                 x[r][0] += a[r][v][0];
@@ -2013,35 +2033,119 @@ rope_short_kernel(const float *__restrict__ partials, int splits, int64_t plane,
             }
         }
     }
-    const float qw1 = bf16_to_f32(q_weight[pair]), qw2 = bf16_to_f32(q_weight[pair + HALF]);
-    const float kw1 = bf16_to_f32(k_weight[pair]), kw2 = bf16_to_f32(k_weight[pair + HALF]);
 #pragma unroll
     for (int r = 0; r < kRounds; ++r) {
         const int u = r * kAtOnce + lane / HALF;
         const float x1 = bf16_to_f32(f32_to_bf16(x[r][0])), x2 = bf16_to_f32(f32_to_bf16(x[r][1]));
         uint16_t o1, o2;
-        norm_rope_pair<D>(x1, x2, true, u < G ? qw1 : kw1, u < G ? qw2 : kw2, pair, eps, log_theta, position,
-                          round_to_input, o1, o2);
+        norm_rope_pair<D>(x1, x2, true, u < G ? qw1 : kw1, u < G ? qw2 : kw2, pair, s_.eps, s_.log_theta, position,
+                          s_.round_to_input, o1, o2);
         if (u < G) {
-            uint16_t *dst = q_out + row * q_s0 + (h * G + u) * q_s1;
-            dst[pair] = sm.q[u][pair] = o1;
-            dst[pair + HALF] = sm.q[u][pair + HALF] = o2;
+            sm.q[u][pair] = o1;
+            sm.q[u][pair + HALF] = o2;
+            if (write && s_.q_out) {
+                uint16_t *dst = s_.q_out + row * s_.q_s0 + (h * G + u) * s_.q_s1;
+                dst[pair] = o1;
+                dst[pair + HALF] = o2;
+            }
         } else if (u == G) {
-            slot[pair] = sm.k[pair] = o1;
-            slot[pair + HALF] = sm.k[pair + HALF] = o2;
+            sm.k[pair] = o1;
+            sm.k[pair + HALF] = o2;
+            if (write) {
+                slot[pair] = o1;
+                slot[pair + HALF] = o2;
+            }
         } else if (u == G + 1) {
-            slot[c_kind + pair] = sm.v[cache_position][pair] = f32_to_bf16(x1);
-            slot[c_kind + pair + HALF] = sm.v[cache_position][pair + HALF] = f32_to_bf16(x2);
+            const uint16_t v1 = f32_to_bf16(x1), v2 = f32_to_bf16(x2);
+            sm.v[cache_position][pair] = v1;
+            sm.v[cache_position][pair + HALF] = v2;
+            if (write) {
+                slot[s_.c_kind + pair] = v1;
+                slot[s_.c_kind + pair + HALF] = v2;
+            }
         }
     }
     short_stage_v(sm, vr, cache_position, lane);
-    __syncthreads();
+    short_sync();
     if ((lane >> 2) == cache_position) {
 #pragma unroll
         for (int i = 0; i < D / 32; ++i)
             kr[i] = *reinterpret_cast<const uint4 *>(&sm.k[(lane & 3) * (D / 4) + i * 8]);
     }
-    short_attend(sm, kr, cache_position + 1, lane, scale_log2, out + row * o_s0 + h * G * o_s1, o_s1);
+    short_attend(sm, kr, cache_position + 1, lane, s_.scale_log2, out, o_s1);
+}
+
+template <int D, int G>
+__global__ void __launch_bounds__(kWave)
+rope_short_kernel(ShortRope src, uint16_t *__restrict__ out, int64_t o_s0, int64_t o_s1) {
+    __shared__ ShortSmem<D, G> sm;
+    const int row = blockIdx.x / src.num_kv_heads, h = blockIdx.x - row * src.num_kv_heads;
+    rope_short_row<D, G>(src, sm, row, h, threadIdx.x, true, out + row * o_s0 + h * G * o_s1, o_s1, [] {});
+}
+
+// The same and the projection of the attention's output behind it, for a few
+// rows: workgroup (128 output columns, kv head pair) attends for its two heads
+// of every row, a wave each (row, head) and again in every column block, and
+// multiplies what it holds in LDS with the 16 columns of weights each wave asked
+// for behind its attention's loads (ahead of them they were waited for first:
+// loads return in order), which have arrived by then.  The pair's 2 G D columns are one
+// K slice: S = num_kv_heads / 2 fp32 planes [S, rows, N], with the bits of
+// nq_decode_linear's where it cuts K alike (32-k products added in order).  The
+// first column block writes the new K and V; all take them from LDS.
+// One row, kernel trace: 6.5 us where the two launches took 4.2 and 2.9 and the
+// gap between them; a one-row code predictor frame 1721 -> 1608 us.
+typedef __bf16 so_bf16x8 __attribute__((ext_vector_type(8)));
+typedef float so_floatx4 __attribute__((ext_vector_type(4)));
+
+constexpr int kShortOWaves = 8;
+constexpr int kShortORows = 8;
+
+template <int D, int G>
+__global__ void __launch_bounds__(kShortOWaves * kWave)
+rope_short_linear_kernel(ShortRope src, int rows, const uint16_t *__restrict__ w, int64_t w_s0, int N,
+                         float *__restrict__ part) {
+    constexpr int KS = 2 * G * D;       // the slice
+    constexpr int XP = KS + 8;          // LDS row pitch
+    __shared__ ShortSmem<D, G> sm[kShortOWaves];
+    __shared__ __attribute__((aligned(16))) uint16_t xs[kShortORows * XP];
+    const int lane = threadIdx.x & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int r16 = lane & 15, kq = lane >> 4;
+    const int col0 = (blockIdx.x * kShortOWaves + wave) * 16, k0 = blockIdx.y * KS;
+    uint4 wr[KS / 32];
+    const uint16_t *wp = w + static_cast<int64_t>(col0 + r16) * w_s0 + k0 + kq * 8;
+    auto load_weights = [&] {
+#pragma unroll
+        for (int i = 0; i < KS / 32; ++i) wr[i] = *reinterpret_cast<const uint4 *>(wp + i * 32);
+    };
+    auto attend = [&](int t, auto after) {
+        const int row = t >> 1, half = t & 1;
+        rope_short_row<D, G>(src, sm[wave], row, blockIdx.y * 2 + half, lane, blockIdx.x == 0,
+                             xs + row * XP + half * G * D, D, after);
+    };
+    if (wave < 2 * rows)
+        attend(wave, load_weights);
+    else
+        load_weights();
+    for (int t = wave + kShortOWaves; t < 2 * rows; t += kShortOWaves) {
+        short_sync();
+        attend(t, [] {});
+    }
+    __syncthreads();
+    const uint16_t *xp = xs + (r16 < rows ? r16 : 0) * XP + kq * 8;  // rows past the last repeat the first; not stored
+    float sum[4];
+#pragma unroll
+    for (int i = 0; i < KS / 32; ++i) {
+        so_floatx4 d = {0.f, 0.f, 0.f, 0.f};
+        d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(so_bf16x8, wr[i]),
+                                                    __builtin_bit_cast(so_bf16x8, *reinterpret_cast<const uint4 *>(xp + i * 32)),
+                                                    d, 0, 0, 0);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sum[e] = i ? sum[e] + d[e] : d[e];
+    }
+    if (r16 < rows)
+        *reinterpret_cast<float4 *>(part + (static_cast<int64_t>(blockIdx.y) * rows + r16) * N + col0 + kq * 4) =
+            make_float4(sum[0], sum[1], sum[2], sum[3]);
 }
 
 // Code-predictor layer attention with the q/k norm + RoPE + K/V write fused
@@ -2693,10 +2797,11 @@ int launch_dense_rope(const float *partials, int splits, int rows, const uint16_
     const int64_t prow = static_cast<int64_t>(Hkv * G + 2 * Hkv) * D;
     const int64_t items = static_cast<int64_t>(rows) * Hkv;
     if (cache_position < kShortLen && items <= 0x7fffffff && (o_s0 % 2 | o_s1 % 2) == 0) {
-        hipLaunchKernelGGL((rope_short_kernel<D, G>), dim3(static_cast<unsigned>(items)), dim3(kWave), 0, stream,
-                           partials, splits, static_cast<int64_t>(rows) * prow, prow, q_weight, k_weight, positions,
-                           pos_stride, eps, logf(rope_theta), round_to_input, q_out, q_s0, q_s1, cache, c_row, c_kind,
-                           c_pos, c_head, cache_position, Hkv, scale * kLog2e, out, o_s0, o_s1);
+        const ShortRope src{partials, splits, static_cast<int64_t>(rows) * prow, prow, q_weight, k_weight, positions,
+                            pos_stride, eps, logf(rope_theta), round_to_input, q_out, q_s0, q_s1, cache, c_row, c_kind,
+                            c_pos, c_head, cache_position, Hkv, scale * kLog2e};
+        hipLaunchKernelGGL((rope_short_kernel<D, G>), dim3(static_cast<unsigned>(items)), dim3(kWave), 0, stream, src,
+                           out, o_s0, o_s1);
         return NQ_LAUNCH_STATUS();
     }
     const int grid = static_cast<int>(items < 8192 ? items : 8192);
@@ -2845,6 +2950,38 @@ extern "C" int nq_cp_rope_short_attention(const float *partials, int splits, int
     NQ_DENSE_ROPE(128, 1) NQ_DENSE_ROPE(128, 2) NQ_DENSE_ROPE(64, 1) NQ_DENSE_ROPE(64, 2)
 #undef NQ_DENSE_ROPE
     return NQ_ERR_UNSUPPORTED;
+}
+
+extern "C" int nq_cp_rope_short_linear_splits(int rows, int num_qo_heads, int num_kv_heads, int head_dim, int N) {
+    const bool takes = rows >= 1 && rows <= nq::kShortORows && head_dim == 64 && num_kv_heads >= 2 &&
+                       num_kv_heads <= 8 && num_kv_heads % 2 == 0 && num_qo_heads == 2 * num_kv_heads && N > 0 &&
+                       N % (16 * nq::kShortOWaves) == 0;
+    return takes ? num_kv_heads / 2 : -1;
+}
+
+extern "C" int nq_cp_rope_short_linear(const float *partials, int splits, int rows, const uint16_t *q_weight,
+                                       const uint16_t *k_weight, const int64_t *positions, int64_t pos_stride,
+                                       float eps, float rope_theta, int round_to_input, uint16_t *cache, int64_t c_row,
+                                       int64_t c_kind, int64_t c_pos, int64_t c_head, int cache_position,
+                                       int num_qo_heads, int num_kv_heads, int head_dim, float sm_scale,
+                                       const uint16_t *w, int64_t w_s0, int N, float *planes, int64_t planes_bytes,
+                                       void *stream) {
+    NQ_CHECK_ARG(partials && splits >= 1 && q_weight && k_weight && positions && cache && w && planes);
+    NQ_CHECK_ARG(rows >= 1 && cache_position >= 0 && rope_theta > 0.f && num_kv_heads >= 1);
+    const int S = nq_cp_rope_short_linear_splits(rows, num_qo_heads, num_kv_heads, head_dim, N);
+    if (S < 0 || cache_position >= nq::kShortLen) return NQ_ERR_UNSUPPORTED;
+    if (!nq::aligned16(cache) || ((c_row | c_kind | c_pos | c_head) & 7)) return NQ_ERR_UNSUPPORTED;
+    NQ_CHECK_ARG(w_s0 >= num_qo_heads * head_dim && w_s0 % 8 == 0 && nq::aligned16(w) && nq::aligned16(planes));
+    NQ_CHECK_ARG(planes_bytes >= static_cast<int64_t>(S) * rows * N * 4);
+    const int64_t prow = static_cast<int64_t>(num_qo_heads + 2 * num_kv_heads) * head_dim;
+    const nq::ShortRope src{partials, splits, static_cast<int64_t>(rows) * prow, prow, q_weight, k_weight, positions,
+                            pos_stride, eps, logf(rope_theta), round_to_input, nullptr, 0, 0, cache, c_row, c_kind,
+                            c_pos, c_head, cache_position, num_kv_heads, sm_scale * nq::kLog2e};
+    hipLaunchKernelGGL((nq::rope_short_linear_kernel<64, 2>),
+                       dim3(static_cast<unsigned>(N / (16 * nq::kShortOWaves)), static_cast<unsigned>(S)),
+                       dim3(nq::kShortOWaves * nq::kWave), 0, static_cast<hipStream_t>(stream), src, rows, w, w_s0, N,
+                       planes);
+    return NQ_LAUNCH_STATUS();
 }
 
 extern "C" int nq_paged_decode_rope_attention(const float *partials, int splits, int tokens, const uint16_t *q_weight,

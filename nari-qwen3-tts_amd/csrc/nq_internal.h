@@ -82,14 +82,16 @@ __device__ __forceinline__ float row_group_scale(float amax) { return amax > 0.f
 // norm weights (w1, w2, loaded by the caller with its inputs); lanes at or
 // above D/2 pass on = false.  inv_freq = exp(-ln(theta) * 2i / D), the
 // normalised values are rounded to bf16 first when round_to_input is set.
-// Every caller (the rope kernel and the fused decode attention) goes through
-// this one sequence of operations, so their q and K agree bit for bit.
+// Every caller (the rope kernel and the fused attentions) goes through this one
+// sequence of operations, so their q and K agree bit for bit; the fused
+// multiply-adds are written out, as which product of a sum the compiler fuses
+// depends on the code around it.
 template <int D>
 __device__ __forceinline__ void norm_rope_pair(float x1, float x2, bool on, float w1, float w2, int lane, float eps,
                                                float log_theta, float position, int round_to_input, uint16_t &o1,
                                                uint16_t &o2) {
     constexpr int HALF = D / 2;
-    const float ss = group_sum<(HALF < kWave ? HALF : kWave)>(on ? x1 * x1 + x2 * x2 : 0.f);
+    const float ss = group_sum<(HALF < kWave ? HALF : kWave)>(on ? fmaf(x1, x1, x2 * x2) : 0.f);
     if (!on) return;
     const float inv_rms = 1.0f / sqrtf(ss / static_cast<float>(D) + eps);
     float f = x1 * inv_rms * w1;
@@ -101,8 +103,8 @@ __device__ __forceinline__ void norm_rope_pair(float x1, float x2, bool on, floa
     const float inv_freq = expf(-log_theta * (static_cast<float>(lane) * 2.0f / static_cast<float>(D)));
     float sn, cs;
     sincosf(position * inv_freq, &sn, &cs);
-    o1 = f32_to_bf16(f * cs - s * sn);
-    o2 = f32_to_bf16(s * cs + f * sn);
+    o1 = f32_to_bf16(fmaf(f, cs, -(s * sn)));
+    o2 = f32_to_bf16(fmaf(s, cs, f * sn));
 }
 
 // Bands (64 output columns each) per GEMM workgroup for `splits` K slices.

@@ -224,6 +224,48 @@ def qkv_partials_rope_short_attention_(
     return out
 
 
+def rope_short_linear_splits(tokens: int, qo_heads: int, kv_heads: int, head_dim: int, out_features: int) -> int:
+    """The planes ``qkv_partials_rope_short_linear_`` leaves for a shape; -1 where it does not take it."""
+
+    return int(_lib.load().nq_cp_rope_short_linear_splits(tokens, qo_heads, kv_heads, head_dim, out_features))
+
+
+def qkv_partials_rope_short_linear_(
+    partials, splits: int, query_weight, key_weight, positions, epsilon, rope_theta, key_cache, value_cache,
+    cache_position: int, weight, planes,
+) -> int:
+    """qkv_partials_rope_short_attention_ and the projection of its output by ``weight`` [out, Hq * D] in one
+    launch, for at most 8 tokens: the caches receive position ``cache_position``'s K and V, ``planes`` the
+    projection as fp32 split-K planes (their number is returned)."""
+
+    _require_bf16(query_weight, key_weight, key_cache, value_cache, weight)
+    tokens, limit, hk, d = key_cache.shape
+    if value_cache.shape != key_cache.shape or value_cache.stride() != key_cache.stride() or key_cache.stride(-1) != 1:
+        raise ValueError("dense CP K and V caches must share one layout")
+    out_features, hq = weight.shape[0], weight.shape[1] // d
+    if weight.ndim != 2 or hq * d != weight.shape[1] or weight.stride(1) != 1 or query_weight.shape != (d,) \
+            or key_weight.shape != (d,):
+        raise ValueError("the weight must be [out, Hq * D] and the norm weights [D]")
+    if not isinstance(cache_position, int) or isinstance(cache_position, bool) or not 0 <= cache_position < min(limit, 16):
+        raise ValueError("dense CP cache position is invalid (short-cache attention covers at most 16)")
+    if positions.dtype != torch.long or positions.shape[0] != tokens:
+        raise ValueError("positions must be int64 with one entry per token")
+    if partials.numel() * partials.element_size() < splits * tokens * (hq + 2 * hk) * d * 4:
+        raise ValueError("partials hold fewer planes than splits")
+    delta = value_cache.data_ptr() - key_cache.data_ptr()
+    if delta % key_cache.element_size():
+        raise ValueError("dense CP K and V caches are misaligned")
+    _lib.require_device(partials, query_weight, key_weight, positions, key_cache, value_cache, weight, planes)
+    _lib.call(
+        "nq_cp_rope_short_linear", partials.data_ptr(), int(splits), tokens, query_weight.data_ptr(),
+        key_weight.data_ptr(), positions.data_ptr(), positions.stride(0), float(epsilon), float(rope_theta), 0,
+        key_cache.data_ptr(), key_cache.stride(0), delta // key_cache.element_size(), key_cache.stride(1),
+        key_cache.stride(2), int(cache_position), hq, hk, d, float(d) ** -0.5, weight.data_ptr(), weight.stride(0),
+        out_features, planes.data_ptr(), planes.numel() * planes.element_size(), _lib.stream(key_cache.device),
+    )
+    return rope_short_linear_splits(tokens, hq, hk, d, out_features)
+
+
 def decode_attn_nhd_short_cache(query, key_cache, value_cache, cache_length: int, out=None):
     """Fixed 16-position code-predictor attention (one query per row)."""
 

@@ -304,6 +304,51 @@ def test_short_cache_head_shapes(nq, device, d, group, position):
         assert torch.equal(x.view(torch.int16), y.view(torch.int16))
 
 
+@pytest.mark.parametrize("rows", [1, 4, 5, 8])
+@pytest.mark.parametrize("position", [0, 7, 15])
+@pytest.mark.parametrize("hkv", [2, 8])
+def test_short_attention_with_its_projection(nq, device, rows, position, hkv):
+    """The launch that projects the attention's output too: the cache's bits and, where the projection alone
+    cuts K into the same 256-wide slices (8 kv heads), the planes' bits of the two launches; else the planes' sum
+    within the fp32 rounding of sums in another order (K terms of |x w|, each rounded at 2^-24)."""
+
+    from nari_qwen3_tts_amd import kernels as K
+    from nari_qwen3_tts_amd.layers import decode_linear, decode_linear_splits
+
+    g = torch.Generator(device=device)
+    g.manual_seed(100 * rows + 10 * position + hkv)
+    d, n, splits = 64, 1024, 3
+    hq = 2 * hkv
+    cache = torch.randn(rows, 2, 16, hkv, d, generator=g, device=device).to(torch.bfloat16)
+    cache[:, :, position:] = float("nan")
+    caches = [cache.clone() for _ in range(2)]
+    planes = torch.randn(splits, rows, (hq + 2 * hkv) * d, generator=g, device=device).view(torch.uint8).flatten()
+    norms = [torch.randn(d, generator=g, device=device).to(torch.bfloat16) for _ in range(2)]
+    weight = torch.randn(n, hq * d, generator=g, device=device).to(torch.bfloat16)
+    at = torch.full((rows,), position, dtype=torch.long, device=device)
+    q = torch.empty(rows, hq, d, dtype=torch.bfloat16, device=device)
+    att = torch.empty_like(q)
+    K.qkv_partials_rope_short_attention_(planes, splits, q, *norms, at, 1e-6, 1e6, caches[0][:, 0], caches[0][:, 1],
+                                         position, att)
+    want = torch.full((decode_linear_splits(rows, n, hq * d), rows, n), float("nan"), device=device)
+    decode_linear(att.view(rows, -1), weight, want.view(torch.uint8).flatten())
+    s = K.rope_short_linear_splits(rows, hq, hkv, d, n)
+    assert s == hkv // 2
+    got = torch.full((s, rows, n), float("nan"), device=device)
+    assert K.qkv_partials_rope_short_linear_(planes, splits, *norms, at, 1e-6, 1e6, caches[1][:, 0], caches[1][:, 1],
+                                             position, weight, got.view(torch.uint8).flatten()) == s
+    assert torch.equal(caches[0].view(torch.int16), caches[1].view(torch.int16))
+    if got.shape == want.shape and hkv == 8:
+        assert torch.equal(got, want)
+    bound = att.view(rows, -1).float().abs() @ weight.float().abs().t() * (hq * d * 2.0**-24)
+    assert bool(((got.sum(0) - want.sum(0)).abs() <= bound).all())
+    # shapes it does not take
+    assert K.rope_short_linear_splits(9, hq, hkv, d, n) == -1
+    assert K.rope_short_linear_splits(rows, hkv, hkv, d, n) == -1
+    assert K.rope_short_linear_splits(rows, hq, hkv, 128, n) == -1
+    assert K.rope_short_linear_splits(rows, hq, hkv, d, n + 16) == -1
+
+
 def _fused_case(nq, device, seed, lengths, capture, pages, ps=16):
     rng = np.random.default_rng(seed)
     kv = make_kv(nq, device, layers=1, pages=pages, ps=ps, scratch=capture)
