@@ -853,7 +853,7 @@ overlap_fixup_kernel(const int32_t *__restrict__ off, int B, int u_in, int s, co
 // i0 - R + kappa < 0, else fresh frame f = i0 - R + kappa, rotated here (and
 // written back in place, so a later block reads it rotated) unless an earlier
 // block already did.  K, V and the rotated q of a block are staged in LDS
-// (rows of D + 4 floats).  Eight queries then go at a time, a thread each
+// (rows of D + 4 floats).  Thirty-two queries then go at a time, a thread each
 // (query j, window step s), which reads key row j + s: 32 lanes read 32
 // consecutive rows, and a 16-byte read spreads over the banks.  A query's
 // scores lie in half a wave, which finds its softmax with shuffles and takes
@@ -861,11 +861,13 @@ overlap_fixup_kernel(const int32_t *__restrict__ off, int B, int u_in, int s, co
 // is written in: with a query a lane and the window's steps unrolled (25 KB
 // of code, four lanes of 64 at work on a four-frame chunk) a launch took
 // 17 us at one stream of four frames and 18.5 us at 32 of 12 - 48, and takes
-// 8.5 and 18.0.  After the last block the new retained rows (the last R positions) are written from
-// LDS: the state is read (staged) before this workgroup overwrites it, and no
-// other workgroup touches this (stream, head).
+// 5.6 and 11.0.  A CU holds one workgroup, so its threads are 1024: with 256
+// the 32 streams took 18.1, with 512 13.2.  After the last block the new
+// retained rows (the last R positions) are written from LDS: the state is read
+// (staged) before this workgroup overwrites it, and no other workgroup touches
+// this (stream, head).
 
-constexpr int kWinThreads = 256;
+constexpr int kWinThreads = 1024;
 constexpr int kWinQ = 64;     // queries per block
 constexpr int kWinMax = 32;   // window (R + 1) the kernel takes
 constexpr int kWinGroup = kWinThreads / kWinMax;  // queries whose (query, step) pairs are one per thread
@@ -992,7 +994,7 @@ window_block_kernel(const float *__restrict__ q, float *__restrict__ k, const fl
         }
         __syncthreads();
 
-        // eight queries at a time, one thread per (query, window step): half a wave holds a query's
+        // kWinGroup queries at a time, one thread per (query, window step): half a wave holds a query's
         // scores, and its lanes then take the query's channels
         for (int j0 = 0; j0 < nq; j0 += kWinGroup) {
             const int j = j0 + threadIdx.x / kWinMax, s = threadIdx.x % kWinMax;

@@ -361,12 +361,11 @@ def test_convolution_tiles_keep_to_their_stream(nq, device, channels, streams):
     assert torch.equal(hist.cpu(), want_hist)
 
 
-@pytest.mark.parametrize("frames", [1, 7, 8, 9, 71, 72, 73])
+@pytest.mark.parametrize("frames", [1, 31, 32, 33, 64, 65, 97])
 @pytest.mark.parametrize("D", [16, 32, 64])
-def test_window_attention_of_few_queries(nq, device, D, frames):
-    """Blocks of up to eight queries take one thread per (query, window step), longer ones one lane per query:
-    chunks around that line (and whose last block lies around it), with five of the retained rows valid and the
-    others infinite or NaN, within 1e-4 of the oracle: an angle below 128 rounds at 2^-18, which moves a score of
+def test_window_attention_query_groups(nq, device, D, frames):
+    """Blocks of 64 queries go 32 at a time, a thread per (query, window step): chunks around both lines, with five
+    of the retained rows valid and the others infinite or NaN, within 1e-4 of the oracle: an angle below 128 rounds at 2^-18, which moves a score of
     at most |q| |k| / sqrt(D) = 8 by at most 2 * 8 * 2^-18 = 6e-5, and outputs of unit size by as much."""
     from nari_qwen3_tts_amd import _lib
 
