@@ -21,7 +21,9 @@ valid positions, o_proj with the residual add + post-attention RMSNorm fused,
 gate_up with the SwiGLU fused (one kernel over interleaved gate/up rows), down
 with the residual add + next RMSNorm fused.  The residual
 adds are the reference's plain bf16 ``residual + projection`` followed by the
-norm (components.py:331-346), which is what the fused epilogue computes.
+norm (components.py:331-346), which is what the fused epilogue computes.  Frames
+of a few rows take four launches a layer: the projections normalise their rows
+themselves, and the attention's launch holds the o projection.
 
 Sampling takes uniforms ([15, rows], one per row and group); with
 ``use_counter_rng`` they are derived on the device from (seed, offsets[:, g-1])
