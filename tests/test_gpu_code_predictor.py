@@ -167,3 +167,57 @@ def test_bench_frame_b128_matches_oracle(nq, device):
         np.testing.assert_array_equal(tokens[k], want_tok)
     np.testing.assert_array_equal(to_np(frame.frames)[:, 1:], tokens.T)
     np.testing.assert_array_equal(to_np(frame.codec_sum), csum)
+
+
+def _few_inputs(frame, cfg, device, seed, temperature=0.9):
+    g = torch.Generator(device=device)
+    g.manual_seed(seed)
+    rows = frame.rows
+    frame.layer0_token.copy_(torch.randint(0, cfg.talker_vocab, (rows,), generator=g, device=device))
+    frame.past_hidden.copy_(torch.randn(rows, cfg.talker_hidden, generator=g, device=device).to(torch.bfloat16))
+    frame.seed.copy_(torch.randint(0, 1 << 40, (rows,), generator=g, device=device))
+    frame.offsets.copy_(torch.arange(rows * 15, device=device).view(rows, 15) * 3)
+    frame.temperature.fill_(temperature)
+    frame.top_k.fill_(50)
+    frame.top_p.fill_(0.95)
+
+
+@pytest.mark.parametrize("rows", [1, 8, 9])
+def test_whole_frame_replays_in_a_graph(nq, device, rows):
+    """All five layers on both sides of the few-row limit: replays on new inputs, eager runs between them,
+    the same bits; and the first pass's K/V and the first group's logits, which no draw precedes, within
+    bf16 rounding of the general layers' (sums in another order)."""
+
+    from nari_qwen3_tts_amd.code_predictor import CodePredictorConfig, CodePredictorFrame, CodePredictorWeights
+    from nari_qwen3_tts_amd.graphs import HipGraphCaptureDriver
+
+    cfg = CodePredictorConfig()
+    w = CodePredictorWeights(cfg, device, seed=80 + rows)
+    frame = CodePredictorFrame(w, rows, use_counter_rng=True)
+    few = frame.few
+    assert few == (rows <= 8)
+    _few_inputs(frame, cfg, device, 81)
+    call = HipGraphCaptureDriver(device=device).capture(frame.forward)
+
+    def outputs():
+        torch.cuda.synchronize()
+        return [t.clone() for t in (frame.frames, frame.codec_sum, frame.logits, frame.kv_cache)]
+
+    for trial in range(3):
+        _few_inputs(frame, cfg, device, 82 + trial)
+        frame.kv_cache.fill_(float("nan"))
+        call.replay()
+        replayed = outputs()
+        frame.kv_cache.fill_(float("nan"))
+        frame.forward()
+        eager = outputs()
+        for a, b in zip(replayed, eager):
+            assert torch.equal(a, b)
+    if few:
+        frame.few = False
+        frame.forward()
+        general = outputs()
+        pairs = [(eager[2][0], general[2][0])] + [(eager[3][i, :, :, :2], general[3][i, :, :, :2])
+                                                  for i in range(cfg.num_layers)]
+        for a, b in pairs:
+            assert float((a.float() - b.float()).norm() / b.float().norm()) <= 1e-2

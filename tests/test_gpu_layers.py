@@ -289,34 +289,52 @@ def test_decode_linear_planes(nq, device, m, n, k):
         L.decode_linear(x, w, planes[: splits * m * n - 1])
 
 
+def _decode_step(nq, device, weights, rows, **options):
+    """A planned decode step of ``rows`` random histories on a 256-page pool, inputs set, not run; and the pool's
+    content before it."""
+
+    from helpers import DecodeKey, adopt_random, make_kv
+    from nari_qwen3_tts_amd.talker import TalkerDecodeStep
+
+    rng = np.random.default_rng(17)
+    kv = make_kv(nq, device, layers=weights.config.num_layers, pages=256)
+    gen = torch.Generator(device=device)
+    gen.manual_seed(4)
+    kv.storage.copy_(torch.randn(kv.storage.shape, generator=gen, device=device))
+    rids = adopt_random(kv, rng, rng.integers(5, 200, size=rows))
+    ctx = kv.create_decode(DecodeKey(rows), slot=0)
+    step = TalkerDecodeStep(weights, ctx, rows, **options)
+    step.step_embed.copy_(torch.randn(rows, weights.config.hidden, generator=gen, device=device))
+    step.temperature.fill_(0.9)
+    step.top_k.fill_(50)
+    step.top_p.fill_(0.95)
+    step.seed.copy_(torch.arange(rows, device=device) + 3)
+    kv.prepare_decode(ctx, DecodeKey(rows), tuple(rids))
+    return kv, ctx, step, kv.storage.clone()
+
+
 @pytest.mark.parametrize("rows", [1, 4])
 def test_few_row_decode_step_equals_the_general_one(nq, device, rows):
     """The step whose projections normalise their rows against the step with its own norm launches:
-    logits, hidden state, residual and written K/V within bf16 rounding of sums in another order."""
+    logits, hidden state, residual and each layer's written K and V within bf16 rounding of sums in another
+    order; no other position of the pool changes."""
 
-    from helpers import DecodeKey, adopt_random, make_kv
-    from nari_qwen3_tts_amd.talker import TalkerConfig, TalkerDecodeStep, TalkerWeights
+    from nari_qwen3_tts_amd.talker import TalkerConfig, TalkerWeights
 
     cfg = TalkerConfig(num_layers=2)
     weights = TalkerWeights(cfg, device, seed=9)
     outs = []
     for few in (True, False):
-        rng = np.random.default_rng(17)
-        kv = make_kv(nq, device, layers=2, pages=256)
-        gen = torch.Generator(device=device)
-        gen.manual_seed(4)
-        kv.storage.copy_(torch.randn(kv.storage.shape, generator=gen, device=device))
-        rids = adopt_random(kv, rng, rng.integers(5, 200, size=rows))
-        ctx = kv.create_decode(DecodeKey(rows), slot=0)
-        step = TalkerDecodeStep(weights, ctx, rows, use_counter_rng=True)
+        kv, ctx, step, before = _decode_step(nq, device, weights, rows, use_counter_rng=True)
         assert step.few
         step.few = few
-        step.step_embed.copy_(torch.randn(rows, cfg.hidden, generator=gen, device=device))
-        step.temperature.fill_(0.9)
-        kv.prepare_decode(ctx, DecodeKey(rows), tuple(rids))
         step.forward()
         torch.cuda.synchronize()
-        outs.append([t.float() for t in (step.logits, step.hidden, step.residual, kv.storage)])
+        pages, slots = ctx.metadata.write_pages.long(), ctx.metadata.write_offsets.long()
+        written = [kv.storage[layer, pages, kind, slots].float() for layer in range(2) for kind in range(2)]
+        before[:, pages, :, slots] = kv.storage[:, pages, :, slots]
+        assert torch.equal(before.view(torch.int16), kv.storage.view(torch.int16))
+        outs.append([t.float() for t in (step.logits, step.hidden, step.residual)] + written)
     for a, b in zip(*outs):
         # two layers: an FP8 code that falls to the other side moves a value by a sixteenth
         assert float((a - b).norm() / b.norm()) <= 1e-2
