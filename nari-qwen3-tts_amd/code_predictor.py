@@ -262,25 +262,38 @@ class CodePredictorFrame:
     # the most rows of 1024 that every workgroup of a projection normalises for itself
     FEW_ROWS = 8
 
-    def _layers_few(self, cache_pos: int):
+    def _layers_few(self, cache_pos: int, head: torch.Tensor | None) -> torch.Tensor | None:
         """The layers from self.h and its first input norm self.x with four launches each: QKV, attention
         and o, gate/up + SwiGLU, down, the add-RMSNorms inside the projections after them.  Returns the
-        final norm's rows, for the head."""
+        logits of ``head`` as one plane [1, rows, vocab]; without a head, none."""
 
         c = self.w.config
         a, b = self.workspace[: self._region], self.workspace[self._region: 2 * self._region]
         h, h2 = self.h, self.h2
         positions = self.position_ids[:, cache_pos]
+        trace = None if self.trace is None else self.trace[cache_pos]
+        if trace is not None:
+            trace[0].copy_(h)
         splits = decode_linear(self.x, self.w.layers[0].qkv, b)
         for index, L in enumerate(self.w.layers):
             if index:
                 splits = decode_norm_linear(NormRows(a, down, h2, h, L.input_norm, c.rms_eps), L.qkv, b)
+                if trace is not None:  # the layer before ended in this launch
+                    trace[index].copy_(h)
             cache = self.kv_cache[index]
             splits = qkv_partials_rope_short_linear_(b, splits, L.q_norm, L.k_norm, positions, c.rms_eps, c.rope_theta,
                                                      cache[:, 0], cache[:, 1], cache_pos, L.o, a)
             decode_norm_swiglu(NormRows(a, splits, h, h2, L.post_norm, c.rms_eps), L.gate_up_packed, self.act)
             down = decode_linear(self.act, L.down, a)
-        return NormRows(a, down, h2, h, self.w.final_norm, c.rms_eps, self.x)
+        if head is None:
+            if trace is None:
+                return None
+            head = self.w.lm_head[0]  # for the record alone: this launch ends the last layer and norms its rows
+        decode_norm_linear(NormRows(a, down, h2, h, self.w.final_norm, c.rms_eps, self.x), head, b)
+        if trace is not None:
+            trace[len(self.w.layers)].copy_(h)
+            trace[len(self.w.layers) + 1].copy_(self.x)
+        return b[: self.rows * c.vocab * 4].view(torch.float32).view(1, self.rows, c.vocab)
 
     def _layers(self, cache_pos: int, normed: bool = False) -> None:
         """The 5 layers at cache position ``cache_pos``; ``normed``: self.x already holds the first
@@ -317,39 +330,41 @@ class CodePredictorFrame:
         groups = c.num_code_groups
         # pass 0: the talker hidden state fills cache position 0
         linear(self.past_hidden, w.proj_w, out=self.h, workspace=ws, bias=w.proj_b)
-        few = self.few and self.trace is None and self.use_counter_rng and self.sampler is None
-        if few:
+        if self.few:
             rmsnorm(self.h, w.layers[0].input_norm, c.rms_eps, out=self.x)
-            self._layers_few(0)
+            self._layers_few(0, None)
         else:
             self._layers(0)
         self.frames[:, 0].copy_(self.layer0_token)
         # the next input (a projected embedding row) and the first input norm in one launch
         first_norm = w.layers[0].input_norm
         embed_add_rmsnorm(self.layer0_token, w.projected_layer0, None, first_norm, c.rms_eps, self.h, self.x)
+        # the draw inside the package from the counters takes the head's split-K planes: summed, rounded and
+        # drawn from in the sampling launch.  Every other one takes the bf16 logits: the same bits
+        from_planes = self.use_counter_rng and self.sampler is None
         for group in range(1, groups):
             logits = self.logits[group - 1]
             token = self.tokens[group - 1]
             head = w.lm_head[group - 1]
-            planes = ws  # the head's planes
-            if few:
-                planes = ws[self._region:]
-                splits = decode_norm_linear(self._layers_few(group), head, planes)
+            planes = None
+            if self.few:
+                planes = self._layers_few(group, head)
+                if not from_planes:
+                    logits.copy_(planes[0])
             else:
                 self._layers(group, normed=True)
+                if from_planes:
+                    splits = linear_partials(self.x, head, ws)
+                    planes = ws[: splits * self.rows * c.vocab * 4].view(torch.float32).view(splits, self.rows, c.vocab)
+                else:
+                    linear(self.x, head, out=logits, workspace=ws)
             if self.sampler is not None:
-                linear(self.x, w.lm_head[group - 1], out=logits, workspace=ws)
                 token.copy_(self.sampler(logits, self.temperature, self.top_k, self.top_p, self.seed,
                                          self.offsets[:, group - 1]))
-            elif self.use_counter_rng:
-                # the head's split-K planes summed, rounded and drawn from in the sampling launch
-                if not few:
-                    splits = linear_partials(self.x, head, ws)
-                planes = planes[: splits * self.rows * c.vocab * 4].view(torch.float32).view(splits, self.rows, c.vocab)
+            elif from_planes:
                 sample_with_counter_from_planes(planes, self.temperature, self.top_k, self.top_p, self.seed,
                                                 self.offsets[:, group - 1], logits_out=logits, out=token)
             else:
-                linear(self.x, w.lm_head[group - 1], out=logits, workspace=ws)
                 sample_with_uniforms(logits, self.temperature, self.top_k, self.top_p, self.uniforms[group - 1],
                                      out=token)
             if group < groups - 1:

@@ -363,27 +363,34 @@ class TalkerDecodeStep:
         return ((c.qkv_width, c.hidden), (c.hidden, c.num_qo_heads * c.head_dim), (c.hidden, c.intermediate),
                 (c.vocab, c.hidden))
 
-    def _forward_few(self) -> int:
+    def _forward_few(self) -> torch.Tensor:
         """The layers with five launches each: QKV, attention, o, gate/up + SwiGLU, down, the add-RMSNorms
-        inside the projections after them; leaves the codec head's plane in the second region."""
+        inside the projections after them; returns the codec head's logits as one plane [1, rows, vocab]."""
 
         c, ctx, n = self.w.config, self.context, self.rows
         q_w = c.num_qo_heads * c.head_dim
         a, b = self.linear_workspace[: self._region], self.linear_workspace[self._region: 2 * self._region]
         h, h2 = self.residual, self.residual2
+        trace = self.trace
+        if trace is not None:
+            trace[0].copy_(h)
         q = self.qkv[:, :q_w].view(n, c.num_qo_heads, c.head_dim)
         splits = decode_linear(self.hidden, self.w.layers[0].qkv, b)
         for index, layer in enumerate(self.w.layers):
             ctx.select_layer(index)
             if index:
                 splits = decode_norm_linear(NormRows(a, down, h2, h, layer.input_norm, c.rms_eps), layer.qkv, b)
+                if trace is not None:  # the layer before ended in this launch
+                    trace[index].copy_(h)
             attended = ctx.attend_partials(layer.attention, b, splits, q).view(n, q_w)
             splits = decode_linear(attended, layer.o, a)
             decode_norm_swiglu(NormRows(a, splits, h, h2, layer.post_norm, c.rms_eps), layer.gate_up_packed, self.act,
                                layer.gate_up_scales)
             down = decode_linear(self.act, layer.down, a)
-        return decode_norm_linear(NormRows(a, down, h2, h, self.w.final_norm, c.rms_eps, self.hidden),
-                                  self.w.codec_head, b)
+        decode_norm_linear(NormRows(a, down, h2, h, self.w.final_norm, c.rms_eps, self.hidden), self.w.codec_head, b)
+        if trace is not None:
+            trace[len(self.w.layers)].copy_(h)
+        return b[: n * c.vocab * 4].view(torch.float32).view(1, n, c.vocab)
 
     def forward(self) -> torch.Tensor:
         c = self.w.config
@@ -393,10 +400,10 @@ class TalkerDecodeStep:
         embed_add_rmsnorm(self.text_ids, self.w.text_embedding, self.step_embed, self.w.layers[0].input_norm,
                           c.rms_eps, self.residual, self.hidden, status=self.embed_status)
         trace = self.trace
-        if self.few and trace is None and self.use_counter_rng:
-            splits = self._forward_few()
+        if self.few:
+            planes = self._forward_few()
             ctx.advance_sequence_lengths()
-            self._sample(self.linear_workspace[self._region:], splits)
+            self._sample(planes)
             self._report()
             return self.tokens
         if trace is not None:
@@ -435,12 +442,12 @@ class TalkerDecodeStep:
                   self.embed_status.data_ptr(), self.tokens.data_ptr(), self.rows, c.eos_id, c.vocab,
                   self.report.device.data_ptr(), _lib.stream(self.device))
 
-    def _sample(self, planes: torch.Tensor | None = None, splits: int = 0) -> None:
-        """``planes``: the codec head's ``splits`` planes, when the layers left them already."""
+    def _sample(self, planes: torch.Tensor | None = None) -> None:
+        """``planes``: the codec head's fp32 planes [S, rows, vocab], when the layers left them already."""
 
         c = self.w.config
         n = self.rows
-        ws = self.linear_workspace if planes is None else planes
+        ws = self.linear_workspace
         options = dict(repetition_penalty=self.penalty, seen_token_mask=self.seen, mask_from=c.codec_vocab,
                        eos_id=c.eos_id, suppress_eos=self.suppress_eos, update_seen=True, out=self.tokens)
         if self.use_counter_rng:
@@ -448,12 +455,15 @@ class TalkerDecodeStep:
             # (the same logits and tokens as the projection followed by the sampler)
             if planes is None:
                 splits = linear_partials(self.hidden, self.w.codec_head, ws)
-            planes = ws[: splits * n * c.vocab * 4].view(torch.float32).view(splits, n, c.vocab)
+                planes = ws[: splits * n * c.vocab * 4].view(torch.float32).view(splits, n, c.vocab)
             sample_with_counter_from_planes(planes, self.temperature, self.top_k, self.top_p, self.seed, self.offsets,
                                             logits_out=self.logits, **options)
             return
         # caller-supplied uniforms
-        linear(self.hidden, self.w.codec_head, out=self.logits, workspace=ws)
+        if planes is None:
+            linear(self.hidden, self.w.codec_head, out=self.logits, workspace=ws)
+        else:
+            self.logits.copy_(planes[0])
         sample_with_uniforms(self.logits, self.temperature, self.top_k, self.top_p, self.uniforms, **options)
 
 

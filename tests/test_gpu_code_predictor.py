@@ -182,6 +182,74 @@ def _few_inputs(frame, cfg, device, seed, temperature=0.9):
     frame.top_p.fill_(0.95)
 
 
+@pytest.mark.parametrize("rows", [1, 5, 8, 9])
+def test_frame_bits_do_not_depend_on_its_observers(nq, device, rows):
+    """A frame that records its residual stream, draws through a sampler hook or takes the uniforms of its
+    counters from the caller has the bits of the frame that does neither, on both sides of the few-row
+    limit; the record's last entries are the residual and the rows the head read."""
+
+    from nari_qwen3_tts_amd.code_predictor import CodePredictorConfig, CodePredictorFrame, CodePredictorWeights
+    from nari_qwen3_tts_amd.sampling import sample_logits_cuda_graph, uniforms_from_counter
+
+    cfg = CodePredictorConfig()
+    w = CodePredictorWeights(cfg, device, seed=60 + rows)
+    got = {}
+    for kind in ("plain", "trace", "hook", "uniforms"):
+        frame = CodePredictorFrame(w, rows, use_counter_rng=kind != "uniforms")
+        _few_inputs(frame, cfg, device, 61)
+        if kind == "trace":
+            frame.trace = torch.full((16, cfg.num_layers + 2, rows, cfg.hidden), float("nan"), dtype=torch.bfloat16,
+                                     device=device)
+        if kind == "hook":
+            frame.sampler = sample_logits_cuda_graph
+        if kind == "uniforms":
+            for k in range(15):
+                frame.uniforms[k].copy_(uniforms_from_counter(frame.seed, frame.offsets[:, k].contiguous()))
+        frame.forward()
+        torch.cuda.synchronize()
+        got[kind] = (frame.frames, frame.tokens, frame.codec_sum, frame.logits, frame.kv_cache, frame.h, frame.x)
+        if kind == "trace":
+            assert not bool(frame.trace.isnan().any())
+            assert torch.equal(frame.trace[15, cfg.num_layers], frame.h)
+            assert torch.equal(frame.trace[15, cfg.num_layers + 1], frame.x)
+    for kind in ("trace", "hook", "uniforms"):
+        for a, b in zip(got["plain"], got[kind]):
+            assert torch.equal(a, b), kind
+
+
+@pytest.mark.parametrize("rows", [1, 8])
+def test_few_row_frame_layers_match_oracle(nq, device, rows):
+    """Every layer of every pass of a few-row frame on the device's own input and earlier K/V, the logits on
+    the device's own normalised rows: the bounds of the 128-row frame."""
+
+    from nari_qwen3_tts_amd.code_predictor import CodePredictorConfig, CodePredictorFrame, CodePredictorWeights
+
+    cfg = CodePredictorConfig()
+    w = CodePredictorWeights(cfg, device, seed=70 + rows)
+    frame = CodePredictorFrame(w, rows, use_counter_rng=True)
+    assert frame.few
+    _few_inputs(frame, cfg, device, 71)
+    layers = cfg.num_layers
+    frame.trace = torch.zeros(16, layers + 2, rows, cfg.hidden, dtype=torch.bfloat16, device=device)
+    frame.forward()
+    torch.cuda.synchronize()
+    hw = _host_weights(w)
+    hcfg = dict(num_qo_heads=cfg.num_qo_heads, num_kv_heads=cfg.num_kv_heads, head_dim=cfg.head_dim,
+                rms_eps=cfg.rms_eps, rope_theta=cfg.rope_theta, num_code_groups=cfg.num_code_groups)
+    trace, got, device_cache = to_np(frame.trace), to_np(frame.logits), to_np(frame.kv_cache)
+    positions = to_np(frame.position_ids)
+    for g in range(16):
+        for i in range(layers):
+            cache = device_cache.copy()
+            _, h = o_cp.layer(hw, hcfg, i, trace[g, i], cache, g, positions[:, g])
+            want, dev = h - trace[g, i], trace[g, i + 1] - trace[g, i]
+            assert np.linalg.norm(dev - want) <= 1e-2 * np.linalg.norm(want), (g, i)
+            assert np.abs(cache[i, :, :, g] - device_cache[i, :, :, g]).max() <= 3e-2, (g, i)
+        if g:
+            err = np.abs(got[g - 1] - o_cp.logits_of(hw, trace[g, layers + 1], g))
+            assert err.mean() <= 2e-3 and err.max() <= 2e-2, (g, err.mean(), err.max())
+
+
 @pytest.mark.parametrize("rows", [1, 8, 9])
 def test_whole_frame_replays_in_a_graph(nq, device, rows):
     """All five layers on both sides of the few-row limit: replays on new inputs, eager runs between them,

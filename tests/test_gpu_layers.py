@@ -338,3 +338,34 @@ def test_few_row_decode_step_equals_the_general_one(nq, device, rows):
     for a, b in zip(*outs):
         # two layers: an FP8 code that falls to the other side moves a value by a sixteenth
         assert float((a - b).norm() / b.norm()) <= 1e-2
+
+
+@pytest.mark.parametrize("rows", [1, 4, 5])
+def test_decode_step_bits_do_not_depend_on_its_observers(nq, device, rows):
+    """A step that records its residual stream, or takes the uniforms of its counters from the caller, has the
+    bits of the step that does neither, on both sides of the few-row limit."""
+
+    from nari_qwen3_tts_amd.sampling import uniforms_from_counter
+    from nari_qwen3_tts_amd.talker import TalkerConfig, TalkerWeights
+
+    cfg = TalkerConfig(num_layers=3)
+    weights = TalkerWeights(cfg, device, seed=9)
+    outs = {}
+    for kind in ("plain", "trace", "uniforms"):
+        kv, ctx, step, _ = _decode_step(nq, device, weights, rows, use_counter_rng=kind != "uniforms")
+        assert step.few == (rows <= 4)
+        if kind == "trace":
+            step.trace = torch.full((cfg.num_layers + 1, rows, cfg.hidden), float("nan"), dtype=torch.bfloat16,
+                                    device=device)
+        if kind == "uniforms":
+            step.uniforms.copy_(uniforms_from_counter(step.seed, step.offsets))
+        step.forward()
+        torch.cuda.synchronize()
+        outs[kind] = [step.logits, step.tokens, step.hidden, step.residual, kv.storage]
+        if kind == "trace":
+            assert not bool(step.trace.isnan().any()) and torch.equal(step.trace[-1], step.residual)
+            # every layer moves every row
+            assert bool((step.trace[1:] != step.trace[:-1]).any(dim=2).all())
+    for kind in ("trace", "uniforms"):
+        for a, b in zip(outs["plain"], outs[kind]):
+            assert torch.equal(a, b), kind
