@@ -802,7 +802,9 @@ struct SoftmaxState {
         }
     }
 
-    // Fold the lane groups of the wave together (result valid in every lane).
+    // Fold the lane groups of the wave together (result valid in every lane).  The fused multiply-adds are
+    // written out: of a sum of two products the compiler fuses the one that the code around it suggests,
+    // and an output's last bit went with it.
     __device__ __forceinline__ void combine_lane_groups() {
         constexpr int LPT = Lanes<D, G>::LPT;
 #pragma unroll
@@ -814,11 +816,11 @@ struct SoftmaxState {
                 const float mn = fmaxf(m[j], mo);
                 const float a = m[j] == -INFINITY ? 0.f : exp2f(m[j] - mn);
                 const float bsc = mo == -INFINITY ? 0.f : exp2f(mo - mn);
-                l[j] = l[j] * a + lo * bsc;
+                l[j] = fmaf(l[j], a, lo * bsc);
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
                     const float ao = __shfl_xor(acc[j][e], mask, kWave);
-                    acc[j][e] = acc[j][e] * a + ao * bsc;
+                    acc[j][e] = fmaf(acc[j][e], a, ao * bsc);
                 }
                 m[j] = mn;
             }
@@ -2631,10 +2633,11 @@ __device__ __forceinline__ void prefill_tiles(
                         const float w0 = wt[p], w1 = wt[p + 1];
 #pragma unroll
                         for (int w = 0; w < kWords; ++w) {
-                            o[2 * w] += w0 * __uint_as_float(static_cast<uint32_t>(u[0][w])) +
-                                        w1 * __uint_as_float(static_cast<uint32_t>(u[1][w]));
-                            o[2 * w + 1] += w0 * __uint_as_float(static_cast<uint32_t>(u[0][w] >> 32)) +
-                                            w1 * __uint_as_float(static_cast<uint32_t>(u[1][w] >> 32));
+                            // the fused multiply-add written out, as in combine_lane_groups
+                            o[2 * w] += fmaf(w0, __uint_as_float(static_cast<uint32_t>(u[0][w])),
+                                             w1 * __uint_as_float(static_cast<uint32_t>(u[1][w])));
+                            o[2 * w + 1] += fmaf(w0, __uint_as_float(static_cast<uint32_t>(u[0][w] >> 32)),
+                                                 w1 * __uint_as_float(static_cast<uint32_t>(u[1][w] >> 32)));
                         }
                     }
                     uint16_t *op = out + static_cast<int64_t>(q0 + mq) * o_s0 + hh * o_s1 + quarter * kQuarter;

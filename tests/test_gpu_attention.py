@@ -413,3 +413,51 @@ def test_fused_decode_rope_attention(nq, device, kind):
         mx, mean = attention_error(to_np(got), want)
         assert mx <= MAX_ABS and mean <= MEAN_ABS, (kind, mx, mean)
     kv.abort(pubs)
+
+
+def _hashed(shape, salt, device):
+    """bf16 values in [-2, 2) from the elements' indexes, the same with every version of every library."""
+
+    n = int(np.prod(shape))
+    at = torch.arange(n, dtype=torch.int64, device=device) + salt * 1_000_003
+    at = (at * 2654435761) & 0xffffffff
+    at = ((at ^ (at >> 15)) * 2246822519) & 0xffffffff
+    return ((at >> 13) % 256).to(torch.float32).sub_(128).div_(64).to(torch.bfloat16).view(shape)
+
+
+@pytest.mark.parametrize("kind,want", [("bins", 1252230173), ("stream", 374597755), ("pieces", 2400189654),
+                                       ("wide-pieces", 2175521152)])
+def test_attention_bits(nq, device, kind, want):
+    """The checksum of what the decode bins, the stream kernel with its merge and the prefill tiles with theirs
+    give on fixed inputs: an output's last bit hangs on which product of a sum of two is fused, and does not
+    move with the compiler's choice.  A change of the arithmetic itself changes the checksums."""
+
+    rng = np.random.default_rng(6)
+    if kind in ("bins", "stream"):
+        kv = make_kv(nq, device, pages=8192, scratch=64)
+        kv.storage.copy_(_hashed(kv.storage.shape, 1, device))
+        rids = adopt_random(kv, rng, rng.integers(64, 1500, size=64))
+        key = DecodeKey(64)
+        ctx = kv.create_decode(key, slot=0)
+        kv.prepare_decode(ctx, key, tuple(rids))
+        outs = []
+        for salt in range(2, 6):
+            q = _hashed((64, 16, 128), salt, device)
+            if kind == "stream":
+                outs.append(_run(nq, ctx, q).clone())
+                continue
+            planes = _hashed((4 * 64 * 4096,), salt, device).float()
+            one = torch.ones(128, dtype=torch.bfloat16, device=device)
+            outs.append(ctx.attend_partials(attention_module(128, weights=(one, one), device=device), planes, 4,
+                                            torch.empty_like(q)).clone())
+            assert ctx.fused_decode
+    else:
+        kv = make_kv(nq, device, pages=2048, scratch=64)
+        kv.storage.copy_(_hashed(kv.storage.shape, 1, device))
+        rids = adopt_random(kv, rng, np.array([3100, 40, 2900]))
+        key = PrefillKey(4, 400)
+        ctx = kv.create_prefill(key, slot=0, decode_rows=kind == "wide-pieces")
+        kv.prepare_prefill(ctx, key, tuple(rids), (200, 1, 190))
+        outs = [_run(nq, ctx, _hashed((400, 16, 128), salt, device))[:391].clone() for salt in range(2, 6)]
+    got = torch.stack(outs).view(torch.int16).cpu().numpy()
+    assert zlib.crc32(got.tobytes()) == want
