@@ -1851,6 +1851,14 @@ dense_short_kernel(const uint16_t *__restrict__ q, int64_t q_s0, int64_t q_s1,
 
 constexpr int kShortLen = 16;
 
+// Where the one-wave kernels run: up to 16 positions, even output strides (a lane stores two outputs as one
+// word) and a grid that a launch can hold (below 2^32 threads).  dense_short_kernel and
+// dense_rope_short_kernel take every other call of the same entries: they walk any length, store single
+// outputs and loop over their items.
+bool short_takes(int length, int64_t items, int64_t o_s0, int64_t o_s1) {
+    return length <= kShortLen && items < (int64_t{1} << 32) / kWave && o_s0 % 2 == 0 && o_s1 % 2 == 0;
+}
+
 // LDS written by one lane of a wave, read by another: a wave's LDS accesses complete in order
 __device__ __forceinline__ void short_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -2778,7 +2786,7 @@ int launch_dense(const uint16_t *q, int64_t q_s0, int64_t q_s1, const uint16_t *
                  int valid_length, int Hkv, float scale, uint16_t *out, int64_t o_s0, int64_t o_s1,
                  hipStream_t stream) {
     int64_t items = static_cast<int64_t>(rows) * Hkv;
-    if (valid_length <= kShortLen && items <= 0x7fffffff && (o_s0 % 2 | o_s1 % 2) == 0) {
+    if (short_takes(valid_length, items, o_s0, o_s1)) {
         hipLaunchKernelGGL((short_kernel<D, G>), dim3(static_cast<unsigned>(items)), dim3(kWave), 0, stream, q, q_s0,
                            q_s1, cache, c_row, c_kind, c_pos, c_head, valid_length, Hkv, scale * kLog2e, out, o_s0,
                            o_s1);
@@ -2799,7 +2807,7 @@ int launch_dense_rope(const float *partials, int splits, int rows, const uint16_
                       int64_t o_s0, int64_t o_s1, hipStream_t stream) {
     const int64_t prow = static_cast<int64_t>(Hkv * G + 2 * Hkv) * D;
     const int64_t items = static_cast<int64_t>(rows) * Hkv;
-    if (cache_position < kShortLen && items <= 0x7fffffff && (o_s0 % 2 | o_s1 % 2) == 0) {
+    if (short_takes(cache_position + 1, items, o_s0, o_s1)) {
         const ShortRope src{partials, splits, static_cast<int64_t>(rows) * prow, prow, q_weight, k_weight, positions,
                             pos_stride, eps, logf(rope_theta), round_to_input, q_out, q_s0, q_s1, cache, c_row, c_kind,
                             c_pos, c_head, cache_position, Hkv, scale * kLog2e};

@@ -304,6 +304,55 @@ def test_short_cache_head_shapes(nq, device, d, group, position):
         assert torch.equal(x.view(torch.int16), y.view(torch.int16))
 
 
+@pytest.mark.parametrize("d,group", [(64, 2), (64, 8), (128, 1), (128, 2)])
+@pytest.mark.parametrize("length,odd", [(17, False), (33, False), (16, True), (40, True)])
+def test_short_cache_entries_past_sixteen_positions(nq, device, d, group, length, odd):
+    """The C entries take any length and output stride (their Python callers at most 16 positions, even
+    strides): the workgroup form, against the oracle, positions past the length holding NaN and the gaps
+    between output rows left alone; the fused entry's q, cache and output bits are those of the two launches."""
+
+    from nari_qwen3_tts_amd import _lib
+    from nari_qwen3_tts_amd import kernels as K
+
+    g = torch.Generator(device=device)
+    g.manual_seed(1000 * d + 10 * length + group)
+    rows, hkv, splits, limit = 3, 4, 3, 48
+    hq = hkv * group
+    cache = torch.randn(rows, 2, limit, hkv, d, generator=g, device=device).to(torch.bfloat16)
+    cache[:, :, length:] = float("nan")
+    q = torch.randn(rows, hq, d, generator=g, device=device).to(torch.bfloat16)
+    pitch = hq * d + (1 if odd else 8)
+
+    def attend(query, store):
+        out = torch.full((rows, pitch), 7.0, dtype=torch.bfloat16, device=device)
+        _lib.call("nq_cp_short_attention", query.data_ptr(), query.stride(0), query.stride(1), store.data_ptr(),
+                  store.stride(0), store.stride(1), store.stride(2), store.stride(3), rows, length, hq, hkv, d,
+                  float(d) ** -0.5, out.data_ptr(), pitch, d, _lib.stream(device))
+        return out
+
+    out = attend(q, cache)
+    want = o_att.short_cache_attention(to_np(q), to_np(cache[:, 0]), to_np(cache[:, 1]), length)
+    mx, mean = attention_error(to_np(out[:, : hq * d].reshape(rows, hq, d)), want)
+    assert mx <= MAX_ABS and mean <= MEAN_ABS
+    assert bool((out[:, hq * d:] == 7.0).all())
+    if group > 2:
+        return
+    planes = torch.randn(splits, rows, (hq + 2 * hkv) * d, generator=g, device=device)
+    w = [torch.randn(d, generator=g, device=device).to(torch.bfloat16) for _ in range(2)]
+    at = torch.full((rows,), length - 1, dtype=torch.long, device=device)
+    caches, qs = [cache.clone() for _ in range(2)], [torch.empty_like(q) for _ in range(2)]
+    K.qkv_partials_norm_rope_dense_cache_(planes.view(torch.uint8).flatten(), splits, qs[0], *w, at, 1e-6, 1e6,
+                                          caches[0][:, 0], caches[0][:, 1], length - 1)
+    outs = [attend(qs[0], caches[0]), torch.full((rows, pitch), 7.0, dtype=torch.bfloat16, device=device)]
+    c = caches[1]
+    _lib.call("nq_cp_rope_short_attention", planes.data_ptr(), splits, rows, w[0].data_ptr(), w[1].data_ptr(),
+              at.data_ptr(), 1, 1e-6, 1e6, 0, qs[1].data_ptr(), qs[1].stride(0), qs[1].stride(1), c.data_ptr(),
+              c.stride(0), c.stride(1), c.stride(2), c.stride(3), length - 1, hq, hkv, d, float(d) ** -0.5,
+              outs[1].data_ptr(), pitch, d, _lib.stream(device))
+    for x, y in (caches, qs, outs):
+        assert torch.equal(x.view(torch.int16), y.view(torch.int16))
+
+
 @pytest.mark.parametrize("rows", [1, 4, 5, 8])
 @pytest.mark.parametrize("position", [0, 7, 15])
 @pytest.mark.parametrize("hkv", [2, 8])
