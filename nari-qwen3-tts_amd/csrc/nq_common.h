@@ -21,9 +21,9 @@ __device__ __forceinline__ float bf16_to_f32(uint16_t v) {
     return __uint_as_float(static_cast<uint32_t>(v) << 16);
 }
 
-// Round-to-nearest-even float -> bfloat16, quiet NaN preserved (matches torch): gfx950's conversion
-// instruction, whose result is that of u + 0x7fff + bit 16 (and of the quieted NaN) for every one of the
-// 2^32 floats.  Spelled out in integers it was five instructions and a branch a value, and the short
+// Round-to-nearest-even float -> bfloat16, NaNs quieted with their upper bits: gfx950's conversion
+// instruction, whose result is that of u + 0x7fff + bit 16 (test_bf16_rounding, on both sides of every
+// boundary and on every NaN's upper half).  Spelled out in integers it was five instructions and a branch a value, and the short
 // kernels, which spend about 9 ns on fetching each 64 bytes of straight-line code, paid for all of them.
 typedef float cvt_f32x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 cvt_bf16x2 __attribute__((ext_vector_type(2)));

@@ -353,6 +353,33 @@ def test_short_cache_entries_past_sixteen_positions(nq, device, d, group, length
         assert torch.equal(x.view(torch.int16), y.view(torch.int16))
 
 
+def test_bf16_rounding(nq, device):
+    """The rounding that every kernel of the library uses, seen through the V half of the K/V write (one
+    plane, its values stored as bf16): round to nearest even, NaNs quieted with their upper bits.  Every
+    upper half of a float, with the lower halves at both ends, beside the tie and on it: between two of
+    those the rounding, which is monotone, cannot change."""
+
+    from nari_qwen3_tts_amd import kernels as K
+
+    rows, hkv, d = 768, 8, 64
+    upper, lower = np.meshgrid(np.arange(1 << 16, dtype=np.uint32),
+                               np.array([0x0000, 0x0001, 0x7fff, 0x8000, 0x8001, 0xffff], np.uint32))
+    bits = ((upper << 16) | lower).reshape(-1)
+    bits[bits == 0x80000000] = 0  # the sum of the planes starts from +0
+    up = bits + 0x7fff + ((bits >> 16) & 1)
+    want = np.where((bits & 0x7fffffff) > 0x7f800000, (bits >> 16) | 0x40, up >> 16).astype(np.uint16)
+    planes = torch.zeros(1, rows, 3 * hkv * d, device=device)
+    planes[0, :, 2 * hkv * d:] = torch.from_numpy(bits.view(np.float32).reshape(rows, -1)).to(device)
+    ones = torch.ones(d, dtype=torch.bfloat16, device=device)
+    cache = torch.zeros(rows, 2, 4, hkv, d, dtype=torch.bfloat16, device=device)
+    q = torch.empty(rows, hkv, d, dtype=torch.bfloat16, device=device)
+    at = torch.zeros(rows, dtype=torch.long, device=device)
+    K.qkv_partials_norm_rope_dense_cache_(planes.view(torch.uint8).flatten(), 1, q, ones, ones, at, 1e-6, 1e6,
+                                          cache[:, 0], cache[:, 1], 0)
+    got = cache[:, 1, 0].contiguous().view(torch.int16).cpu().numpy().view(np.uint16).reshape(-1)
+    np.testing.assert_array_equal(got, want)
+
+
 @pytest.mark.parametrize("rows", [1, 4, 5, 8])
 @pytest.mark.parametrize("position", [0, 7, 15])
 @pytest.mark.parametrize("hkv", [2, 8])
