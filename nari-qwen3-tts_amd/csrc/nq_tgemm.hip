@@ -236,36 +236,42 @@ tgemm_kernel(const uint16_t *__restrict__ x, int64_t x_s0, int M, const uint16_t
 // Tile shapes of a launch: 128 x 128 over 4 x 4 waves of 32 x 32 (68 registers, 80 KB of LDS: one
 // workgroup of sixteen waves a CU), and 64 x 64 and 96 x 64 over 2 x 2 waves of 32 x 32 and 48 x 32,
 // three workgroups a CU.  Up to about 400 rows the large tiles leave CUs idle or rows padded, and more
-// K slices to fill them write more planes: QKV (N 4096, K 2048), o (2048, 2048) and down (2048, 6144)
-// with the add-RMSNorm took 11.3, 15.5 and 22.5 us at 192 rows and take 9.8 - 10.5, 13.0 and 18.6 in
-// 96 x 64 tiles; 10.2, 14.6 and 22.3 at 128 rows, and 8.3 - 9.3, 11.7 and 17.1 in 64 x 64.  At 448 rows
-// and more the large tiles read half the LDS bytes a product and win (QKV 15.9 us, small tiles 18).
+// K slices to fill them write more planes; from there on they read half the LDS bytes a product.
+// Measured in a graph with the consumer of the planes behind (24 layers' weights in turn, so from HBM), us
+// in 128 x 128 tiles at their best number of slices and as planned: QKV (N 4096, K 2048; q/k norm + RoPE)
+// at 128 rows 18.6 -> 16.9, 192 20.9 -> 20.2, 544 32.8 -> 30.6; o (2048, 2048; add-RMSNorm to FP8) 128
+// 14.9 -> 11.9, 192 16.0 -> 13.6, 320 18.6 -> 17.8, 448 20.7 -> 18.2; down (2048, 6144; add-RMSNorm) 128
+// 20.4 -> 17.9, 192 21.0 -> 20.7; at 640 rows the large tiles themselves (34.9, 22.8, 33.0).
 struct TgShape {
     int bm, bn;
-    double stage, overlap;  // us a 64-wide K stage of a workgroup costs, and how many it costs alone beyond its share
+    double stage, latency;  // us a 64-wide K stage costs: for each workgroup that shares a CU, and once
     double fixed;           // us of a launch beside its stages
 };
-constexpr TgShape kTgShapes[] = {{128, 128, 0.469, 0.0, 4.92}, {64, 64, 0.160, 0.8, 3.16}, {96, 64, 0.198, 0.8, 3.38}};
+constexpr TgShape kTgShapes[] = {{128, 128, 0.390, 0.109, 7.685}, {64, 64, 0.150, 0.349, 3.181}, {96, 64, 0.165, 0.431, 2.491}};
 constexpr int kTgBM = 128, kTgBN = 128;  // the large tile; every shape divides its columns
-constexpr double kTgPlane = 0.865e-6;    // us an element of a plane costs, written and read back
+constexpr double kTgPlane = 2.566e-6;    // us an element of a plane costs, written and read back
 
 struct TgPlan {
     int shape, S;
 };
 
 // The shape and the number of K slices (each a multiple of 64 columns and at least 256 of them) with
-// the least time by a model fitted to 200 measured launches of 128 - 640 rows (within 5 % of them on
-// average): a CU's workgroups share it, so a launch takes the stages of the fullest CU.
+// the least time by a model: a CU's workgroups share it, so a launch takes the stages of the fullest CU.
+// The constants rank 1,479 measured launches, every shape and number of slices of the three projections
+// above at 36 row counts from 128 to 2560: the planned launch is 0.7 % off the best one on average (11 % at
+// o of 304 rows, which planned two slices would gain) and at most 0.4 % slower than the best of the large
+// tiles.  (Fitted to fewer slices and rows, the rule had planned down at 128 rows 7 % slower than the large
+// tiles, o at 528 - 576 rows 5 % and QKV at 272 - 288 rows 3 %.)
 TgPlan tgemm_plan(int M, int N, int K) {
     TgPlan best = {0, 1};
     double best_cost = 1e30;
     for (int shape = 0; shape < 3; ++shape) {
         const TgShape &t = kTgShapes[shape];
         const int64_t tiles = static_cast<int64_t>((M + t.bm - 1) / t.bm) * (N / t.bn);
-        for (int s = 1; s <= (shape == 0 ? 8 : 4); ++s) {
+        for (int s = 1; s <= 8; ++s) {
             if (s > 1 && (K % (s * kTgK) || K / s < 256)) continue;
             const double share = static_cast<double>((tiles * s + 255) / 256);
-            const double cost = t.stage * (share + t.overlap) * (K / s / kTgK) + t.fixed +
+            const double cost = (t.stage * share + t.latency) * (K / s / kTgK) + t.fixed +
                                 kTgPlane * s * static_cast<double>(M) * N;
             if (cost < best_cost) {
                 best_cost = cost;

@@ -83,6 +83,20 @@ def test_host_side_metadata_queries_need_no_gpu(nq):
     assert lib.nq_attention_workspace_bytes(0, 1, 16, 16, 8, 128) == -1
 
 
+@pytest.mark.parametrize("m,n,k,splits", [
+    (128, 2048, 6144, 8),  # us at 4 slices 21.8, the large tiles' best 20.4, planned 17.9
+    (544, 2048, 2048, 2),  # 4 slices 23.4, large 22.2, planned 21.8
+    (272, 4096, 2048, 2),  # 4 slices 24.5, large 23.7, planned 23.7
+    (448, 2048, 6144, 4), (640, 2048, 6144, 3), (640, 4096, 2048, 1),  # the large tiles themselves
+])
+def test_prefill_plan_is_not_behind_the_large_tiles(nq, m, n, k, splits):
+    """Row counts at which a plan's slices were measured against the 128 x 128 tiles' best."""
+
+    from nari_qwen3_tts_amd import _lib
+
+    assert _lib.load().nq_tgemm_splits(m, n, k) == splits
+
+
 def test_argument_errors_are_caught_on_the_host(nq):
     """Invalid shapes return NQ_ERR_* before anything is launched."""
 

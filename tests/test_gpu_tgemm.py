@@ -52,6 +52,22 @@ def test_tgemm_exact_on_integer_operands(nq, device, m, n, k):
     assert torch.equal(out.view(torch.int16), want.view(torch.int16))
 
 
+@pytest.mark.parametrize("m,n,k", [(128, 2048, 6144), (145, 2048, 6144), (192, 2048, 6144), (193, 2048, 2048),
+                                   (97, 4096, 2048), (289, 2048, 6144), (448, 2048, 2048), (545, 4096, 2048)])
+def test_tgemm_planned_tiles_exact(nq, device, m, n, k):
+    """Row counts at which the plan takes each tile shape and the most and the fewest slices, on and beside a
+    tile's last row: the planes' sum is the exact product, and nothing behind the last plane is written."""
+
+    from nari_qwen3_tts_amd.layers import tgemm_partials
+
+    gen = torch.Generator().manual_seed(m + 3 * n + k)
+    x, w = _int_bf16((m, k), gen, device), _int_bf16((n, k), gen, device)
+    planes = torch.full((9 * m * n,), float("nan"), device=device)
+    s = tgemm_partials(x, w, planes.view(torch.uint8))
+    assert torch.equal(planes[: s * m * n].view(s, m, n).sum(0), x.float() @ w.float().t())
+    assert bool(planes[s * m * n:].isnan().all())
+
+
 @pytest.mark.parametrize("m,n,k", SHAPES[:5])
 def test_tgemm_random_within_fp32_accumulation(nq, device, m, n, k):
     from nari_qwen3_tts_amd.layers import tgemm
