@@ -245,9 +245,10 @@ gemm_fp8_kernel(const uint8_t *__restrict__ x, int64_t x_s0, const float *__rest
 
 // ---------------------------------------------------------------------------
 // Gate/up with the SwiGLU fused, for <= 64 rows and K = 2048 (the talker's
-// MLP).  The FP8 activation block [64, K] is 128 KiB, so one workgroup per CU
-// stages all of it in LDS and computes whole dot products: no split-K planes
-// and no second kernel.  The gate/up weight rows are held interleaved
+// MLP).  A workgroup stages the whole FP8 activation block in LDS (32 KiB for
+// up to 16 rows, 64 for 32, 128 for 64: there one workgroup per CU) and
+// computes whole dot products: no split-K planes and no second kernel.  The
+// gate/up weight rows are held interleaved
 // (nq_fp8_pack_swiglu): 16-row tile t holds, for q = 0..3, gate rows
 // 8t + 2q, 8t + 2q + 1 then up rows 8t + 2q, 8t + 2q + 1, so MFMA lane group q
 // ends with two gate/up pairs of the same act columns 8t + 2q + {0, 1}.  The

@@ -271,10 +271,11 @@ void dispatch_gemm(const uint16_t *x, int64_t x_s0, int M, const uint16_t *w, in
 }
 
 // ---------------------------------------------------------------------------
-// Gate/up with the SwiGLU fused, bf16, for rows in blocks of 64 and K = 1024
-// (the code predictor's MLP).  The activation block [64, K] is 128 KiB, so one
-// workgroup per CU stages all of it in LDS and computes whole dot products:
-// no split-K planes and no second kernel.  The weight rows are interleaved
+// Gate/up with the SwiGLU fused, bf16, for rows in blocks of 16, 32 or 64 and
+// K = 1024 (the code predictor's MLP).  A workgroup stages its whole activation
+// block in LDS (32, 64 or 128 KiB, the last one workgroup per CU) and computes
+// whole dot products: no split-K planes and no second kernel.  The weight rows
+// are interleaved
 // (nq_fp8_pack_swiglu on the bf16 rows): 16-row tile t holds, for q = 0..3,
 // gate rows 8t + 2q, 8t + 2q + 1 then up rows 8t + 2q, 8t + 2q + 1, so MFMA
 // lane group q ends with two gate/up pairs of the same act columns
@@ -285,7 +286,6 @@ void dispatch_gemm(const uint16_t *x, int64_t x_s0, int M, const uint16_t *w, in
 // order through LDS, and the epilogue rounds gate and up to bf16 and stores
 // bf16(silu(g) * u) -- the bits of the split-K projection with four 256-wide
 // slices (its choice at 128 rows) followed by the SiLU-mul kernel.
-
 //
 // MT 16-row tiles (1, 2 or 4) of rows and kTiles column tiles (2 or 3) a
 // workgroup.  The kernel is a chain of latencies and LDS passes: the staging and
