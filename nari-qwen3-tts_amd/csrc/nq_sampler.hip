@@ -248,7 +248,10 @@ sample_kernel(const InT *__restrict__ logits, int64_t logits_s0, int vocab,
             if ((id >= mask_from && id != eos_id) || (id == eos_id && sup_eos)) xv = -INFINITY;
             if (sn[i]) xv = xv > 0.0f ? xv / r : xv * r;
             val[i] = greedy ? xv : xv / T;
-            key[i] = id < vocab ? sort_key(val[i]) : 0u;
+            // at least 1: the NaN of all ones (memory filled with 0xff) has sort key 0, and a selection that
+            // left it out would be short of k ids and draw from what the LDS held
+            const uint32_t sk = sort_key(val[i]);
+            key[i] = id < vocab ? (sk > 1u ? sk : 1u) : 0u;
             if (id < vocab) s_val[id] = val[i];
         }
     }

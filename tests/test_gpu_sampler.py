@@ -107,6 +107,35 @@ def test_narrow_top_k_bit_exact(nq, device, vocab, top_k, values):
     _check(logits, t, k, p, u, r, seen)
 
 
+@pytest.mark.parametrize("top_k", [1, 50, 64, 65, 0])
+def test_logits_of_all_ones_bits_stay_in_the_vocabulary(nq, device, top_k):
+    """fp32 logits whose bytes are all 0xff (a NaN that sorts below every value): a row of them draws id 0,
+    among others they are never drawn ahead of a number, and nothing beside the seen mask is written."""
+
+    from nari_qwen3_tts_amd.sampling import sample_with_uniforms
+
+    rows, vocab = 4, 512
+    logits, t, k, p, u, r, seen = _inputs(device, 5, rows, vocab, dtype=torch.float32, top_k=top_k)
+    t.fill_(0.9)
+    p.fill_(0.95)
+    numbers = logits.clone()
+    numbers[:, ::3] = -float("inf")
+    logits.view(torch.int32)[:, ::3] = -1
+    logits.view(torch.int32)[0] = -1
+    guard = torch.zeros(rows + 2, vocab, dtype=torch.bool, device=device)
+    guard[1:-1].copy_(seen)
+    before = guard.clone()
+    options = dict(repetition_penalty=r, update_seen=True)
+    got = sample_with_uniforms(logits, t, k, p, u, seen_token_mask=guard[1:-1], **options)
+    assert int(got[0]) == 0
+    assert bool(((got >= 0) & (got < vocab)).all())
+    before[1:-1].scatter_(1, got[:, None], True)
+    assert torch.equal(guard, before)
+    if top_k:  # the whole vocabulary holds the NaNs themselves, whose weights are NaN
+        want = sample_with_uniforms(numbers, t, k, p, u, seen_token_mask=seen, **options)
+        assert torch.equal(got[1:], want[1:])
+
+
 def test_update_seen_marks_sampled_token(nq, device):
     from nari_qwen3_tts_amd.sampling import sample_with_uniforms
 
